@@ -304,9 +304,9 @@ PAIR = 20.0  # operations of one pair force, the usual count
 
 
 def _bh_per_particle(n, theta):
-    """Interactions per particle, a fit to counted runs: 1,341 on the encounter of 4,194,304 and 779 on that of
-    200,003 (theta 0.5), 926 on a sphere of 32,768 (0.6), 224 on one of 4,096 (1.0)."""
-    return min(n, 25.0 * math.log2(n) * (0.6 / max(theta, 0.3)) ** 1.8 + 80.0)
+    """Interactions per particle, a fit within about half of counted runs: 1,341 on the encounter of
+    4,194,304 and 779 on that of 200,003 (theta 0.5), 926 on a sphere of 32,768 (0.6), 224 on one of 4,096 (1.0)."""
+    return min(n, 220.0 / max(theta, 0.3) ** 2 * (1.0 + 0.06 * (math.log2(n) - 12.0)))
 
 
 def work(case):
