@@ -198,8 +198,8 @@ nbody_status check_masses(const double* mass, size_t n) {
     return NBODY_OK;
 }
 
-// Staging of nbody_field_noalloc: the points (first half) and their
-// accelerations (second half), 2 x NBODY_FIELD_NOALLOC_MAX_POINTS records,
+// Staging of nbody_field_noalloc: partial sums (first half) and the points,
+// then their accelerations (second half), 2 x NBODY_FIELD_NOALLOC_MAX_POINTS records,
 // 2 MiB held by every device the library runs on until the process ends.
 // In host code `field_scratch_array` names a host-side stand-in, not device
 // memory: only the address hipGetSymbolAddress returns (per device) is used.
@@ -641,30 +641,26 @@ nbody_status nbody_field(nbody_sim* s, const float* points, size_t m, float* acc
     NB_CHECK(m <= (size_t(1) << 30), NBODY_ERR_CAPACITY, "too many points");
     if (m == 0) return NBODY_OK;
     NB_HIP(hipSetDevice(s->cfg.device));
-    std::vector<float4> h(m);
-    for (size_t i = 0; i < m; ++i) h[i] = make_float4(points[3 * i], points[3 * i + 1], points[3 * i + 2], 0.f);
+    // partial sums, the packed points, their accelerations
+    const size_t part = direct_field_scratch(static_cast<int>(m), static_cast<int>(s->n_pad));
     float4* d = nullptr;
-    NB_HIP(hipMalloc(reinterpret_cast<void**>(&d), 2 * m * sizeof(float4)));
-    nbody_status st = NBODY_OK;
-    hipError_t e = hipMemcpyAsync(d, h.data(), m * sizeof(float4), hipMemcpyHostToDevice, s->stream);
+    NB_HIP(hipMalloc(reinterpret_cast<void**>(&d), part * sizeof(float4) + 6 * m * sizeof(float)));
+    float* pts = reinterpret_cast<float*>(d + part);
+    float* out = pts + 3 * m;
+    hipError_t e = hipMemcpyAsync(pts, points, 3 * m * sizeof(float), hipMemcpyHostToDevice, s->stream);
     if (e == hipSuccess)
-        e = direct_field(s->pos[s->cur], static_cast<int>(s->n_pad), d, static_cast<int>(m), s->cfg.law, s->dscale,
-                         d + m, s->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(h.data(), d + m, m * sizeof(float4), hipMemcpyDeviceToHost, s->stream);
+        e = direct_field(s->pos[s->cur], static_cast<int>(s->n_pad), pts, static_cast<int>(m), s->cfg.law, s->dscale,
+                         d, out, s->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(acc, out, 3 * m * sizeof(float), hipMemcpyDeviceToHost, s->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
+    nbody_status st = NBODY_OK;
     if (e != hipSuccess) {
         set_error("nbody_field: %s", hipGetErrorString(e));
         st = NBODY_ERR_DEVICE;
+        (void)hipStreamSynchronize(s->stream);
     }
-    (void)hipStreamSynchronize(s->stream);
     (void)hipFree(d);
-    if (st != NBODY_OK) return st;
-    for (size_t i = 0; i < m; ++i) {
-        acc[3 * i] = h[i].x;
-        acc[3 * i + 1] = h[i].y;
-        acc[3 * i + 2] = h[i].z;
-    }
-    return NBODY_OK;
+    return st;
 }
 
 nbody_status nbody_field_noalloc(nbody_sim* s, const float* points, size_t m, float* acc) {
@@ -679,15 +675,14 @@ nbody_status nbody_field_noalloc(nbody_sim* s, const float* points, size_t m, fl
     NB_HIP(hipSetDevice(s->cfg.device));
     float4* d = nullptr;
     NB_TRY(field_scratch(s->cfg.device, &d));
-    const int cap = NBODY_FIELD_NOALLOC_MAX_POINTS;
-    // the caller's packed points into the second half; direct_field_staged
-    // packs, evaluates and unpacks them inside the array
-    NB_HIP(hipMemcpyAsync(reinterpret_cast<float*>(d + cap), points, 3 * m * sizeof(float), hipMemcpyHostToDevice,
-                          s->stream));
-    NB_HIP(direct_field_staged(s->pos[s->cur], static_cast<int>(s->n_pad), d, cap, static_cast<int>(m), s->cfg.law,
-                               s->dscale, s->stream));
-    NB_HIP(hipMemcpyAsync(acc, reinterpret_cast<const float*>(d), 3 * m * sizeof(float), hipMemcpyDeviceToHost,
-                          s->stream));
+    // The packed points and then their accelerations in the second half, the
+    // chunks' partial sums (at most the array's half for so few points) in the
+    // first.
+    float* pts = reinterpret_cast<float*>(d + NBODY_FIELD_NOALLOC_MAX_POINTS);
+    NB_HIP(hipMemcpyAsync(pts, points, 3 * m * sizeof(float), hipMemcpyHostToDevice, s->stream));
+    NB_HIP(direct_field(s->pos[s->cur], static_cast<int>(s->n_pad), pts, static_cast<int>(m), s->cfg.law, s->dscale,
+                        d, pts, s->stream));
+    NB_HIP(hipMemcpyAsync(acc, pts, 3 * m * sizeof(float), hipMemcpyDeviceToHost, s->stream));
     NB_HIP(hipStreamSynchronize(s->stream));
     return NBODY_OK;
 }

@@ -106,36 +106,88 @@ __global__ __launch_bounds__(256) void reduce_kick_kernel(DirectLaunch L, int sp
     if (kick) kick_drift(L, i, ax, ay, az);
 }
 
-// Acceleration at arbitrary points from all sources: one target per lane,
-// every workgroup over the whole source range.
+// Acceleration at arbitrary points (3m packed floats) from all sources: one
+// target per lane, every workgroup over the whole source range.
 template <int LAW>
 __global__ __launch_bounds__(256) void field_kernel(const float4* __restrict__ src, int n_src_pad,
-                                                    const float4* __restrict__ tgt, int m, DirectScale sc,
-                                                    float4* __restrict__ out) {
+                                                    const float* __restrict__ pts, int m, DirectScale sc,
+                                                    float* __restrict__ out) {
     __shared__ core::SrcTile tiles[2];
     const int i = blockIdx.x * 256 + threadIdx.x;
-    const float4 q = tgt[min(i, m - 1)];
-    float xi[1] = {q.x * sc.inv_len}, yi[1] = {q.y * sc.inv_len}, zi[1] = {q.z * sc.inv_len};
+    const size_t p = 3 * static_cast<size_t>(min(i, m - 1));
+    float xi[1] = {pts[p] * sc.inv_len}, yi[1] = {pts[p + 1] * sc.inv_len}, zi[1] = {pts[p + 2] * sc.inv_len};
     float sx[1], sy[1], sz[1];
     core::block_forces<LAW, 1, 256>(tiles, src, 0, n_src_pad, sc, xi, yi, zi, sx, sy, sz);
-    if (i < m) out[i] = make_float4(sx[0] * sc.out, sy[0] * sc.out, sz[0] * sc.out, 0.f);
-}
-
-// (x, y, z) floats -> float4 targets.
-__global__ __launch_bounds__(256) void pack_points_kernel(const float* __restrict__ in, int m, float4* __restrict__ out) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < m) out[i] = make_float4(in[3 * i], in[3 * i + 1], in[3 * i + 2], 0.f);
-}
-
-// float4 accelerations -> (ax, ay, az) floats.
-__global__ __launch_bounds__(256) void unpack_points_kernel(const float4* __restrict__ in, int m, float* __restrict__ out) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
     if (i < m) {
-        const float4 a = in[i];
-        out[3 * i] = a.x;
-        out[3 * i + 1] = a.y;
-        out[3 * i + 2] = a.z;
+        out[p] = sx[0] * sc.out;
+        out[p + 1] = sy[0] * sc.out;
+        out[p + 2] = sz[0] * sc.out;
     }
+}
+
+// The same with the sources shared out twice, for few points: a workgroup
+// holds 64 points (every wavefront the same ones, wave w a quarter of each
+// source tile) and takes the tiles of one chunk, [blockIdx.y * jchunk, +jchunk).
+// part[chunk * m + i] receives the chunk's sums in scaled units.
+//
+// Bound by the pair arithmetic once the chip is full: 4,096 points from
+// 262,144 sources take 0.376 ms with the copies and the sum (2.9e12 pairs/s)
+// on 64 x 16 workgroups, 8.60 ms on the 16 that one workgroup per 256 points
+// over all sources makes.
+template <int LAW>
+__global__ __launch_bounds__(256) void field_slice_kernel(const float4* __restrict__ src, int n_src_pad,
+                                                          const float* __restrict__ pts, int m, DirectScale sc,
+                                                          int jchunk, float4* __restrict__ part) {
+    __shared__ core::SrcTile tiles[2];
+    __shared__ core::SliceSums sums;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i = blockIdx.x * 64 + lane;
+    const size_t p = 3 * static_cast<size_t>(min(i, m - 1));
+    float xi[1] = {pts[p] * sc.inv_len}, yi[1] = {pts[p + 1] * sc.inv_len}, zi[1] = {pts[p + 2] * sc.inv_len};
+    float sx[1], sy[1], sz[1];
+    const int j0 = blockIdx.y * jchunk, j1 = min(j0 + jchunk, n_src_pad);
+    core::block_forces<LAW, 1, 256, 4>(tiles, src, j0, j1, sc, xi, yi, zi, sx, sy, sz);
+    core::add_slices(sums, wave, lane, sx[0], sy[0], sz[0]);
+    if (wave == 0 && i < m)
+        part[static_cast<size_t>(blockIdx.y) * m + i] = make_float4(sx[0], sy[0], sz[0], 0.f);
+}
+
+// Adds the chunks' sums of each point in chunk order (compensated) and scales
+// them back.
+__global__ __launch_bounds__(256) void field_sum_kernel(const float4* __restrict__ part, int split, int m,
+                                                        DirectScale sc, float* __restrict__ out) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= m) return;
+    float sx = 0.f, sy = 0.f, sz = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;
+    for (int s = 0; s < split; ++s) {
+        const float4 p = part[static_cast<size_t>(s) * m + i];
+        kahan_add(sx, cx, p.x);
+        kahan_add(sy, cy, p.y);
+        kahan_add(sz, cz, p.z);
+    }
+    float* o = out + 3 * static_cast<size_t>(i);
+    o[0] = sx * sc.out;
+    o[1] = sy * sc.out;
+    o[2] = sz * sc.out;
+}
+
+// Chunks the field's sources are split into (0: field_kernel, no partial
+// sums).  One workgroup per 256 points over all sources fills the chip's
+// 2,048 workgroup places of eight waves per SIMD only from 524,288 points on;
+// below 262,144 (the half of it, still faster than 64 points each, whose
+// workgroups stage every tile four times as often per pair) a workgroup takes
+// 64 points and the sources are split until there are 2,048 workgroups, as far
+// as there are tiles and as the partial sums fit kFieldPartials records (from
+// 65,537 points on a single chunk).  Depends on the two sizes only, so the
+// entry with a staging array of its own gives the same bits.
+constexpr int kFieldPartials = NBODY_FIELD_NOALLOC_MAX_POINTS;
+
+int field_split(int m, int n_src_pad) {
+    if (m >= 262144) return 0;
+    const int tiles = n_src_pad / kTile, blocks = (m + 63) / 64;
+    const int want = std::max(1, std::min({(2048 + blocks - 1) / blocks, kFieldPartials / m, tiles}));
+    const int per = (tiles + want - 1) / want;
+    return (tiles + per - 1) / per;  // no empty chunk
 }
 
 using ForceFn = void (*)(DirectLaunch, int);
@@ -228,30 +280,27 @@ DirectShape direct_default_shape(int n_pad) {
     return s;
 }
 
-hipError_t direct_field(const float4* src, int n_src_pad, const float4* tgt, int m, int law, const DirectScale& sc,
-                        float4* out, hipStream_t stream) {
-    if (m <= 0) return hipSuccess;
-    const dim3 grid((m + 255) / 256);
-    if (law == NBODY_LAW_R)
-        hipLaunchKernelGGL(field_kernel<NBODY_LAW_R>, grid, dim3(256), 0, stream, src, n_src_pad, tgt, m, sc, out);
-    else
-        hipLaunchKernelGGL(field_kernel<NBODY_LAW_P>, grid, dim3(256), 0, stream, src, n_src_pad, tgt, m, sc, out);
-    return hipGetLastError();
+size_t direct_field_scratch(int m, int n_src_pad) {
+    return static_cast<size_t>(field_split(m, n_src_pad)) * static_cast<size_t>(m);
 }
 
-hipError_t direct_field_staged(const float4* src, int n_src_pad, float4* staging, int cap, int m, int law,
-                               const DirectScale& sc, hipStream_t stream) {
+hipError_t direct_field(const float4* src, int n_src_pad, const float* pts, int m, int law, const DirectScale& sc,
+                        float4* part, float* out, hipStream_t stream) {
     if (m <= 0) return hipSuccess;
-    if (m > cap) return hipErrorInvalidValue;
-    const dim3 grid((m + 255) / 256);
-    float4* half0 = staging;
-    float4* half1 = staging + cap;
-    hipLaunchKernelGGL(pack_points_kernel, grid, dim3(256), 0, stream, reinterpret_cast<const float*>(half1), m, half0);
+    const bool r = law == NBODY_LAW_R;
+    const int split = field_split(m, n_src_pad);
+    if (split == 0) {
+        hipLaunchKernelGGL((r ? field_kernel<NBODY_LAW_R> : field_kernel<NBODY_LAW_P>), dim3((m + 255) / 256),
+                           dim3(256), 0, stream, src, n_src_pad, pts, m, sc, out);
+        return hipGetLastError();
+    }
+    const int tiles = n_src_pad / kTile;
+    const int jchunk = ((tiles + split - 1) / split) * kTile;
+    hipLaunchKernelGGL((r ? field_slice_kernel<NBODY_LAW_R> : field_slice_kernel<NBODY_LAW_P>),
+                       dim3((m + 63) / 64, split), dim3(256), 0, stream, src, n_src_pad, pts, m, sc, jchunk, part);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    e = direct_field(src, n_src_pad, half0, m, law, sc, half1, stream);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(unpack_points_kernel, grid, dim3(256), 0, stream, half1, m, reinterpret_cast<float*>(half0));
+    hipLaunchKernelGGL(field_sum_kernel, dim3((m + 255) / 256), dim3(256), 0, stream, part, split, m, sc, out);
     return hipGetLastError();
 }
 

@@ -73,19 +73,13 @@ DirectShape direct_default_shape(int n_pad);
 hipError_t direct_step(const DirectLaunch& L, const DirectShape& s, bool kick, hipStream_t stream,
                        hipEvent_t ev_force_begin, hipEvent_t ev_force_end);
 
-// Accelerations at m points tgt[] (float4, w ignored) from the n_src_pad
-// sources src[] (padded with massless dummies) in the sources' scaled units:
-// out[i], float4 (ax, ay, az, 0).
-hipError_t direct_field(const float4* src, int n_src_pad, const float4* tgt, int m, int law, const DirectScale& sc,
-                        float4* out, hipStream_t stream);
-
-// The same in a caller's staging array of 2 * cap float4 records, without any
-// allocation: on entry the second half holds the 3m packed floats of the
-// points; the first half receives them as float4 targets, the second half
-// their accelerations, and on return the first half holds the 3m packed floats
-// of the accelerations (m <= cap).  Three stream-ordered kernels, each reading
-// one half and writing the other.
-hipError_t direct_field_staged(const float4* src, int n_src_pad, float4* staging, int cap, int m, int law,
-                               const DirectScale& sc, hipStream_t stream);
+// Accelerations at m points (pts, 3m packed floats) from the n_src_pad sources
+// src[] (padded with massless dummies) in the sources' scaled units: out, 3m
+// packed floats (may be pts itself when part is used).  part holds
+// direct_field_scratch(m, n_src_pad) records: at most
+// NBODY_FIELD_NOALLOC_MAX_POINTS, or m if that is more.
+size_t direct_field_scratch(int m, int n_src_pad);
+hipError_t direct_field(const float4* src, int n_src_pad, const float* pts, int m, int law, const DirectScale& sc,
+                        float4* part, float* out, hipStream_t stream);
 
 }  // namespace nbody

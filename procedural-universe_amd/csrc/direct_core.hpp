@@ -143,11 +143,19 @@ __device__ __forceinline__ void stage_source(const float4 s, const DirectScale& 
 // the current one is consumed, and written to the other buffer, so one
 // barrier per tile separates the writes from the reads.  Every thread of the
 // workgroup must call it; targets are already in scaled units.
-template <int LAW, int K, int BLOCK>
+//
+// SLICES > 1: the sources of every tile are dealt to the workgroup's
+// wavefronts (wave w takes the w-th of SLICES equal runs of the tile), so the
+// lanes of different waves may hold the same targets; the caller adds the
+// waves' sums.
+template <int LAW, int K, int BLOCK, int SLICES = 1>
 __device__ __forceinline__ void block_forces(SrcTile* tiles, const float4* __restrict__ src, const int j0, const int j1,
                                              const DirectScale& sc, const float (&xi)[K], const float (&yi)[K],
                                              const float (&zi)[K], float (&sx)[K], float (&sy)[K], float (&sz)[K]) {
     static_assert(kTile % BLOCK == 0, "tile must be a multiple of the block");
+    static_assert(SLICES == 1 || SLICES == BLOCK / 64, "one slice of the tile per wavefront");
+    constexpr int kSlice = kTile / SLICES;
+    const int s0 = SLICES == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6) * kSlice;
     constexpr int PER = kTile / BLOCK;
     const int tid = threadIdx.x;
     const float tiny = in_vgpr(__FLT_MIN__);
@@ -181,7 +189,7 @@ __device__ __forceinline__ void block_forces(SrcTile* tiles, const float4* __res
         // Groups of four sources: four rsq arguments per target, then one
         // grouped rsq4 per target, then the accumulation.
 #pragma unroll NBODY_GROUP_UNROLL
-        for (int j = 0; j < kTile; j += 4) {
+        for (int j = s0; j < s0 + kSlice; j += 4) {
             float4 pj[4];
 #pragma unroll
             for (int g = 0; g < 4; ++g) pj[g] = T.p[j + g];
@@ -232,6 +240,31 @@ __device__ __forceinline__ void block_forces(SrcTile* tiles, const float4* __res
                 stage_source<LAW>(pre[l], sc, tiles[buf ^ 1].p[tid + l * BLOCK], tiles[buf ^ 1].k[tid + l * BLOCK]);
             __syncthreads();
             buf ^= 1;
+        }
+    }
+}
+
+// The waves' sums of the same 64 targets (block_forces with SLICES = 4),
+// added in wave order into wave 0's.  Every thread of the workgroup must call
+// it; only wave 0 returns the totals.
+struct SliceSums {
+    float v[3][3][64];
+};
+
+__device__ __forceinline__ void add_slices(SliceSums& S, int wave, int lane, float& x, float& y, float& z) {
+    if (wave > 0) {
+        S.v[wave - 1][0][lane] = x;
+        S.v[wave - 1][1][lane] = y;
+        S.v[wave - 1][2][lane] = z;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        float cx = 0.f, cy = 0.f, cz = 0.f;
+#pragma unroll
+        for (int w = 0; w < 3; ++w) {
+            kahan_add(x, cx, S.v[w][0][lane]);
+            kahan_add(y, cy, S.v[w][1][lane]);
+            kahan_add(z, cz, S.v[w][2][lane]);
         }
     }
 }
