@@ -144,12 +144,12 @@ __global__ __launch_bounds__(256) void field_slice_kernel(const float4* __restri
     const int i = blockIdx.x * 64 + lane;
     const size_t p = 3 * static_cast<size_t>(min(i, m - 1));
     float xi[1] = {pts[p] * sc.inv_len}, yi[1] = {pts[p + 1] * sc.inv_len}, zi[1] = {pts[p + 2] * sc.inv_len};
-    float sx[1], sy[1], sz[1];
+    float sx[1], sy[1], sz[1], cx[1], cy[1], cz[1];
     const int j0 = blockIdx.y * jchunk, j1 = min(j0 + jchunk, n_src_pad);
-    core::block_forces<LAW, 1, 256, 4>(tiles, src, j0, j1, sc, xi, yi, zi, sx, sy, sz);
-    core::add_slices(sums, wave, lane, sx[0], sy[0], sz[0]);
-    if (wave == 0 && i < m)
-        part[static_cast<size_t>(blockIdx.y) * m + i] = make_float4(sx[0], sy[0], sz[0], 0.f);
+    core::block_forces_comp<LAW, 1, 256, 4>(tiles, src, j0, j1, sc, xi, yi, zi, sx, sy, sz, cx, cy, cz);
+    float s[3] = {sx[0], sy[0], sz[0]}, c[3] = {cx[0], cy[0], cz[0]};
+    core::add_slices(sums, wave, lane, s, c);
+    if (wave == 0 && i < m) part[static_cast<size_t>(blockIdx.y) * m + i] = make_float4(s[0], s[1], s[2], 0.f);
 }
 
 // Adds the chunks' sums of each point in chunk order (compensated) and scales

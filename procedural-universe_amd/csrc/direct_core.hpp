@@ -70,6 +70,16 @@ __device__ __forceinline__ float in_vgpr(float x) {
 // covers the transcendental-result forwarding wait before the first use.
 // The compiler itself separates a v_rsq_f32 result from its first VALU use by
 // one wait state; the group ends with NBODY_RSQ_NOP + 1 of them.
+//
+// The group issues at raised wave priority: a v_rsq_f32 keeps one of the two
+// issue paths a SIMD shares among its waves busy for four FMAs' time, and a
+// wave that gets to its group first leaves the other path to the other waves'
+// arithmetic instead of queueing behind it.  In a register-only loop of the
+// unordered pair's mix (68 FMA-class + 4 rsq) at six waves per SIMD it took
+// 184 SIMD cycles instead of 236; raised over the FMAs instead of the rsq, 240;
+// one step of the one-sided sum at N = 2^20 300 -> 288 ms, of the sum over
+// unordered pairs 219 -> 191 ms.  The priority outside the group is 0 in every
+// kernel that uses it.
 #ifndef NBODY_RSQ_NOP
 #define NBODY_RSQ_NOP 1
 #endif
@@ -82,10 +92,12 @@ __device__ __forceinline__ float in_vgpr(float x) {
 
 __device__ __forceinline__ void rsq4(float& a, float& b, float& c, float& d) {
     asm volatile(
+        "s_setprio 1\n\t"
         "v_rsq_f32 %0, %0\n\t"
         "v_rsq_f32 %1, %1\n\t"
         "v_rsq_f32 %2, %2\n\t"
         "v_rsq_f32 %3, %3\n\t"
+        "s_setprio 0\n\t"
         "s_nop " NBODY_STR(NBODY_RSQ_NOP)
         : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
 }
@@ -147,11 +159,13 @@ __device__ __forceinline__ void stage_source(const float4 s, const DirectScale& 
 // SLICES > 1: the sources of every tile are dealt to the workgroup's
 // wavefronts (wave w takes the w-th of SLICES equal runs of the tile), so the
 // lanes of different waves may hold the same targets; the caller adds the
-// waves' sums.
-template <int LAW, int K, int BLOCK, int SLICES = 1>
-__device__ __forceinline__ void block_forces(SrcTile* tiles, const float4* __restrict__ src, const int j0, const int j1,
-                                             const DirectScale& sc, const float (&xi)[K], const float (&yi)[K],
-                                             const float (&zi)[K], float (&sx)[K], float (&sy)[K], float (&sz)[K]) {
+// waves' sums.  (cx, cy, cz) receive the sums' compensations.
+template <int LAW, int K, int BLOCK, int SLICES>
+__device__ __forceinline__ void block_forces_comp(SrcTile* tiles, const float4* __restrict__ src, const int j0,
+                                                  const int j1, const DirectScale& sc, const float (&xi)[K],
+                                                  const float (&yi)[K], const float (&zi)[K], float (&sx)[K],
+                                                  float (&sy)[K], float (&sz)[K], float (&cx)[K], float (&cy)[K],
+                                                  float (&cz)[K]) {
     static_assert(kTile % BLOCK == 0, "tile must be a multiple of the block");
     static_assert(SLICES == 1 || SLICES == BLOCK / 64, "one slice of the tile per wavefront");
     constexpr int kSlice = kTile / SLICES;
@@ -160,7 +174,6 @@ __device__ __forceinline__ void block_forces(SrcTile* tiles, const float4* __res
     const int tid = threadIdx.x;
     const float tiny = in_vgpr(__FLT_MIN__);
     const float soft = in_vgpr(sc.soft);
-    float cx[K], cy[K], cz[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         sx[k] = sy[k] = sz[k] = 0.f;
@@ -244,28 +257,39 @@ __device__ __forceinline__ void block_forces(SrcTile* tiles, const float4* __res
     }
 }
 
-// The waves' sums of the same 64 targets (block_forces with SLICES = 4),
-// added in wave order into wave 0's.  Every thread of the workgroup must call
-// it; only wave 0 returns the totals.
+template <int LAW, int K, int BLOCK>
+__device__ __forceinline__ void block_forces(SrcTile* tiles, const float4* __restrict__ src, const int j0, const int j1,
+                                             const DirectScale& sc, const float (&xi)[K], const float (&yi)[K],
+                                             const float (&zi)[K], float (&sx)[K], float (&sy)[K], float (&sz)[K]) {
+    float cx[K], cy[K], cz[K];
+    block_forces_comp<LAW, K, BLOCK, 1>(tiles, src, j0, j1, sc, xi, yi, zi, sx, sy, sz, cx, cy, cz);
+}
+
+// The waves' compensated sums (s, c: Kahan's sum and compensation) of the same
+// 64 targets, added in wave order into wave 0's, compensations included (four
+// sums rounded apart cost a third more error than one).  Every thread of the
+// workgroup must call it; only wave 0 returns the totals, in s.
 struct SliceSums {
-    float v[3][3][64];
+    float s[3][3][64], c[3][3][64];
 };
 
-__device__ __forceinline__ void add_slices(SliceSums& S, int wave, int lane, float& x, float& y, float& z) {
+__device__ __forceinline__ void add_slices(SliceSums& S, int wave, int lane, float (&s)[3], float (&c)[3]) {
     if (wave > 0) {
-        S.v[wave - 1][0][lane] = x;
-        S.v[wave - 1][1][lane] = y;
-        S.v[wave - 1][2][lane] = z;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            S.s[wave - 1][a][lane] = s[a];
+            S.c[wave - 1][a][lane] = c[a];
+        }
     }
     __syncthreads();
     if (wave == 0) {
-        float cx = 0.f, cy = 0.f, cz = 0.f;
 #pragma unroll
-        for (int w = 0; w < 3; ++w) {
-            kahan_add(x, cx, S.v[w][0][lane]);
-            kahan_add(y, cy, S.v[w][1][lane]);
-            kahan_add(z, cz, S.v[w][2][lane]);
-        }
+        for (int w = 0; w < 3; ++w)
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                kahan_add(s[a], c[a], S.s[w][a][lane]);
+                kahan_add(s[a], c[a], -S.c[w][a][lane]);
+            }
     }
 }
 
