@@ -134,6 +134,13 @@ DirectShape shape_for(const nbody_sim* s) {
     return d;
 }
 
+nbody_status grow_part(nbody_sim* s, size_t records) {
+    s->part_elems = 0;
+    NB_TRY(dev_alloc(&s->part, records));
+    s->part_elems = records;
+    return NBODY_OK;
+}
+
 // Size the device buffers for n particles (keeping larger ones) and set the
 // launch shape; the contents are left to the caller.
 nbody_status prepare_state(nbody_sim* s, size_t n) {
@@ -156,15 +163,24 @@ nbody_status prepare_state(nbody_sim* s, size_t n) {
     s->cur = 0;
     s->shape = shape_for(s);
     const size_t split = static_cast<size_t>(direct_effective_split(s->shape, static_cast<int>(n_pad)));
-    // Partial sums serve the direct kernel only (a Barnes-Hut handle uses it
-    // for a single particle alone).
+    // Partial sums serve the direct kernels only (a Barnes-Hut handle uses
+    // them for a single particle alone).
     const bool direct = s->cfg.method == NBODY_METHOD_DIRECT || n < 2;
-    const size_t need_part = direct ? std::max<size_t>(split, 1) * n_pad : 0;
-    if (need_part > s->part_elems) {
-        NB_TRY(dev_alloc(&s->part, need_part));
-        s->part_elems = need_part;
+    const bool tuned = s->cfg.tune_i_per_lane || s->cfg.tune_block || s->cfg.tune_split;
+    s->sym = direct && !tuned ? sym_plan(static_cast<int>(n_pad)) : SymPlan{};
+    if (s->sym.nsb > 0) {
+        const size_t need = sym_part_records(s->sym, static_cast<int>(n_pad));
+        if (need <= s->part_elems) return NBODY_OK;
+        // Its rows take up to 2 KB per particle: on a device too full for them
+        // the one-sided sum runs instead.
+        const nbody_status st = grow_part(s, need);
+        if (st != NBODY_ERR_OUT_OF_MEMORY) return st;
+        (void)hipGetLastError();
+        clear_error();
+        s->sym = SymPlan{};
     }
-    return NBODY_OK;
+    const size_t need_part = direct ? std::max<size_t>(split, 1) * n_pad : 0;
+    return need_part > s->part_elems ? grow_part(s, need_part) : NBODY_OK;
 }
 
 // The largest coordinate range of n positions (x, y, z in .x .y .z).
@@ -188,6 +204,15 @@ double extent_of(const float4* p, size_t n) {
 // orders of magnitude keeps them, which the pair arithmetic's range allows).
 void set_scale(nbody_sim* s, double extent) {
     s->dscale = direct_scale_for(s->cfg.law, s->cfg.softening, extent, s->max_gm);
+}
+
+// Whether every particle has the same positive G m (in FP32, as the records
+// hold it); mass: n FP64 masses.
+void set_equal(nbody_sim* s, const std::vector<double>& mass) {
+    const float first = s->n ? static_cast<float>(s->cfg.G * mass[0]) : 0.f;
+    bool equal = first > 0.f && std::isfinite(first);
+    for (size_t i = 1; i < s->n && equal; ++i) equal = static_cast<float>(s->cfg.G * mass[i]) == first;
+    s->gm_equal = equal ? first : 0.f;
 }
 
 // Masses must be finite and >= 0 (the direct sum folds G m into a square).
@@ -239,6 +264,7 @@ nbody_status upload_state(nbody_sim* s, const std::vector<float4>& pos, const st
         hg[i] = s->cfg.G * mass[i];
         s->max_gm = std::max(s->max_gm, std::fabs(hg[i]));
     }
+    set_equal(s, mass);
     set_scale(s, extent_of(pos.data(), n));
     NB_HIP(hipMemcpyAsync(s->pos[0], hp.data(), n_pad * sizeof(float4), hipMemcpyHostToDevice, s->stream));
     NB_HIP(hipMemcpyAsync(s->pos[1], hp.data(), n_pad * sizeof(float4), hipMemcpyHostToDevice, s->stream));
@@ -274,9 +300,18 @@ DirectLaunch launch_for(nbody_sim* s, float dt) {
     L.n_pad = static_cast<int>(s->n_pad);
     L.law = s->cfg.law;
     L.sc = s->dscale;
+    L.gm_equal = s->gm_equal * (s->cfg.law == NBODY_LAW_R ? 1.0f / s->dscale.mass_k : s->dscale.mass_k);
     L.dt = dt;
     L.dts = static_cast<float>(static_cast<double>(dt) / s->cfg.scale);
     return L;
+}
+
+// The launch shape in use, for nbody_get_timing.
+void report_shape(nbody_sim* s) {
+    const bool sym = s->sym.nsb > 0;
+    s->last.i_per_lane = sym ? 4 : s->shape.i_per_lane;
+    s->last.block = sym ? kTile : s->shape.block;
+    s->last.split = sym ? s->sym.split : direct_effective_split(s->shape, static_cast<int>(s->n_pad));
 }
 
 // One force evaluation (kick: a full step).  ev_b/ev_e bracket the force kernel(s).
@@ -285,7 +320,8 @@ nbody_status force_pass(nbody_sim* s, float dt, bool kick, hipEvent_t ev_b, hipE
         NB_TRY(bh_step(s, dt, kick, ev_b, ev_e));
     } else {
         DirectLaunch L = launch_for(s, dt);
-        NB_HIP(direct_step(L, s->shape, kick, s->stream, ev_b, ev_e));
+        NB_HIP(s->sym.nsb > 0 ? sym_step(L, s->sym, kick, s->stream, ev_b, ev_e)
+                              : direct_step(L, s->shape, kick, s->stream, ev_b, ev_e));
         s->step_interactions += static_cast<uint64_t>(s->n) * static_cast<uint64_t>(s->n);
     }
     if (kick) s->cur ^= 1;
@@ -431,6 +467,7 @@ nbody_status nbody_init_plummer(nbody_sim* s, uint64_t seed, size_t n, double a,
     const double m = total_mass / static_cast<double>(n);
     s->mass_host.assign(n, m);
     s->max_gm = std::fabs(s->cfg.G * m);
+    set_equal(s, s->mass_host);
     set_scale(s, 40.0 * a);  // radii are cut at 20 a
     s->initialised = true;
     s->acc_valid = false;
@@ -476,9 +513,7 @@ nbody_status step_graph(nbody_sim* s, float dt, int32_t nsteps) {
     s->step_interactions = s->bh ? 0 : static_cast<uint64_t>(nsteps) * s->n * s->n;
     s->last.steps = nsteps;
     s->last.interactions = s->step_interactions;
-    s->last.i_per_lane = s->shape.i_per_lane;
-    s->last.block = s->shape.block;
-    s->last.split = direct_effective_split(s->shape, static_cast<int>(s->n_pad));
+    report_shape(s);
     s->timed_steps = 0;
     return NBODY_OK;
 }
@@ -509,6 +544,7 @@ nbody_status nbody_init_seeded(nbody_sim* s, int32_t seeder, uint64_t seed, size
     NB_HIP(hipStreamSynchronize(s->stream));
     s->max_gm = 0.0;
     for (double m : s->mass_host) s->max_gm = std::max(s->max_gm, std::fabs(s->cfg.G * m));
+    set_equal(s, s->mass_host);
     set_scale(s, extent_of(pos_host.data(), n));
     s->initialised = true;
     s->acc_valid = false;
@@ -544,9 +580,7 @@ nbody_status nbody_step(nbody_sim* s, float dt, int32_t nsteps) {
     s->last.steps = nsteps;
     s->last.force_launches = s->timing ? nsteps : 0;
     s->last.interactions = s->step_interactions;
-    s->last.i_per_lane = s->shape.i_per_lane;
-    s->last.block = s->shape.block;
-    s->last.split = direct_effective_split(s->shape, static_cast<int>(s->n_pad));
+    report_shape(s);
     s->timed_steps = s->timing ? nsteps : 0;
     return NBODY_OK;
 }

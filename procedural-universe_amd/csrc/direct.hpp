@@ -53,6 +53,7 @@ struct DirectLaunch {
     int n_pad;          // padded count, multiple of kTile
     int law;            // nbody_law
     DirectScale sc;     // the system's scaled units
+    float gm_equal;     // sym_step: every real particle's G m in scaled units if all are equal, else 0
     float dt;           // kick step
     float dts;          // drift factor dt / scale
 };
@@ -72,6 +73,21 @@ DirectShape direct_default_shape(int n_pad);
 // kernel writes partial sums and a second kernel adds them in chunk order.
 hipError_t direct_step(const DirectLaunch& L, const DirectShape& s, bool kick, hipStream_t stream,
                        hipEvent_t ev_force_begin, hipEvent_t ev_force_end);
+
+// The sum over unordered pairs (direct_sym.hip): nsb blocks of `block`
+// particles, every streamed block cut into `split` runs.
+struct SymPlan {
+    int block;  // particles per block, a multiple of 1,024
+    int nsb;    // blocks; 0: not used at this size
+    int split;  // 1, 2 or 4
+};
+
+SymPlan sym_plan(int n_pad);
+// Records of `part` that the plan writes.
+size_t sym_part_records(const SymPlan& p, int n_pad);
+// One force evaluation (kick: a full step), as direct_step.
+hipError_t sym_step(const DirectLaunch& L, const SymPlan& p, bool kick, hipStream_t stream, hipEvent_t ev_force_begin,
+                    hipEvent_t ev_force_end);
 
 // Accelerations at m points (pts, 3m packed floats) from the n_src_pad sources
 // src[] (padded with massless dummies) in the sources' scaled units: out, 3m

@@ -29,7 +29,7 @@ struct nbody_sim {
     int cur = 0;                          // index of the current positions
     float4* vel = nullptr;                // (vx, vy, vz, 0)
     float4* acc = nullptr;                // last accelerations (ax, ay, az, 0)
-    float4* part = nullptr;               // direct: partial sums [split][n_pad]
+    float4* part = nullptr;               // direct: partial sums (direct_step's or sym_step's)
     size_t part_elems = 0;
     double* mass_dev = nullptr;           // FP64 masses (diagnostics)
     double* gm_dev = nullptr;             // FP64 G*m (diagnostics)
@@ -38,10 +38,12 @@ struct nbody_sim {
     size_t diag_elems = 0;
     std::vector<double> mass_host;        // FP64 masses (FORCES read-back = m * a)
     double max_gm = 0.0;                  // largest |G*m| (the direct sum's mass scale)
+    float gm_equal = 0.f;                 // FP32 G*m if every particle has the same positive one, else 0
     nbody::DirectScale dscale{1.f, 1.f, 0.f, 1.f};  // direct sum's scaled units
     bool acc_valid = false;
 
     nbody::DirectShape shape{4, 256, 1};
+    nbody::SymPlan sym{};  // nsb > 0: the direct sum over unordered pairs instead
     nbody::BHState* bh = nullptr;
 
     // Timing of the last nbody_step call.
