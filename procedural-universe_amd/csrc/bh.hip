@@ -1200,6 +1200,11 @@ __device__ __forceinline__ float lane_masked(float x, unsigned w, int lane) {
 // namespace (nb_writelane).
 
 
+// Lane l's value of x (l uniform over the wave), in every lane.
+__device__ __forceinline__ float read_lane(float x, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
+}
+
 // (lo, hi) = x in lane l only (register writes; the other lanes keep lo and
 // hi).  l and x are uniform over the wave.
 __device__ __forceinline__ void write_lane64(unsigned& lo, unsigned& hi, unsigned long long x, int l) {
@@ -1227,16 +1232,25 @@ __device__ __forceinline__ void write_entry(float4* lsrc, float* lk, uint2* lmas
 // full evaluation; the direct sum's pair arithmetic, direct_core.hpp), each term zeroed for
 // lanes outside its entry; (px, py, pz) is the lane's particle in scaled
 // units.  The sums (scaled units) go to the lane's compensated accumulator.
-template <int LAW>
+//
+// SLOTS > 1 (a wave of 64 / SLOTS particles): slot s evaluates the s-th of every
+// SLOTS groups of four; the caller has padded the list to whole rounds of
+// 4 x SLOTS entries.  `lane` is then the lane's particle.
+template <int LAW, int SLOTS>
 __device__ __forceinline__ void flush_list(const float4* lsrc, const float* lk, const uint2* lmask, int cnt, int lane,
-                                           float px, float py, float pz, float soft, float& sx, float& sy, float& sz,
-                                           float& cx, float& cy, float& cz) {
+                                           int slot, float px, float py, float pz, float soft, float& sx, float& sy,
+                                           float& sz, float& cx, float& cy, float& cz) {
     const float tiny = core::in_vgpr(__FLT_MIN__);
     float ax = 0.f, ay = 0.f, az = 0.f;
     // the lane's word of every entry's mask
     const unsigned* words = reinterpret_cast<const unsigned*>(lmask) + (lane >> 5);
-    const int cnt4 = cnt & ~3;
-    for (int e = 0; e < cnt4; e += 4) {
+    if constexpr (SLOTS > 1) {
+        lsrc += 4 * slot;
+        lk += 4 * slot;
+        words += 8 * slot;
+    }
+    const int cnt4 = SLOTS == 1 ? cnt & ~3 : cnt;
+    for (int e = 0; e < cnt4; e += 4 * SLOTS) {
         float4 src[4];
         float dx[4], dy[4], dz[4], q[4];
         const float4 k4 = *reinterpret_cast<const float4*>(lk + e);
@@ -1273,7 +1287,7 @@ __device__ __forceinline__ void flush_list(const float4* lsrc, const float* lk, 
     }
     // the last one to three entries one at a time (the same arithmetic and
     // order; v_rsq_f32 through the compiler's builtin)
-    for (int e = cnt4; e < cnt; ++e) {
+    for (int e = cnt4; SLOTS == 1 && e < cnt; ++e) {
         const float4 src = lsrc[e];
         const float dx = src.x - px, dy = src.y - py, dz = src.z - pz;
         float q;
@@ -1310,8 +1324,9 @@ __device__ __forceinline__ void flush_list(const float4* lsrc, const float* lk, 
 // dense and sparse regions spread over all of them.  A bijection on [0, nb).
 constexpr int kXcds = 8;
 
+template <int G>
 __device__ __forceinline__ int xcd_block(int b, int nb) {
-    constexpr int C = 2048 / kTravThreads;  // runs of 2048 particles
+    constexpr int C = 2048 / G;  // runs of 2048 particles
     const int full = (nb / (kXcds * C)) * (kXcds * C);
     if (b >= full) return b;
     const int x = b % kXcds, k = b / kXcds;
@@ -1322,7 +1337,13 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
 // workgroup limit keeps 24 one-wave workgroups per CU (six per SIMD)
 // resident.  The box's six bounds stay in vector registers: held in scalar
 // registers they were spilled and reloaded every batch (2.3% slower).
-template <int LAW>
+//
+// G particles per wavefront (64, 32, 16 or 8).  Below 64 the lanes hold the
+// particles 64 / G times over: every copy takes part in the walk alike (masks
+// have G bits), and in the list each copy, a slot, evaluates its share of the
+// entries; the slots' sums are added at the end.  A small system is then more
+// and shorter wavefronts.
+template <int LAW, int G>
 __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __restrict__ pos_sorted,
                                                                 const ChildBlock* __restrict__ blocks,
                                                                 const int* __restrict__ node_first,
@@ -1341,9 +1362,12 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
     __shared__ unsigned long long red[3][kTravWaves];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: list and stack addresses in SGPRs
-    const int blk = xcd_block(blockIdx.x, gridDim.x);
-    const int t = blk * kTravThreads + tid;
-    const int wave_base = blk * kTravThreads + wave * 64;
+    constexpr int SLOTS = 64 / G;
+    constexpr unsigned long long kGroup = G == 64 ? ~0ull : (1ull << (G & 63)) - 1ull;  // the particles' mask bits
+    const int mine = lane & (G - 1), slot = lane / G;
+    const int blk = xcd_block<G>(blockIdx.x, gridDim.x);
+    const int t = blk * G + mine;
+    const int wave_base = blk * G;
     const bool valid = t < A.n;
     const float4 me = pos_sorted[valid ? t : A.n - 1];
     // the particle in the pair arithmetic's scaled units (the decisions use me)
@@ -1374,10 +1398,22 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
     };
     auto flush = [&]() {
         entries += static_cast<unsigned long long>(cnt);
-        const int total = __builtin_amdgcn_readfirstlane(cnt);
+        int total = __builtin_amdgcn_readfirstlane(cnt);
         __builtin_amdgcn_wave_barrier();
+        if constexpr (SLOTS > 1) {
+            // whole rounds of four entries per slot: empty masks, finite sources
+            const int whole = (total + 4 * SLOTS - 1) & ~(4 * SLOTS - 1);
+            if (total + lane < whole) {
+                lsrc[wave][total + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+                lk[wave][total + lane] = 0.f;
+                lmask[wave][total + lane] = make_uint2(0u, 0u);
+            }
+            total = whole;
+            __builtin_amdgcn_wave_barrier();
+        }
         __builtin_amdgcn_s_setprio(0);  // the list at normal priority, the walk raised (kernel start)
-        flush_list<LAW>(lsrc[wave], lk[wave], lmask[wave], total, lane, mx, my, mz, soft, sx, sy, sz, cx, cy, cz);
+        flush_list<LAW, SLOTS>(lsrc[wave], lk[wave], lmask[wave], total, mine, slot, mx, my, mz, soft, sx, sy, sz, cx,
+                               cy, cz);
         __builtin_amdgcn_s_setprio(1);
         __builtin_amdgcn_wave_barrier();
         cnt = 0;
@@ -1387,7 +1423,7 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
     // the lanes of a particle's own position never interact with it
     auto without_self = [&](unsigned long long m, int q) {
         const int l = q - wave_base;
-        return (l >= 0 && l < 64) ? (m & ~(1ULL << l)) : m;
+        return (l >= 0 && l < G) ? (m & ~(1ULL << l)) : m;
     };
 
     // The wave's bounding box (lanes past n hold the last particle, inside it).
@@ -1412,7 +1448,7 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
         __builtin_amdgcn_ballot_w64(!(__builtin_isfinite(me.x) && __builtin_isfinite(me.y) &&
                                       __builtin_isfinite(me.z))) == 0ull;
 
-    const unsigned long long all = __builtin_amdgcn_ballot_w64(valid);
+    const unsigned long long all = __builtin_amdgcn_ballot_w64(valid) & kGroup;
     if (all) {
         // the root: approximated by the lanes beyond its threshold (the
         // reference's side / |p - COM| < theta as r2 >= thr, see
@@ -1511,7 +1547,20 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
         // every lane (the lanes' masks start as all lanes).
         ge_lo = open_all ? 0u : ~0u;
         ge_hi = open_all ? 0u : ~0u;
-        for (int j = 0; j < k; ++j) {
+        if constexpr (G < 64) {
+            // From the registers of the lane that holds the child: with few
+            // wavefronts per SIMD a scalar load of each block would be waited
+            // for in full, cell after cell.
+            for (unsigned long long todo = tested; todo != 0ull; todo &= todo - 1ull) {
+                const int l = static_cast<int>(__builtin_ctzll(todo));
+                const float dx = me.x - read_lane(vsrc.x, l), dy = me.y - read_lane(vsrc.y, l),
+                            dz = me.z - read_lane(vsrc.z, l);
+                const float r2 = (dx * dx + dy * dy) + dz * dz;
+                const unsigned long long ge = __builtin_amdgcn_ballot_w64(!(r2 < read_lane(vthr, l)));
+                if (ge != ~0ull) write_lane64(ge_lo, ge_hi, ge, l);
+            }
+        }
+        for (int j = 0; G == 64 && j < k; ++j) {
             const unsigned tj = static_cast<unsigned>(tested >> (8 * j)) & 0xffu;
             if (tj == 0u) continue;  // every child cell of cell j has its box verdict
             const int code = __builtin_amdgcn_readlane(vcell, j * 8);
@@ -1547,7 +1596,7 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
         const unsigned long long children = __builtin_amdgcn_ballot_w64(vcode != kEmpty) & batch;
         const bool leaf = vcode < 0;
         const unsigned own = static_cast<unsigned>(dec_leaf(vcode) - wave_base);
-        const unsigned long long self = (leaf && own < 64u) ? (1ull << own) : 0ull;
+        const unsigned long long self = (leaf && own < static_cast<unsigned>(G)) ? (1ull << own) : 0ull;
         const unsigned long long ge = leaf ? ~0ull : ((static_cast<unsigned long long>(ge_hi) << 32) | ge_lo);
         const unsigned long long am = mask & ge & ~self;
         const unsigned long long om = mask & ~ge;
@@ -1597,7 +1646,17 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
     for (int off = 32; off > 0; off >>= 1) lane_total += __shfl_xor(lane_total, off);
     count += lane_total;
 
-    if (valid) {
+    if constexpr (SLOTS > 1) {
+        // the slots' sums, compensations included, in a fixed order
+#pragma unroll
+        for (int off = G; off < 64; off <<= 1) {
+            const float ox = __shfl_xor(sx, off), oy = __shfl_xor(sy, off), oz = __shfl_xor(sz, off);
+            const float qx = __shfl_xor(cx, off), qy = __shfl_xor(cy, off), qz = __shfl_xor(cz, off);
+            kahan_add(sx, cx, ox), kahan_add(sy, cy, oy), kahan_add(sz, cz, oz);
+            kahan_add(sx, cx, -qx), kahan_add(sy, cy, -qy), kahan_add(sz, cz, -qz);
+        }
+    }
+    if (valid && slot == 0) {
         const unsigned p = A.order[t];
         // back from scaled units (a power of two: exact)
         const float ax = sx * A.sc.out, ay = sy * A.sc.out, az = sz * A.sc.out;
@@ -1711,6 +1770,20 @@ inline int mass_rows(int n) {
         if (blocks_for(static_cast<size_t>(n) + 1, rows * kMassThreads) <= kMassFusedChunks) return rows;
     return kMassPer;
 }
+
+// Particles per wavefront of the traversal.  Few particles make short
+// wavefronts and many of them (a walk over few cells, the list shared by the
+// slots) but more walks in all, so the smallest systems take eight, and 64 pay
+// off from about a million on.  Force pass, ms, with 64 / 32 / 16 / 8:
+//   Plummer sphere, theta 0.6:    16,384  0.256 / 0.168 / 0.123 / 0.099
+//                                 32,768  0.293 / 0.187 / 0.144 / 0.138
+//                                 65,536  0.331 / 0.209 / 0.169 / 0.203
+//                                131,072  0.326 / 0.234 / 0.269 / 0.316
+//   two-disc encounter, 0.5:     524,288  0.858 / 0.708 / 0.853 / 1.120
+//                              1,048,576  1.353 / 1.434 / 1.719 / 2.354
+// Where systems share the device the total work counts, so the next larger
+// count is taken where it costs one alone little (32,768).
+inline int trav_group(int n) { return n <= 24576 ? 8 : n <= 98304 ? 16 : n <= 786432 ? 32 : 64; }
 
 float theta_below(double theta) {
     float t = static_cast<float>(theta);
@@ -1966,13 +2039,14 @@ nbody_status bh_step(nbody_sim* s, float dt, bool kick, hipEvent_t ev_b, hipEven
     A.dt = dt;
     A.dts = static_cast<float>(static_cast<double>(dt) / s->cfg.scale);
     if (ev_b) NB_HIP(hipEventRecord(ev_b, st));
-    const dim3 tgrid(blocks_for(n, kTravThreads));
-    if (s->cfg.law == NBODY_LAW_R)
-        hipLaunchKernelGGL(traverse_kernel<NBODY_LAW_R>, tgrid, dim3(kTravThreads), 0, st, b->pos_sorted, b->blocks,
-                           b->first, b->last, A);
-    else
-        hipLaunchKernelGGL(traverse_kernel<NBODY_LAW_P>, tgrid, dim3(kTravThreads), 0, st, b->pos_sorted, b->blocks,
-                           b->first, b->last, A);
+    const int group = trav_group(n);
+    const bool r = s->cfg.law == NBODY_LAW_R;
+    const auto fn = group == 8    ? (r ? traverse_kernel<NBODY_LAW_R, 8> : traverse_kernel<NBODY_LAW_P, 8>)
+                    : group == 16 ? (r ? traverse_kernel<NBODY_LAW_R, 16> : traverse_kernel<NBODY_LAW_P, 16>)
+                    : group == 32 ? (r ? traverse_kernel<NBODY_LAW_R, 32> : traverse_kernel<NBODY_LAW_P, 32>)
+                                  : (r ? traverse_kernel<NBODY_LAW_R, 64> : traverse_kernel<NBODY_LAW_P, 64>);
+    hipLaunchKernelGGL(fn, dim3(blocks_for(n, group)), dim3(kTravThreads), 0, st, b->pos_sorted, b->blocks, b->first,
+                       b->last, A);
     NB_HIP(hipGetLastError());
     if (ev_e) NB_HIP(hipEventRecord(ev_e, st));
     hipLaunchKernelGGL(publish_counters_kernel, dim3(1), dim3(64), 0, st, b->counters, b->walk, b->host_ctr);
