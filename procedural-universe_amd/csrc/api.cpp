@@ -12,6 +12,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <string>
@@ -404,6 +405,7 @@ nbody_status nbody_destroy(nbody_sim* s) {
     drop_graphs(s);
     if (s->bh) bh_destroy(s->bh);
     release_state(s);
+    release_stage(s->read_stage);
     for (hipEvent_t e : s->events) (void)hipEventDestroy(e);
     for (hipEvent_t e : s->tree_ms_pending) (void)hipEventDestroy(e);
     (void)hipStreamDestroy(s->stream);
@@ -613,23 +615,9 @@ nbody_status nbody_read_soa(nbody_sim* s, float* pos, float* vel, float* acc, si
     NB_CHECK(s->initialised, NBODY_ERR_NOT_INITIALISED, "read before nbody_init");
     NB_CHECK(n == s->n, NBODY_ERR_INVALID_ARG, "n = %zu does not match the state's %zu particles", n, s->n);
     NB_HIP(hipSetDevice(s->cfg.device));
-    std::vector<float4> tmp(n);
-    auto fetch = [&](const float4* src, float* dst) -> nbody_status {
-        if (!dst || n == 0) return NBODY_OK;
-        NB_HIP(hipMemcpyAsync(tmp.data(), src, n * sizeof(float4), hipMemcpyDeviceToHost, s->stream));
-        NB_HIP(hipStreamSynchronize(s->stream));
-        for (size_t i = 0; i < n; ++i) {
-            dst[3 * i] = tmp[i].x;
-            dst[3 * i + 1] = tmp[i].y;
-            dst[3 * i + 2] = tmp[i].z;
-        }
-        return NBODY_OK;
-    };
-    NB_HIP(hipStreamSynchronize(s->stream));
-    NB_TRY(fetch(s->pos[s->cur], pos));
-    NB_TRY(fetch(s->vel, vel));
-    NB_TRY(fetch(s->acc, acc));
-    return NBODY_OK;
+    const float4* const src[kReadFields] = {s->pos[s->cur], s->vel, s->acc};
+    float* const dst[kReadFields] = {pos, vel, acc};
+    return read_packed(s->read_stage, src, dst, n, s->stream);
 }
 
 nbody_status nbody_read(nbody_sim* s, nbody_particle* p, size_t n, uint32_t fields) {
@@ -637,16 +625,34 @@ nbody_status nbody_read(nbody_sim* s, nbody_particle* p, size_t n, uint32_t fiel
     NB_CHECK(s, NBODY_ERR_INVALID_ARG, "sim is null");
     NB_CHECK(p || n == 0, NBODY_ERR_INVALID_ARG, "particles is null");
     NB_CHECK((fields & ~15u) == 0, NBODY_ERR_INVALID_ARG, "unknown field bits 0x%x", fields);
-    std::vector<float> pos(3 * n), vel(3 * n), acc(3 * n);
-    NB_TRY(nbody_read_soa(s, (fields & NBODY_FIELD_POSITION) ? pos.data() : nullptr,
-                          (fields & NBODY_FIELD_VELOCITY) ? vel.data() : nullptr,
-                          (fields & NBODY_FIELD_FORCES) ? acc.data() : nullptr, n));
+    NB_CHECK(s->initialised, NBODY_ERR_NOT_INITIALISED, "read before nbody_init");
+    NB_CHECK(n == s->n, NBODY_ERR_INVALID_ARG, "n = %zu does not match the state's %zu particles", n, s->n);
+    NB_HIP(hipSetDevice(s->cfg.device));
+    const bool want[kReadFields] = {(fields & NBODY_FIELD_POSITION) != 0, (fields & NBODY_FIELD_VELOCITY) != 0,
+                                    (fields & NBODY_FIELD_FORCES) != 0};
+    const float4* const src[kReadFields] = {s->pos[s->cur], s->vel, s->acc};
+    const float* from[kReadFields];
+    std::unique_ptr<float[]> host[kReadFields];
+    nbody_status st = read_pinned(s->read_stage, src, want, n, s->stream, from);
+    if (st == NBODY_ERR_CAPACITY) {
+        float* dst[kReadFields] = {nullptr, nullptr, nullptr};
+        for (int f = 0; f < kReadFields; ++f) {
+            if (!want[f]) continue;
+            host[f].reset(new (std::nothrow) float[3 * n]);
+            NB_CHECK(host[f], NBODY_ERR_OUT_OF_MEMORY, "no host memory to read %zu particles", n);
+            from[f] = dst[f] = host[f].get();
+        }
+        float* const out[kReadFields] = {dst[0], dst[1], dst[2]};
+        st = read_packed(s->read_stage, src, out, n, s->stream);
+    }
+    NB_TRY(st);
+    const float *pos = from[0], *vel = from[1], *acc = from[2];
     for (size_t i = 0; i < n; ++i) {
-        if (fields & NBODY_FIELD_POSITION)
+        if (want[0])
             for (int c = 0; c < 3; ++c) p[i].position[c] = pos[3 * i + c];
-        if (fields & NBODY_FIELD_VELOCITY)
+        if (want[1])
             for (int c = 0; c < 3; ++c) p[i].velocity[c] = vel[3 * i + c];
-        if (fields & NBODY_FIELD_FORCES)
+        if (want[2])
             for (int c = 0; c < 3; ++c) p[i].forces[c] = s->mass_host[i] * static_cast<double>(acc[3 * i + c]);
         if (fields & NBODY_FIELD_MASS) p[i].mass = s->mass_host[i];
     }

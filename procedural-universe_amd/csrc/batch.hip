@@ -27,6 +27,7 @@
 #include "direct.hpp"
 #include "direct_core.hpp"
 #include "ic_device.hpp"
+#include "readback.hpp"
 #include "sim.hpp"
 
 namespace nbody {
@@ -197,6 +198,8 @@ struct nbody_batch {
     // sequential baseline: partial-sum buffer of the plain kernel
     float4* part = nullptr;
     size_t part_elems = 0;
+
+    ReadStage read_stage;
 
     hipEvent_t ev[2] = {nullptr, nullptr};
     bool timed = false;
@@ -395,6 +398,7 @@ nbody_status nbody_batch_destroy(nbody_batch* b) {
     (void)hipSetDevice(b->cfg.device);
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     drop_graph(b);
+    release_stage(b->read_stage);
     for (void* p : {static_cast<void*>(b->pos[0]), static_cast<void*>(b->pos[1]), static_cast<void*>(b->vel),
                     static_cast<void*>(b->acc), static_cast<void*>(b->d_sys), static_cast<void*>(b->d_items),
                     static_cast<void*>(b->d_n_items), static_cast<void*>(b->d_counters), static_cast<void*>(b->part),
@@ -676,22 +680,9 @@ nbody_status nbody_batch_read(nbody_batch* b, int32_t id, float* pos, float* vel
     const auto& y = b->systems[id];
     NB_CHECK(n == y.n, NBODY_ERR_INVALID_ARG, "system %d has %zu particles, not %zu", id, y.n, n);
     NB_HIP(hipSetDevice(b->cfg.device));
-    NB_HIP(hipStreamSynchronize(b->stream));
-    std::vector<float4> tmp(n);
-    auto fetch = [&](const float4* src, float* dst) -> nbody_status {
-        if (!dst) return NBODY_OK;
-        NB_HIP(hipMemcpy(tmp.data(), src + y.off, n * sizeof(float4), hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < n; ++i) {
-            dst[3 * i] = tmp[i].x;
-            dst[3 * i + 1] = tmp[i].y;
-            dst[3 * i + 2] = tmp[i].z;
-        }
-        return NBODY_OK;
-    };
-    NB_TRY(fetch(b->pos[b->cur], pos));
-    NB_TRY(fetch(b->vel, vel));
-    NB_TRY(fetch(b->acc, acc));
-    return NBODY_OK;
+    const float4* const src[kReadFields] = {b->pos[b->cur] + y.off, b->vel + y.off, b->acc + y.off};
+    float* const dst[kReadFields] = {pos, vel, acc};
+    return read_packed(b->read_stage, src, dst, n, b->stream);
 }
 
 nbody_status nbody_batch_get_info(nbody_batch* b, nbody_batch_info* out) {

@@ -9,6 +9,7 @@
 
 #include "../../include/nbody.h"
 #include "direct.hpp"
+#include "readback.hpp"
 
 namespace nbody {
 struct BHState;
@@ -36,6 +37,7 @@ struct nbody_sim {
     double* diag_buf = nullptr;
     double* ic_scratch = nullptr;         // device initial conditions: recentring sums
     size_t diag_elems = 0;
+    nbody::ReadStage read_stage;
     std::vector<double> mass_host;        // FP64 masses (FORCES read-back = m * a)
     double max_gm = 0.0;                  // largest |G*m| (the direct sum's mass scale)
     float gm_equal = 0.f;                 // FP32 G*m if every particle has the same positive one, else 0
