@@ -354,7 +354,9 @@ typedef struct nbody_batch_info {
 } nbody_batch_info;
 
 /* cfg->method must be NBODY_METHOD_DIRECT; capacity = arena size in particles
- * (each system takes its size rounded up to 256). */
+ * (each system takes its size rounded up to 256).  Steps of systems of 8,192
+ * particles or more also use up to 1 GiB of device memory for partial sums,
+ * allocated as they need it (without it, slower and rounded differently). */
 nbody_status nbody_batch_create(const nbody_config* cfg, size_t capacity, nbody_batch** out);
 nbody_status nbody_batch_destroy(nbody_batch* batch);
 
@@ -372,7 +374,7 @@ nbody_status nbody_batch_add_plummer(nbody_batch* batch, uint64_t seed, size_t n
 /* Advance every system nsteps kick-drift steps (asynchronous, one graph launch). */
 nbody_status nbody_batch_step(nbody_batch* batch, float dt, int32_t nsteps);
 
-/* The baseline: each system alone, one single-system launch per step, waiting
+/* The baseline: each system alone, one-sided single-system launches, waiting
  * for each system before the next.  split_small = 0: the plain launch (one
  * workgroup per 256 targets, all sources); 1: the single-system default,
  * which splits a small system's sources over more workgroups. */

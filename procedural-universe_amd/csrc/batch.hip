@@ -9,6 +9,13 @@
 // core (direct_core.hpp) over its own system's sources, so a system's forces are
 // the same bits whether it runs alone or in any mix.
 //
+// Systems from 8,192 particles on take the sum over unordered pairs
+// (direct_sym.hip) instead: a persistent kernel drains their tasks, then one adds
+// their rows of partial sums and kicks.  The rows lie in a buffer of at most
+// kRowsBytes; where a batch's systems need more, they are taken in groups, one
+// group's two kernels after the other's.  Which way a system takes, and its
+// tasks, depend on its size alone.
+//
 // The queue lives in device memory (items, their count, per-step counters), so
 // a captured hipGraph of k steps stays valid while systems join and leave: only
 // the item list is rewritten between launches.  The per-step counters are
@@ -21,11 +28,13 @@
 #include <cstring>
 #include <map>
 #include <new>
+#include <tuple>
 #include <vector>
 
 #include "common.hpp"
 #include "direct.hpp"
 #include "direct_core.hpp"
+#include "direct_sym_core.hpp"
 #include "ic_device.hpp"
 #include "readback.hpp"
 #include "sim.hpp"
@@ -38,9 +47,46 @@ struct SysDesc {
     int off;         // first record in the arena
     int n;           // real particles
     int n_pad;       // padded to kTile
-    int pad_;
+    float gm_equal;  // every particle's G m in scaled units if all are equal, else 0
     DirectScale sc;  // the system's scaled units
+    SymPlan sym;     // nsb > 0: over unordered pairs
+    size_t rows;     // its partial sums in the rows buffer (floats)
 };
+
+// A task of the sum over unordered pairs: blocks a and a + d, run h of the
+// streamed one.
+struct SymTask {
+    int sys, a, d, h;
+};
+
+// 64 particles of a system whose rows are to be added.
+struct SumItem {
+    int sys, i;
+};
+
+// The tasks and sums of the systems that share the rows buffer at a time.
+struct SymGroup {
+    int task0, task1;
+    int sum0, sum1;
+};
+
+// Partial sums of at most this many bytes in flight (the 512 galaxies of up to
+// 65,536 particles need about 4 GB in all); a system that needs more alone
+// stays with the one-sided sum.
+constexpr size_t kRowsBytes = size_t(1) << 30;
+
+// Below this the blocks with themselves, one-sided, are too large a part.
+constexpr size_t kSymMin = 8192;
+
+SymPlan batch_sym_plan(size_t n_pad) {
+    SymPlan p{};
+    if (n_pad < kSymMin) return p;
+    p.block = 1024;
+    p.nsb = static_cast<int>((n_pad + 1023) / 1024);
+    p.split = p.nsb <= 16 ? 4 : 2;
+    if (sym_part_records(p, static_cast<int>(n_pad)) * sizeof(float4) > kRowsBytes) p = SymPlan{};
+    return p;
+}
 
 struct WorkItem {
     int sys;    // slot in the descriptor table
@@ -55,6 +101,10 @@ struct BatchLaunch {
     const SysDesc* sys;
     const WorkItem* items;
     const int* n_items;
+    const SymTask* tasks;
+    const SumItem* sums;
+    const SymGroup* groups;
+    float* rows;
     float dt;
     float dts;
 };
@@ -62,6 +112,20 @@ struct BatchLaunch {
 __global__ void fill_u32_kernel(unsigned* p, int n, unsigned v) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
+}
+
+// Kick then drift of record r (positions x) with the acceleration (ax, ay, az).
+__device__ __forceinline__ void batch_kick(const BatchLaunch& B, int r, float4 x, float ax, float ay, float az) {
+    float4 v = B.vel[r];
+    v.x = __builtin_fmaf(ax, B.dt, v.x);
+    v.y = __builtin_fmaf(ay, B.dt, v.y);
+    v.z = __builtin_fmaf(az, B.dt, v.z);
+    x.x = __builtin_fmaf(v.x, B.dts, x.x);
+    x.y = __builtin_fmaf(v.y, B.dts, x.y);
+    x.z = __builtin_fmaf(v.z, B.dts, x.z);
+    B.vel[r] = v;
+    B.pos_out[r] = x;
+    B.acc[r] = make_float4(ax, ay, az, 0.f);
 }
 
 // The barriers around the item fetch also separate one item's last reads of
@@ -95,21 +159,62 @@ __global__ __launch_bounds__(BLOCK) void batch_step_kernel(BatchLaunch B, unsign
         for (int k = 0; k < K; ++k) {  // K is 1 or 2: fully unrolled without a pragma
             const int i = w.ibase + tid + k * BLOCK;
             if (i < d.n) {
-                const int r = d.off + i;
-                const float ax = sx[k] * d.sc.out, ay = sy[k] * d.sc.out, az = sz[k] * d.sc.out;
-                float4 v = B.vel[r];
-                float4 x = src[i];
-                v.x = __builtin_fmaf(ax, B.dt, v.x);
-                v.y = __builtin_fmaf(ay, B.dt, v.y);
-                v.z = __builtin_fmaf(az, B.dt, v.z);
-                x.x = __builtin_fmaf(v.x, B.dts, x.x);
-                x.y = __builtin_fmaf(v.y, B.dts, x.y);
-                x.z = __builtin_fmaf(v.z, B.dts, x.z);
-                B.vel[r] = v;
-                B.pos_out[r] = x;
-                B.acc[r] = make_float4(ax, ay, az, 0.f);
+                batch_kick(B, d.off + i, src[i], sx[k] * d.sc.out, sy[k] * d.sc.out, sz[k] * d.sc.out);
             }
         }
+    }
+}
+
+// The tasks of one group, largest systems first, from a counter.  Every branch is
+// uniform over the workgroup.  Bound by the pair arithmetic's issue: 96 systems
+// of 1,024 to 32,768 particles, five steps and their reads, 21.9 ms, 29.0 ms with
+// every system one-sided; a burst of 16 served requests 66.6 -> 50.8 ms.
+template <int LAW>
+__global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(6))) void batch_sym_kernel(BatchLaunch B,
+                                                                                                 int group,
+                                                                                                 unsigned* counter) {
+    __shared__ core::SymShared S;
+    __shared__ int item_sh;
+    const SymGroup G = B.groups[group];
+    for (;;) {
+        if (threadIdx.x == 0) item_sh = G.task0 + static_cast<int>(atomicAdd(counter, 1u));
+        __syncthreads();
+        const int it = item_sh;
+        __syncthreads();
+        if (it >= G.task1) break;
+        const SymTask w = B.tasks[it];
+        const SysDesc D = B.sys[w.sys];
+        const core::SymArgs A{B.pos_in + D.off, B.rows + D.rows, D.n_pad, D.sym, D.sc};
+        const int H = D.sym.nsb / 2;
+        if (w.d == 0) {
+            if (D.gm_equal > 0.f) core::sym_task<LAW, false, true>(A, S, w.a, w.a, w.h, w.h, 0);
+            else core::sym_task<LAW, false, false>(A, S, w.a, w.a, w.h, w.h, 0);
+        } else {
+            int b = w.a + w.d;
+            if (b >= D.sym.nsb) b -= D.sym.nsb;
+            const int rowi = w.d * D.sym.split + w.h, rowj = (H + 1) * D.sym.split + w.d - 1;
+            if (D.gm_equal > 0.f) core::sym_task<LAW, true, true>(A, S, w.a, b, w.h, rowi, rowj);
+            else core::sym_task<LAW, true, false>(A, S, w.a, b, w.h, rowi, rowj);
+        }
+    }
+}
+
+// Adds the rows of one group's systems, 64 particles a workgroup at a time.
+__global__ __launch_bounds__(256) void batch_sum_kernel(BatchLaunch B, int group) {
+    __shared__ core::SliceSums sums;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const SymGroup G = B.groups[group];
+    for (int it = G.sum0 + static_cast<int>(blockIdx.x); it < G.sum1; it += static_cast<int>(gridDim.x)) {
+        const SumItem w = B.sums[it];
+        const SysDesc D = B.sys[w.sys];
+        const int i = w.i + lane;
+        float s[3];
+        core::sum_rows(B.rows + D.rows, D.sym, D.n_pad, i, sums, wave, lane, s);
+        if (wave == 0 && i < D.n) {
+            const float out = D.gm_equal > 0.f ? D.gm_equal * D.sc.out : D.sc.out;
+            batch_kick(B, D.off + i, B.pos_in[D.off + i], s[0] * out, s[1] * out, s[2] * out);
+        }
+        __syncthreads();  // the sums are read before the next item's
     }
 }
 
@@ -165,6 +270,7 @@ struct nbody_batch {
         size_t off = 0, n = 0, n_pad = 0;
         DirectScale sc{};
         double max_gm = 0.0;
+        float gm_equal = 0.f;  // FP32 G*m if every particle has the same positive one, else 0
     };
     std::vector<Sys> systems;  // index = id = descriptor slot
     std::vector<int> free_ids;
@@ -174,6 +280,16 @@ struct nbody_batch {
     WorkItem* d_items = nullptr;
     size_t items_cap = 0;
     int* d_n_items = nullptr;
+    SymTask* d_tasks = nullptr;
+    size_t tasks_cap = 0;
+    SumItem* d_sums = nullptr;
+    size_t sums_cap = 0;
+    SymGroup* d_groups = nullptr;
+    size_t groups_cap = 0;
+    float* d_rows = nullptr;
+    size_t rows_cap = 0;
+    int n_tasks = 0, n_groups = 0;
+    bool no_rows = false;  // the rows buffer could not be allocated
     unsigned* d_counters = nullptr;
     int counters_cap = 0;
     bool items_dirty = true;
@@ -212,9 +328,10 @@ namespace {
 
 // Grow a device buffer; the old one is freed once the steps queued on the
 // batch's stream (which may read it) have completed.
-nbody_status ensure_dev(void** p, size_t& cap, size_t need, size_t elem, hipStream_t stream) {
+nbody_status ensure_dev(void** p, size_t& cap, size_t need, size_t elem, hipStream_t stream,
+                        size_t limit = ~size_t(0)) {
     if (need <= cap && *p) return NBODY_OK;
-    size_t ncap = std::max<size_t>(need, cap * 2);
+    size_t ncap = std::max(need, std::min(limit, cap * 2));
     if (ncap == 0) ncap = 1;
     void* q = nullptr;
     NB_HIP(hipMalloc(&q, ncap * elem));
@@ -274,30 +391,83 @@ nbody_status rebuild_items(nbody_batch* b) {
     std::stable_sort(order.begin(), order.end(),
                      [&](int a, int c) { return b->systems[a].n_pad > b->systems[c].n_pad; });
     std::vector<WorkItem> items;
+    std::vector<SymTask> tasks;
+    std::vector<SumItem> sums;
+    std::vector<SymGroup> groups;
     std::vector<SysDesc> descs(b->systems.size());
     uint64_t inter = 0;
     for (size_t s = 0; s < b->systems.size(); ++s) {
         const auto& y = b->systems[s];
-        descs[s] = SysDesc{static_cast<int>(y.off), static_cast<int>(y.n), static_cast<int>(y.n_pad), 0, y.sc};
+        const float gm = y.gm_equal * (b->cfg.law == NBODY_LAW_R ? 1.0f / y.sc.mass_k : y.sc.mass_k);
+        descs[s] = SysDesc{static_cast<int>(y.off), static_cast<int>(y.n), static_cast<int>(y.n_pad), gm, y.sc, {}, 0};
     }
+    // Groups of systems, largest first, whose rows fit the buffer together.
+    size_t rows = 0, rows_max = 0;
+    std::vector<int> in_group;
+    auto close_group = [&] {
+        if (in_group.empty()) return;
+        SymGroup g{static_cast<int>(tasks.size()), 0, static_cast<int>(sums.size()), 0};
+        for (const bool diagonal : {false, true})  // the shorter tasks last
+            for (int s : in_group) {
+                const SymPlan& P = descs[s].sym;
+                for (int d = diagonal ? 0 : 1; d <= (diagonal ? 0 : P.nsb / 2); ++d)
+                    for (int a = 0; a < (d > 0 && 2 * d == P.nsb ? d : P.nsb); ++a)
+                        for (int h = 0; h < P.split; ++h) tasks.push_back(SymTask{s, a, d, h});
+            }
+        for (int s : in_group)
+            for (int i = 0; i < descs[s].n; i += 64) sums.push_back(SumItem{s, i});
+        g.task1 = static_cast<int>(tasks.size());
+        g.sum1 = static_cast<int>(sums.size());
+        groups.push_back(g);
+        in_group.clear();
+        rows_max = std::max(rows_max, rows);
+        rows = 0;
+    };
     for (int s : order) {
         const auto& y = b->systems[s];
         inter += static_cast<uint64_t>(y.n) * y.n;
-        for (size_t i = 0; i < y.n_pad; i += per) items.push_back(WorkItem{s, static_cast<int>(i)});
+        const SymPlan P = b->no_rows ? SymPlan{} : batch_sym_plan(y.n_pad);
+        if (P.nsb > 0) {
+            const size_t need = sym_part_records(P, static_cast<int>(y.n_pad)) * 4;
+            if ((rows + need) * sizeof(float) > kRowsBytes) close_group();
+            descs[s].sym = P;
+            descs[s].rows = rows;
+            rows += need;
+            in_group.push_back(s);
+        } else {
+            for (size_t i = 0; i < y.n_pad; i += per) items.push_back(WorkItem{s, static_cast<int>(i)});
+        }
     }
-    NB_TRY(ensure_dev(reinterpret_cast<void**>(&b->d_items), b->items_cap, std::max<size_t>(items.size(), 1),
-                      sizeof(WorkItem), b->stream));
-    NB_TRY(ensure_dev(reinterpret_cast<void**>(&b->d_sys), b->sys_cap, std::max<size_t>(descs.size(), 1),
-                      sizeof(SysDesc), b->stream));
-    // The graph holds the item and descriptor pointers: a reallocation above
-    // invalidates it.
-    if (!items.empty())
-        NB_HIP(hipMemcpyAsync(b->d_items, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice,
-                              b->stream));
-    if (!descs.empty())
-        NB_HIP(hipMemcpyAsync(b->d_sys, descs.data(), descs.size() * sizeof(SysDesc), hipMemcpyHostToDevice,
-                              b->stream));
+    close_group();
+    if (rows_max > b->rows_cap) {
+        const nbody_status st = ensure_dev(reinterpret_cast<void**>(&b->d_rows), b->rows_cap, rows_max, sizeof(float),
+                                           b->stream, kRowsBytes / sizeof(float));
+        if (st == NBODY_ERR_OUT_OF_MEMORY) {
+            // A device too full for the rows: the one-sided sum for every
+            // system, from now on.
+            (void)hipGetLastError();
+            clear_error();
+            b->no_rows = true;
+            return rebuild_items(b);
+        }
+        NB_TRY(st);
+    }
+    auto upload = [&](auto** dev, size_t& cap, const auto& host) -> nbody_status {
+        const size_t elem = sizeof(host[0]);
+        NB_TRY(ensure_dev(reinterpret_cast<void**>(dev), cap, std::max<size_t>(host.size(), 1), elem, b->stream));
+        if (!host.empty())
+            NB_HIP(hipMemcpyAsync(*dev, host.data(), host.size() * elem, hipMemcpyHostToDevice, b->stream));
+        return NBODY_OK;
+    };
+    // The graph holds these pointers: a reallocation invalidates it.
+    NB_TRY(upload(&b->d_items, b->items_cap, items));
+    NB_TRY(upload(&b->d_sys, b->sys_cap, descs));
+    NB_TRY(upload(&b->d_tasks, b->tasks_cap, tasks));
+    NB_TRY(upload(&b->d_sums, b->sums_cap, sums));
+    NB_TRY(upload(&b->d_groups, b->groups_cap, groups));
     b->n_items = static_cast<int>(items.size());
+    b->n_tasks = static_cast<int>(tasks.size());
+    b->n_groups = static_cast<int>(groups.size());
     NB_HIP(hipMemcpyAsync(b->d_n_items, &b->n_items, sizeof(int), hipMemcpyHostToDevice, b->stream));
     NB_HIP(hipStreamSynchronize(b->stream));  // host vectors go out of scope
     b->interactions_per_step = inter;
@@ -327,20 +497,35 @@ BatchLaunch launch_for(nbody_batch* b, int parity, float dt) {
     L.sys = b->d_sys;
     L.items = b->d_items;
     L.n_items = b->d_n_items;
+    L.tasks = b->d_tasks;
+    L.sums = b->d_sums;
+    L.groups = b->d_groups;
+    L.rows = b->d_rows;
     L.dt = dt;
     L.dts = static_cast<float>(static_cast<double>(dt) / b->cfg.scale);
     return L;
 }
 
+// Counters a step needs: one for the one-sided items and one per group.
+int counters_per_step(const nbody_batch* b) { return 1 + b->n_groups; }
+
 // Enqueue nsteps persistent launches on the batch stream (captured or not).
 nbody_status enqueue_steps(nbody_batch* b, float dt, int nsteps) {
     BatchFn fn = pick(b->cfg.law, b->tuning.i_per_lane, b->tuning.block);
     NB_CHECK(fn, NBODY_ERR_INVALID_ARG, "no batch kernel for this tuning");
-    hipLaunchKernelGGL(fill_u32_kernel, dim3((nsteps + 255) / 256), dim3(256), 0, b->stream, b->d_counters, nsteps, 0u);
+    const int per = counters_per_step(b), counters = per * nsteps;
+    hipLaunchKernelGGL(fill_u32_kernel, dim3((counters + 255) / 256), dim3(256), 0, b->stream, b->d_counters, counters, 0u);
     const dim3 grid(static_cast<unsigned>(b->tuning.wg_per_cu * b->cus));
+    const auto sym = b->cfg.law == NBODY_LAW_R ? batch_sym_kernel<NBODY_LAW_R> : batch_sym_kernel<NBODY_LAW_P>;
     int parity = b->cur;
     for (int s = 0; s < nsteps; ++s) {
-        hipLaunchKernelGGL(fn, grid, dim3(b->tuning.block), 0, b->stream, launch_for(b, parity, dt), b->d_counters + s);
+        const BatchLaunch L = launch_for(b, parity, dt);
+        unsigned* counter = b->d_counters + static_cast<size_t>(s) * per;
+        for (int g = 0; g < b->n_groups; ++g) {
+            hipLaunchKernelGGL(sym, dim3(6 * b->cus), dim3(kTile), 0, b->stream, L, g, counter + 1 + g);
+            hipLaunchKernelGGL(batch_sum_kernel, dim3(8 * b->cus), dim3(256), 0, b->stream, L, g);
+        }
+        if (b->n_items > 0) hipLaunchKernelGGL(fn, grid, dim3(b->tuning.block), 0, b->stream, L, counter);
         parity ^= 1;
     }
     NB_HIP(hipGetLastError());
@@ -401,7 +586,9 @@ nbody_status nbody_batch_destroy(nbody_batch* b) {
     release_stage(b->read_stage);
     for (void* p : {static_cast<void*>(b->pos[0]), static_cast<void*>(b->pos[1]), static_cast<void*>(b->vel),
                     static_cast<void*>(b->acc), static_cast<void*>(b->d_sys), static_cast<void*>(b->d_items),
-                    static_cast<void*>(b->d_n_items), static_cast<void*>(b->d_counters), static_cast<void*>(b->part),
+                    static_cast<void*>(b->d_n_items), static_cast<void*>(b->d_tasks), static_cast<void*>(b->d_sums),
+                    static_cast<void*>(b->d_groups), static_cast<void*>(b->d_rows), static_cast<void*>(b->d_counters),
+                    static_cast<void*>(b->part),
                     static_cast<void*>(b->ic_scratch)})
         if (p) (void)hipFree(p);
     for (hipEvent_t e : b->ev)
@@ -424,10 +611,13 @@ nbody_status nbody_batch_add(nbody_batch* b, const float* pos3, const float* vel
     NB_TRY(arena_alloc(b, n_pad, &off));
     std::vector<float4> hp(n_pad, make_float4(0.f, 0.f, 0.f, 0.f)), hv(n_pad, make_float4(0.f, 0.f, 0.f, 0.f));
     double max_gm = 0.0;
+    const float gm0 = static_cast<float>(b->cfg.G * mass[0]);
+    bool equal = gm0 > 0.f && std::isfinite(gm0);
     float lo[3] = {pos3[0], pos3[1], pos3[2]}, hi[3] = {pos3[0], pos3[1], pos3[2]};
     for (size_t i = 0; i < n; ++i) {
         const double gm = b->cfg.G * mass[i];
         max_gm = std::max(max_gm, std::fabs(gm));
+        equal = equal && static_cast<float>(gm) == gm0;
         hp[i] = make_float4(pos3[3 * i], pos3[3 * i + 1], pos3[3 * i + 2], static_cast<float>(gm));
         if (vel3) hv[i] = make_float4(vel3[3 * i], vel3[3 * i + 1], vel3[3 * i + 2], 0.f);
         for (int c = 0; c < 3; ++c) {
@@ -462,6 +652,7 @@ nbody_status nbody_batch_add(nbody_batch* b, const float* pos3, const float* vel
     y.n = n;
     y.n_pad = n_pad;
     y.max_gm = max_gm;
+    y.gm_equal = equal ? gm0 : 0.f;
     y.sc = direct_scale_for(b->cfg.law, b->cfg.softening, extent, max_gm);
     b->items_dirty = true;
     *id = slot;
@@ -505,6 +696,8 @@ nbody_status nbody_batch_add_plummer(nbody_batch* b, uint64_t seed, size_t n, do
     y.n = n;
     y.n_pad = n_pad;
     y.max_gm = std::fabs(b->cfg.G * total_mass / static_cast<double>(n));
+    const float gm = static_cast<float>(b->cfg.G * (total_mass / static_cast<double>(n)));
+    y.gm_equal = gm > 0.f && std::isfinite(gm) ? gm : 0.f;
     // Plummer radii are cut at 20 a, so the sphere spans at most 40 a
     y.sc = direct_scale_for(b->cfg.law, b->cfg.softening, 40.0 * a, y.max_gm);
     b->items_dirty = true;
@@ -537,18 +730,24 @@ nbody_status nbody_batch_step(nbody_batch* b, float dt, int32_t nsteps) {
     b->last_interactions = 0;
     b->timed = false;
     if (nsteps == 0) return NBODY_OK;
-    const void* old_items = b->d_items;
-    const void* old_sys = b->d_sys;
+    // What a captured graph holds besides its own (steps, dt, launch shape).
+    const auto held = [b] {
+        return std::make_tuple(b->d_items, b->d_sys, b->d_tasks, b->d_sums, b->d_groups, b->d_rows, b->n_groups,
+                               b->n_items > 0);
+    };
+    const auto before = held();
     NB_TRY(rebuild_items(b));
-    if (b->d_items != old_items || b->d_sys != old_sys) drop_graph(b);
-    if (b->n_items == 0) return NBODY_OK;
-    if (static_cast<int>(nsteps) > b->counters_cap) {
+    if (held() != before) drop_graph(b);
+    if (b->n_items == 0 && b->n_tasks == 0) return NBODY_OK;
+    const int counters = counters_per_step(b) * nsteps;
+    if (counters > b->counters_cap) {
         drop_graph(b);
         NB_HIP(hipStreamSynchronize(b->stream));  // plain launches may still use the counters
         if (b->d_counters) (void)hipFree(b->d_counters);
         b->d_counters = nullptr;
-        NB_HIP(hipMalloc(reinterpret_cast<void**>(&b->d_counters), static_cast<size_t>(nsteps) * sizeof(unsigned)));
-        b->counters_cap = nsteps;
+        b->counters_cap = 0;
+        NB_HIP(hipMalloc(reinterpret_cast<void**>(&b->d_counters), static_cast<size_t>(counters) * sizeof(unsigned)));
+        b->counters_cap = counters;
     }
     NB_HIP(hipEventRecord(b->ev[0], b->stream));
     if (b->use_graph) {
@@ -696,7 +895,7 @@ nbody_status nbody_batch_get_info(nbody_batch* b, nbody_batch_info* out) {
             out->particles += y.n;
         }
     out->interactions_per_step = b->interactions_per_step;
-    out->work_items = b->n_items;
+    out->work_items = b->n_items + b->n_tasks;
     out->capacity = b->capacity;
     size_t free_total = 0, largest = 0;
     for (const auto& f : b->free_list) {
@@ -756,7 +955,7 @@ nbody_status nbody_batch_tune(nbody_batch* b, float dt, nbody_batch_tuning* out)
     NB_CHECK(b, NBODY_ERR_INVALID_ARG, "batch is null");
     NB_HIP(hipSetDevice(b->cfg.device));
     NB_TRY(rebuild_items(b));
-    if (b->n_items == 0) {
+    if (b->n_items == 0 && b->n_tasks == 0) {
         if (out) *out = b->tuning;
         return NBODY_OK;
     }
