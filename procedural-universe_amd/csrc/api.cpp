@@ -169,6 +169,9 @@ nbody_status prepare_state(nbody_sim* s, size_t n) {
     const bool direct = s->cfg.method == NBODY_METHOD_DIRECT || n < 2;
     const bool tuned = s->cfg.tune_i_per_lane || s->cfg.tune_block || s->cfg.tune_split;
     s->sym = direct && !tuned ? sym_plan(static_cast<int>(n_pad)) : SymPlan{};
+    // below the sizes that take unordered pairs
+    s->small = s->cfg.method == NBODY_METHOD_DIRECT && !tuned && s->sym.nsb == 0;
+    if (s->small) return NBODY_OK;
     if (s->sym.nsb > 0) {
         const size_t need = sym_part_records(s->sym, static_cast<int>(n_pad));
         if (need <= s->part_elems) return NBODY_OK;
@@ -310,9 +313,9 @@ DirectLaunch launch_for(nbody_sim* s, float dt) {
 // The launch shape in use, for nbody_get_timing.
 void report_shape(nbody_sim* s) {
     const bool sym = s->sym.nsb > 0;
-    s->last.i_per_lane = sym ? 4 : s->shape.i_per_lane;
-    s->last.block = sym ? kTile : s->shape.block;
-    s->last.split = sym ? s->sym.split : direct_effective_split(s->shape, static_cast<int>(s->n_pad));
+    s->last.i_per_lane = sym ? 4 : s->small ? 1 : s->shape.i_per_lane;
+    s->last.block = sym ? kTile : s->small ? 1024 : s->shape.block;
+    s->last.split = sym ? s->sym.split : s->small ? 1 : direct_effective_split(s->shape, static_cast<int>(s->n_pad));
 }
 
 // One force evaluation (kick: a full step).  ev_b/ev_e bracket the force kernel(s).
@@ -321,8 +324,9 @@ nbody_status force_pass(nbody_sim* s, float dt, bool kick, hipEvent_t ev_b, hipE
         NB_TRY(bh_step(s, dt, kick, ev_b, ev_e));
     } else {
         DirectLaunch L = launch_for(s, dt);
-        NB_HIP(s->sym.nsb > 0 ? sym_step(L, s->sym, kick, s->stream, ev_b, ev_e)
-                              : direct_step(L, s->shape, kick, s->stream, ev_b, ev_e));
+        NB_HIP(s->small         ? small_step(L, kick, s->stream, ev_b, ev_e)
+               : s->sym.nsb > 0 ? sym_step(L, s->sym, kick, s->stream, ev_b, ev_e)
+                                : direct_step(L, s->shape, kick, s->stream, ev_b, ev_e));
         s->step_interactions += static_cast<uint64_t>(s->n) * static_cast<uint64_t>(s->n);
     }
     if (kick) s->cur ^= 1;

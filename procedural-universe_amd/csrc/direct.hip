@@ -106,6 +106,119 @@ __global__ __launch_bounds__(256) void reduce_kick_kernel(DirectLaunch L, int sp
     if (kick) kick_drift(L, i, ax, ay, az);
 }
 
+// A whole step of a small system in one launch.  A workgroup of sixteen
+// wavefronts owns T targets and all sources: a wavefront holds its T targets
+// 64 / T times over, and each of the 1,024 / T copies takes every (1,024 / T)-th
+// source of a tile of 1,024, so that a system of a few thousand particles fills
+// the chip without chunks of sources whose sums a second kernel has to add.
+// The copies' compensated sums are added lane by lane, then wave by wave, in a
+// fixed order.  The pair is unfolded (13 FP32 instructions and one v_rsq_f32,
+// the mass multiplied in last): folding it costs a division per staged source,
+// and every workgroup stages them all.
+//
+// Bound by latency up to about 4,000 particles (a launch, the staging, one to
+// four tiles), then by the pair arithmetic.  A step, ms, against the chunked
+// one-sided sum and its second kernel, with T = 8 / 16 targets: 1,000 particles
+// 0.0127 -> 0.0050 / 0.0053; 2,000 0.0130 -> 0.0062 / 0.0070; 3,000 0.0152 ->
+// 0.0095 / 0.0087; 4,096 0.0147 -> 0.0112 / 0.0103; 8,192 0.0276 -> 0.0299 /
+// 0.0252; 12,288 0.0549 -> 0.0600 / 0.0516.  (T = 4 and 32 lose everywhere.)
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallWaves = kSmallThreads / 64;
+
+template <int LAW, int T, bool KICK>
+__global__ __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(8))) void small_step_kernel(DirectLaunch L) {
+    constexpr int COPIES = kSmallThreads / T;       // copies of each target
+    constexpr int PER = kSmallThreads / COPIES;     // sources a copy takes of a tile
+    static_assert(PER % 4 == 0, "whole groups of four reciprocal square roots");
+    __shared__ float4 tile[2][kSmallThreads];
+    __shared__ float sums[6][kSmallWaves][T];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int i = blockIdx.x * T + (lane & (T - 1));
+    const int copy = wave * (64 / T) + lane / T;
+    const float tiny = core::in_vgpr(__FLT_MIN__);
+    const float soft = core::in_vgpr(L.sc.soft);
+    const float inv_c = LAW == NBODY_LAW_R ? 1.0f / L.sc.mass_k : L.sc.mass_k;  // a power of two
+    auto scaled = [&](int j) {
+        const float4 p = j < L.n_pad ? L.src[j] : make_float4(0.f, 0.f, 0.f, 0.f);
+        return make_float4(p.x * L.sc.inv_len, p.y * L.sc.inv_len, p.z * L.sc.inv_len, p.w * inv_c);
+    };
+    const float4 me = scaled(min(i, L.n_pad - 1));
+    float s[3] = {0.f, 0.f, 0.f}, c[3] = {0.f, 0.f, 0.f};
+    tile[0][tid] = scaled(tid);
+    __syncthreads();
+    int buf = 0;
+    for (int jt = 0; jt < L.n_pad; jt += kSmallThreads) {
+        const bool more = jt + kSmallThreads < L.n_pad;
+        float4 next;
+        if (more) next = scaled(jt + kSmallThreads + tid);
+        float ax = 0.f, ay = 0.f, az = 0.f;
+#pragma unroll 2
+        for (int g = 0; g < PER; g += 4) {
+            float4 p[4];
+            float dx[4], dy[4], dz[4], q[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                p[k] = tile[buf][(g + k) * COPIES + copy];
+                dx[k] = p[k].x - me.x;
+                dy[k] = p[k].y - me.y;
+                dz[k] = p[k].z - me.z;
+                if constexpr (LAW == NBODY_LAW_R) {
+                    const float r2 = __builtin_fmaf(dz[k], dz[k], __builtin_fmaf(dy[k], dy[k], dx[k] * dx[k]));
+                    const float t = r2 + soft;
+                    const float u = r2 * t;
+                    q[k] = __builtin_fmaf(u, t, tiny);
+                } else {
+                    q[k] = __builtin_fmaf(dz[k], dz[k], __builtin_fmaf(dy[k], dy[k], __builtin_fmaf(dx[k], dx[k], soft)));
+                }
+            }
+            core::rsq4(q[0], q[1], q[2], q[3]);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float f = LAW == NBODY_LAW_R ? q[k] * p[k].w : (p[k].w * q[k]) * (q[k] * q[k]);
+                ax = __builtin_fmaf(dx[k], f, ax);
+                ay = __builtin_fmaf(dy[k], f, ay);
+                az = __builtin_fmaf(dz[k], f, az);
+            }
+        }
+        kahan_add(s[0], c[0], ax);
+        kahan_add(s[1], c[1], ay);
+        kahan_add(s[2], c[2], az);
+        if (more) {
+            // the other buffer was last read before the previous barrier
+            tile[buf ^ 1][tid] = next;
+            __syncthreads();
+            buf ^= 1;
+        }
+    }
+#pragma unroll
+    for (int off = T; off < 64; off <<= 1) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const float os = __shfl_xor(s[a], off), oc = __shfl_xor(c[a], off);
+            kahan_add(s[a], c[a], os);
+            kahan_add(s[a], c[a], -oc);
+        }
+    }
+    if (lane < T) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            sums[a][wave][lane] = s[a];
+            sums[3 + a][wave][lane] = c[a];
+        }
+    }
+    __syncthreads();
+    if (tid >= T || i >= L.n) return;
+    for (int w = 1; w < kSmallWaves; ++w)
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            kahan_add(s[a], c[a], sums[a][w][lane]);
+            kahan_add(s[a], c[a], -sums[3 + a][w][lane]);
+        }
+    const float ax = s[0] * L.sc.out, ay = s[1] * L.sc.out, az = s[2] * L.sc.out;
+    L.acc[i] = make_float4(ax, ay, az, 0.f);
+    if constexpr (KICK) kick_drift(L, i, ax, ay, az);
+}
+
 // Acceleration at arbitrary points (3m packed floats) from all sources: one
 // target per lane, every workgroup over the whole source range.
 template <int LAW>
@@ -302,6 +415,23 @@ hipError_t direct_field(const float4* src, int n_src_pad, const float* pts, int 
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(field_sum_kernel, dim3((m + 255) / 256), dim3(256), 0, stream, part, split, m, sc, out);
     return hipGetLastError();
+}
+
+hipError_t small_step(const DirectLaunch& L, bool kick, hipStream_t stream, hipEvent_t ev_b, hipEvent_t ev_e) {
+    using Fn = void (*)(DirectLaunch);
+    const bool r = L.law == NBODY_LAW_R;
+    // Fewer targets a workgroup while the workgroups do not fill the 256 CUs.
+    const int t = L.n_pad <= 2048 ? 8 : 16;
+    const Fn fn = t == 8 ? (r ? (kick ? small_step_kernel<NBODY_LAW_R, 8, true> : small_step_kernel<NBODY_LAW_R, 8, false>)
+                              : (kick ? small_step_kernel<NBODY_LAW_P, 8, true> : small_step_kernel<NBODY_LAW_P, 8, false>))
+                         : (r ? (kick ? small_step_kernel<NBODY_LAW_R, 16, true> : small_step_kernel<NBODY_LAW_R, 16, false>)
+                              : (kick ? small_step_kernel<NBODY_LAW_P, 16, true> : small_step_kernel<NBODY_LAW_P, 16, false>));
+    hipError_t e = hipSuccess;
+    if (ev_b && (e = hipEventRecord(ev_b, stream)) != hipSuccess) return e;
+    hipLaunchKernelGGL(fn, dim3((L.n + t - 1) / t), dim3(kSmallThreads), 0, stream, L);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if (ev_e && (e = hipEventRecord(ev_e, stream)) != hipSuccess) return e;
+    return hipSuccess;
 }
 
 hipError_t direct_step(const DirectLaunch& L, const DirectShape& s, bool kick, hipStream_t stream,

@@ -74,6 +74,11 @@ DirectShape direct_default_shape(int n_pad);
 hipError_t direct_step(const DirectLaunch& L, const DirectShape& s, bool kick, hipStream_t stream,
                        hipEvent_t ev_force_begin, hipEvent_t ev_force_end);
 
+// Whole steps of small systems in one launch each, as direct_step without
+// partial sums.
+hipError_t small_step(const DirectLaunch& L, bool kick, hipStream_t stream, hipEvent_t ev_force_begin,
+                      hipEvent_t ev_force_end);
+
 // The sum over unordered pairs (direct_sym.hip): nsb blocks of `block`
 // particles, every streamed block cut into `split` runs.
 struct SymPlan {
