@@ -14,11 +14,10 @@
 //                    power of two (exact), floored, and divided by the odd part
 //                    of the root size in integers, so keys equal the CPU's bit
 //                    for bit and the cells are the reference's half-open cubes;
-//  3. sort           least-significant-digit radix sort of (key, index), eight
-//                    8-bit passes of histogram / scan / scatter; the scatter
-//                    ranks equal digits with wave ballots, orders each tile by
-//                    digit in LDS and writes it out in runs, so the order is
-//                    stable and equals std::stable_sort of the keys;
+//  3. sort           merge sort of (key, index): the keys are formed and sorted
+//                    in LDS in tiles of 4,096, then pairs of sorted runs are
+//                    merged, the earlier run first among equal keys, so the
+//                    order is stable and equals std::stable_sort of the keys;
 //  4. radix tree     binary radix tree over the sorted keys (Karras 2012);
 //                    a node whose common prefix reaches a deeper 3-bit group
 //                    than its parent's is an octree cell ("kept"), the others
@@ -79,21 +78,6 @@ namespace {
 
 constexpr int kLevels = 21;
 constexpr int kBucketLevel = kLevels;
-constexpr int kSortThreads = 256;
-// Keys per thread of a sort tile (tile = 256 x items keys): small systems take
-// small tiles for more workgroups per pass, large ones large tiles for fewer
-// tile counts to scan (measured tree builds: 0.19 / 0.21 / 0.24 ms at 65,536
-// particles with 2 / 4 / 8 items, 1.66 / 1.43 / 1.30 ms at 4,194,304).
-inline int sort_items(size_t n) { return n <= (size_t(1) << 17) ? 2 : n <= (size_t(1) << 20) ? 4 : 8; }
-// The most tiles of any system of at most n particles (the tile grows with
-// the size, so a smaller system can have more tiles than a larger one): the
-// count buffer of a handle holds that many, whatever size it runs later.
-inline size_t sort_max_tiles(size_t n) {
-    const auto tiles = [](size_t k, size_t tile) { return (k + tile - 1) / tile; };
-    size_t t = tiles(std::min(n, size_t(1) << 17), kSortThreads * 2);
-    t = std::max(t, tiles(std::min(n, size_t(1) << 20), kSortThreads * 4));
-    return std::max(t, tiles(n, kSortThreads * 8));
-}
 constexpr int kTravThreads = 64;  // one wavefront per workgroup: the finest tail
 constexpr int kTravWaves = kTravThreads / 64;
 // Pending (cell, lanes) entries per wave.  Popping one cell at a time (a
@@ -304,109 +288,19 @@ __global__ __launch_bounds__(256) void dynamic_root_kernel(const float* __restri
 
 // ---- 2. keys ---------------------------------------------------------------
 
-__global__ __launch_bounds__(256) void keys_kernel(const float4* __restrict__ pos, int n,
-                                                   const RootParams* __restrict__ Rp,
-                                                   unsigned long long* __restrict__ keys,
-                                                   unsigned* __restrict__ idx, unsigned* __restrict__ outside) {
-    build_priority();
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const RootParams R = *Rp;
-    const double inv_odd = 1.0 / static_cast<double>(R.odd);
-    const float4 p = pos[i];
+// A position's key; *out is set if it lies outside the root (clamped into it).
+__device__ inline unsigned long long position_key(const float4 p, const RootParams& R, double inv_odd, bool* out) {
     const float c[3] = {p.x, p.y, p.z};
     unsigned long long key = 0;
-    bool out = false;
+    bool outside = false;
     for (int a = 0; a < 3; ++a) {
         long long k = cell_index(c[a], R, a, inv_odd);
-        if (k < 0) k = 0, out = true;
-        if (k > 0x1fffff) k = 0x1fffff, out = true;
+        if (k < 0) k = 0, outside = true;
+        if (k > 0x1fffff) k = 0x1fffff, outside = true;
         key |= spread3(static_cast<unsigned long long>(k)) << a;
     }
-    keys[i] = key;
-    idx[i] = static_cast<unsigned>(i);
-    if (out) atomicAdd(outside, 1u);
-}
-
-// ---- 3. radix sort -----------------------------------------------------------
-
-// Digits of kRadixBits bits: kRadixPasses passes cover the 63-bit keys.
-// Nine-bit digits (seven passes) were slower from 131,072 keys up: a tile's
-// digit runs are half as long, so the scatter's writes coalesce less
-// (46.5 against 33 us per pass at 4,194,304 keys).
-constexpr int kRadixBits = 8;
-constexpr int kRadixBins = 1 << kRadixBits;
-constexpr unsigned kRadixMask = kRadixBins - 1;
-constexpr int kRadixPasses = (63 + kRadixBits - 1) / kRadixBits;
-constexpr int kDigitsPerThread = kRadixBins / kSortThreads;  // the digit phases' digits per thread
-static_assert(kRadixBins % kSortThreads == 0, "whole digits per thread");
-
-// Digit counts of each tile, digit-major (hist[d * nblocks + tile]).
-template <int ITEMS>
-__global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const unsigned long long* __restrict__ keys, int n,
-                                                                  int shift, unsigned* __restrict__ hist,
-                                                                  int nblocks) {
-    build_priority();
-    __shared__ unsigned h[kRadixBins];
-    for (int d = threadIdx.x; d < kRadixBins; d += kSortThreads) h[d] = 0;
-    __syncthreads();
-    const int base = blockIdx.x * kSortThreads * ITEMS;
-    for (int k = 0; k < ITEMS; ++k) {
-        const int i = base + k * kSortThreads + threadIdx.x;
-        if (i < n) atomicAdd(&h[(keys[i] >> shift) & kRadixMask], 1u);
-    }
-    __syncthreads();
-    for (int d = threadIdx.x; d < kRadixBins; d += kSortThreads) hist[d * nblocks + blockIdx.x] = h[d];
-}
-
-constexpr int kScanThreads2 = 256;
-constexpr int kScanPer = 16;
-
-__device__ inline unsigned block_exclusive_scan_u32(unsigned v, unsigned* sh, unsigned* total) {
-    const int t = threadIdx.x;
-    sh[t] = v;
-    __syncthreads();
-    for (int off = 1; off < kScanThreads2; off <<= 1) {
-        const unsigned a = t >= off ? sh[t - off] : 0u;
-        __syncthreads();
-        sh[t] += a;
-        __syncthreads();
-    }
-    const unsigned incl = sh[t];
-    if (total) *total = sh[kScanThreads2 - 1];
-    __syncthreads();
-    return incl - v;
-}
-
-// Workgroup d replaces digit d's row of tile counts by its exclusive scan
-// (the tile's offset among the keys with digit d) and writes the row's total
-// to totals[d]; the scatter adds the totals of the smaller digits.
-__global__ __launch_bounds__(kScanThreads2) void radix_rowscan_kernel(unsigned* __restrict__ hist, int nblocks,
-                                                                      unsigned* __restrict__ totals) {
-    build_priority();
-    __shared__ unsigned sh[kScanThreads2];
-    const int d = blockIdx.x, t = threadIdx.x;
-    unsigned* row = hist + static_cast<size_t>(d) * nblocks;
-    unsigned carry = 0;
-    for (int base = 0; base < nblocks; base += kScanThreads2 * kScanPer) {
-        const int at = base + t * kScanPer;  // a contiguous run per thread
-        unsigned v[kScanPer];
-        unsigned sum = 0;
-#pragma unroll
-        for (int k = 0; k < kScanPer; ++k) {
-            v[k] = at + k < nblocks ? row[at + k] : 0u;
-            sum += v[k];
-        }
-        unsigned chunk = 0;
-        unsigned run = carry + block_exclusive_scan_u32(sum, sh, &chunk);
-#pragma unroll
-        for (int k = 0; k < kScanPer; ++k) {
-            if (at + k < nblocks) row[at + k] = run;
-            run += v[k];
-        }
-        carry += chunk;
-    }
-    if (t == 0) totals[d] = carry;
+    *out = outside;
+    return key;
 }
 
 // Counters: walk[3] (interactions, list entries, cells opened) and
@@ -428,165 +322,231 @@ __global__ void publish_counters_kernel(const unsigned* __restrict__ counters,
     if (threadIdx.x >= 3 && threadIdx.x < 5) host[threadIdx.x] = counters[threadIdx.x - 3];
 }
 
-// One radix pass over a tile of 256 x ITEMS keys, stable.  Each wavefront owns
-// a contiguous share of the tile (ITEMS rounds of 64 consecutive keys) and
-// ranks every key among the earlier keys of its wavefront with the same digit
-// (the lanes with equal digits found by kRadixBits ballots, running per-digit
-// counts in LDS; no workgroup barrier).  One pass over the digits then gives each
-// wavefront's offset within the tile's digit run and the runs' starts; the
-// keys are placed in LDS in digit order and written out in that order, so
-// consecutive threads write consecutive addresses within a digit's run of the
-// output.
+// ---- 3. sort -----------------------------------------------------------------
 //
-// FUSED: `counts` holds the raw per-tile digit counts ([digit * nblocks +
-// tile], at most kFusedScanTiles tiles) and each workgroup forms its own
-// output places: thread d sums digit d's row before its tile and in total
-// (no separate scan launch).  Otherwise `counts` holds each tile's offset
-// among the keys of its digit and `totals` each digit's count (the row scan).
-// Either way one scan over the digits' totals gives the digits' starts.
-// GATHER (the last pass): the sorted positions are written beside the keys.
-constexpr int kSortWaves = kSortThreads / 64;
+// A merge sort, the index carried with the key: one launch forms the keys and
+// sorts tiles of 4,096 in LDS, and each further launch merges pairs of sorted
+// runs, the earlier run first among equal keys; the last one also writes the
+// sorted positions.  In a small system a launch is the cost (about 5 us however
+// little it does), in a large one the bytes: a merge reads and writes each key
+// once.  Eight radix passes of histogram, row scan and scatter, which this
+// replaced, took 17 to 24 launches and read the keys twice a pass.  Tree
+// build, us, radix / merge: 86 / 56 at 1,000 particles, 104 / 72 at 4,000,
+// 130 / 93 at 32,768, 172 / 131 at 200,003, 366 / 291 at 1,048,576,
+// 1,108 / 1,019 at 4,194,304, 4,450 / 4,287 at 16,777,216.
+//
+// The tile kernel is bound by one compute unit's arithmetic and LDS while there
+// are few tiles (28 us: keys 4.5, nine rounds of merging 1.3 to 2.2 each).
+// Eight keys per thread, four take the same time and sixteen 11 us more; the
+// same eight digit passes with ballots, all in LDS, took 37 us.
+constexpr int kTileItems = 8;
+constexpr int kTileThreads = 512;
+constexpr int kTileKeys = kTileThreads * kTileItems;
 
-// Above this many tiles the row scan's extra launch costs less than every
-// workgroup summing the digits' rows itself (measured: equal at 16 tiles,
-// 0.01 ms less at 32, 0.04 at 64, 0.24 at 256).
-constexpr int kFusedScanTiles = 16;
+// A tile's place in LDS: one key skipped in every 32, so that threads reading
+// four consecutive keys each do not meet in the same banks.
+__device__ constexpr int tile_at(int i) { return i + (i >> 5); }
 
-template <bool FUSED, bool GATHER, int ITEMS>
-__global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
-    const unsigned long long* __restrict__ keys_in, const unsigned* __restrict__ idx_in,
-    unsigned long long* __restrict__ keys_out, unsigned* __restrict__ idx_out, int n, int shift,
-    const unsigned* __restrict__ counts, const unsigned* __restrict__ totals, int nblocks,
-    const float4* __restrict__ pos_in, float4* __restrict__ pos_out) {
+template <bool GATHER>
+__global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(const float4* __restrict__ pos, int n,
+                                                                 const RootParams* __restrict__ Rp,
+                                                                 unsigned long long* __restrict__ keys,
+                                                                 unsigned* __restrict__ idx,
+                                                                 unsigned* __restrict__ outside,
+                                                                 float4* __restrict__ pos_out) {
     build_priority();
-    constexpr int kSortTile = kSortThreads * ITEMS;
-    constexpr int kSortPerWave = 64 * ITEMS;  // a wavefront's share: ITEMS rounds of 64 keys
-    __shared__ unsigned cnt[kSortWaves][kRadixBins];  // per-wave digit counts, then per-wave offsets in the run
-    __shared__ unsigned run_start[kRadixBins];        // the tile's digit runs
-    __shared__ unsigned dst_base[kRadixBins];         // the runs' places in the output
-    __shared__ unsigned wave_sum[2][kSortWaves];
-    __shared__ unsigned long long skeys[kSortTile];
-    __shared__ unsigned sidx[kSortTile];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const unsigned long long below = (1ULL << lane) - 1ULL;
-    const int base = blockIdx.x * kSortTile;
-    const int wbase = base + wave * kSortPerWave;
+    __shared__ unsigned long long sk[tile_at(kTileKeys)];
+    __shared__ unsigned short sl[tile_at(kTileKeys)];
+    const int tid = threadIdx.x;
+    const int base = blockIdx.x * kTileKeys, count = min(kTileKeys, n - base);
+    const int mine = tid * kTileItems;  // this thread's keys, and its outputs of every merge
+    const RootParams R = *Rp;
+    const double inv_odd = 1.0 / static_cast<double>(R.odd);
+    unsigned long long key[kTileItems];
+    unsigned loc[kTileItems];
 #pragma unroll
-    for (int d = lane; d < kRadixBins; d += 64) cnt[wave][d] = 0u;  // this wave's counters only
-    unsigned long long key[ITEMS];
-    unsigned idx[ITEMS], rank[ITEMS];
-#pragma unroll
-    for (int r = 0; r < ITEMS; ++r) {
-        const int i = wbase + r * 64 + lane;
-        const bool valid = i < n;
-        key[r] = valid ? keys_in[i] : 0ULL;
-        idx[r] = valid ? idx_in[i] : 0u;
-        const unsigned digit = static_cast<unsigned>((key[r] >> shift) & kRadixMask);
-        unsigned long long peers = __builtin_amdgcn_ballot_w64(valid);
-#pragma unroll
-        for (int bit = 0; bit < kRadixBits; ++bit) {
-            const bool set = (digit >> bit) & 1u;
-            const unsigned long long bm = __builtin_amdgcn_ballot_w64(valid && set);
-            peers &= set ? bm : ~bm;
+    for (int k = 0; k < kTileItems; ++k) {
+        const int i = k * kTileThreads + tid;
+        unsigned long long v = ~0ULL;  // past the end: after every key
+        if (i < count) {
+            bool out;
+            v = position_key(pos[base + i], R, inv_odd, &out);
+            if (out) atomicAdd(outside, 1u);
         }
-        const unsigned within = static_cast<unsigned>(__popcll(peers & below));
-        const unsigned prior = valid ? cnt[wave][digit] : 0u;  // read by every lane before the leader's update
-        rank[r] = prior + within;
-        __builtin_amdgcn_wave_barrier();
-        if (valid && within == 0) cnt[wave][digit] = prior + static_cast<unsigned>(__popcll(peers));
-        __builtin_amdgcn_wave_barrier();
-    }
-    __syncthreads();
-    {
-        // Thread tid's kDigitsPerThread consecutive digits: offsets of the
-        // wavefronts' shares within each digit's run and the run's length,
-        // then the runs' starts (an exclusive scan over digits)
-        constexpr int D = kDigitsPerThread;
-        unsigned run[D], before[D], total[D];
-        unsigned rsum = 0, tsum = 0;
-#pragma unroll
-        for (int j = 0; j < D; ++j) {
-            const int d = tid * D + j;
-            unsigned acc = 0;
-#pragma unroll
-            for (int w = 0; w < kSortWaves; ++w) {
-                const unsigned c = cnt[w][d];
-                cnt[w][d] = acc;
-                acc += c;
-            }
-            run[j] = acc;
-            // digit d's place in the output: the digit's start (the totals of
-            // the smaller digits) plus the tile's offset among the digit's
-            // keys, both formed here from the raw counts or given by the row
-            // scan
-            before[j] = 0;
-            total[j] = 0;
-            if constexpr (FUSED) {
-                const unsigned* row = counts + static_cast<size_t>(d) * nblocks;
-                for (int b = 0; b < nblocks; ++b) {
-                    const unsigned c = row[b];
-                    before[j] += b < static_cast<int>(blockIdx.x) ? c : 0u;
-                    total[j] += c;
-                }
-            } else {
-                before[j] = counts[d * nblocks + blockIdx.x];
-                total[j] = totals[d];
-            }
-            rsum += run[j];
-            tsum += total[j];
-        }
-        unsigned x = rsum, y = tsum;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const unsigned xs = __shfl_up(x, off, 64);
-            const unsigned ys = __shfl_up(y, off, 64);
-            if (lane >= off) {
-                x += xs;
-                y += ys;
-            }
-        }
-        if (lane == 63) {
-            wave_sum[0][wave] = x;
-            wave_sum[1][wave] = y;
-        }
-        __syncthreads();
-        unsigned start = x - rsum, digit_start = y - tsum;
-        for (int w = 0; w < wave; ++w) {
-            start += wave_sum[0][w];
-            digit_start += wave_sum[1][w];
-        }
-#pragma unroll
-        for (int j = 0; j < D; ++j) {
-            const int d = tid * D + j;
-            run_start[d] = start;
-            dst_base[d] = digit_start + before[j];
-            start += run[j];
-            digit_start += total[j];
-        }
+        sk[tile_at(i)] = v;
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < ITEMS; ++r) {
-        const int i = wbase + r * 64 + lane;
-        if (i < n) {
-            const unsigned digit = static_cast<unsigned>((key[r] >> shift) & kRadixMask);
-            const unsigned at = run_start[digit] + cnt[wave][digit] + rank[r];
-            skeys[at] = key[r];
-            sidx[at] = idx[r];
+    for (int k = 0; k < kTileItems; ++k) {
+        key[k] = sk[tile_at(mine + k)];
+        loc[k] = static_cast<unsigned>(mine + k);
+    }
+    // neighbours change places only where they are strictly out of order
+#pragma unroll
+    for (int phase = 0; phase < kTileItems; ++phase)
+#pragma unroll
+        for (int k = phase & 1; k + 1 < kTileItems; k += 2)
+            if (key[k] > key[k + 1]) {
+                const unsigned long long t = key[k];
+                key[k] = key[k + 1];
+                key[k + 1] = t;
+                const unsigned l = loc[k];
+                loc[k] = loc[k + 1];
+                loc[k + 1] = l;
+            }
+#pragma unroll 1
+    for (int w = kTileItems; w < count; w *= 2) {
+        // a wavefront's runs of up to 256 keys are its own: no other waits for it
+        const bool alone = 2 * w <= 64 * kTileItems;
+        if (!alone) __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kTileItems; ++k) {
+            sk[tile_at(mine + k)] = key[k];
+            sl[tile_at(mine + k)] = static_cast<unsigned short>(loc[k]);
+        }
+        if (alone) __builtin_amdgcn_wave_barrier();
+        else __syncthreads();
+        const int A = mine & ~(2 * w - 1), B = A + w, d = mine - A;
+        int lo = max(0, d - w), hi = min(d, w);
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (sk[tile_at(A + mid)] <= sk[tile_at(B + d - 1 - mid)]) lo = mid + 1;
+            else hi = mid;
+        }
+        int a = A + lo, b = B + d - lo;
+        unsigned long long ka = sk[tile_at(min(a, B - 1))], kb = sk[tile_at(min(b, B + w - 1))];
+#pragma unroll
+        for (int k = 0; k < kTileItems; ++k) {
+            const bool from_a = a < B && (b >= B + w || ka <= kb);
+            const int at = from_a ? a++ : b++;
+            key[k] = from_a ? ka : kb;
+            loc[k] = sl[tile_at(at)];
+            if (k + 1 < kTileItems) {
+                const unsigned long long next = sk[tile_at(from_a ? min(a, B - 1) : min(b, B + w - 1))];
+                if (from_a) ka = next;
+                else kb = next;
+            }
+        }
+        if (alone) __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kTileItems; ++k) {
+        sk[tile_at(mine + k)] = key[k];
+        sl[tile_at(mine + k)] = static_cast<unsigned short>(loc[k]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kTileItems; ++k) {
+        const int i = k * kTileThreads + tid;
+        if (i < count) {
+            const unsigned from = static_cast<unsigned>(base) + sl[tile_at(i)];
+            keys[base + i] = sk[tile_at(i)];
+            idx[base + i] = from;
+            if constexpr (GATHER) pos_out[base + i] = pos[from];
+        }
+    }
+}
+
+// Where the merge of sorted runs A (la keys) and B (lb keys) stands after d
+// outputs: the number of them that come from A (A's first among equals).  Every
+// lane of the wavefront searches with a probe of its own: three rounds for runs
+// of up to 2^18 keys instead of eighteen dependent loads.
+__device__ inline int merge_split(const unsigned long long* __restrict__ A, int la,
+                                  const unsigned long long* __restrict__ B, int lb, int d, int lane) {
+    int lo = max(0, d - lb), hi = min(d, la);  // the answer is in [lo, hi]
+    while (lo < hi) {
+        // A[p] is among the first d outputs iff A[p] <= B[d - 1 - p]: true up to
+        // the answer, false from it on
+        const int step = (hi - lo + 63) / 64;
+        const int p = lo + lane * step;
+        const bool in = p < hi && A[p] <= B[d - 1 - p];
+        const int k = static_cast<int>(__popcll(__builtin_amdgcn_ballot_w64(in)));  // probes passed
+        if (step == 1) return lo + k;
+        if (k == 0) return lo;
+        lo += (k - 1) * step + 1;
+        hi = min(hi, lo + step - 1);
+    }
+    return lo;
+}
+
+// Merges the pairs of sorted runs of `run` keys (the last pair may be short or
+// one run alone); a workgroup writes THREADS x ITEMS consecutive outputs (2 x run
+// is a multiple of that, so they belong to one pair).
+template <int THREADS, int ITEMS, bool GATHER>
+__global__ __launch_bounds__(THREADS) void merge_kernel(const unsigned long long* __restrict__ keys_in,
+                                                        const unsigned* __restrict__ idx_in,
+                                                        unsigned long long* __restrict__ keys_out,
+                                                        unsigned* __restrict__ idx_out, int n, int run,
+                                                        const float4* __restrict__ pos,
+                                                        float4* __restrict__ pos_out) {
+    constexpr int kMergeKeys = THREADS * ITEMS;
+    static_assert(2 * kTileKeys % kMergeKeys == 0, "a workgroup's outputs belong to one pair");
+    build_priority();
+    __shared__ unsigned long long sk[kMergeKeys];
+    __shared__ unsigned si[kMergeKeys];
+    __shared__ int split_sh[2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int o0 = blockIdx.x * kMergeKeys;
+    const int pair = o0 / (2 * run) * (2 * run);
+    const unsigned long long* A = keys_in + pair;
+    const int la = min(run, n - pair);
+    const unsigned long long* B = A + la;
+    const int lb = max(0, min(run, n - pair - run));
+    const int d0 = o0 - pair, d1 = min(d0 + kMergeKeys, la + lb);
+    if (wave < 2) {
+        const int a = merge_split(A, la, B, lb, wave == 0 ? d0 : d1, lane);
+        if (lane == 0) split_sh[wave] = a;
+    }
+    __syncthreads();
+    const int a0 = split_sh[0], a1 = split_sh[1], b0 = d0 - a0;
+    const int na = a1 - a0, count = d1 - d0;
+    // A's part, then B's
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+        const int i = k * THREADS + tid;
+        if (i < count) {
+            const int from = pair + (i < na ? a0 + i : la + b0 + (i - na));
+            sk[i] = keys_in[from];
+            si[i] = idx_in[from];
         }
     }
     __syncthreads();
-    const int count = min(kSortTile, n - base);
+    // thread t's outputs [t, t + 1) * ITEMS: its place by bisection, then one by one
+    const int nb = count - na, dt = min(tid * ITEMS, count);
+    int lo = max(0, dt - nb), hi = min(dt, na);
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (sk[mid] <= sk[na + dt - 1 - mid]) lo = mid + 1;
+        else hi = mid;
+    }
+    int a = lo, b = dt - lo;
+    unsigned long long ok[ITEMS];
+    unsigned oi[ITEMS];
 #pragma unroll
-    for (int r = 0; r < ITEMS; ++r) {
-        const int at = r * kSortThreads + tid;
-        if (at < count) {
-            const unsigned long long k = skeys[at];
-            const unsigned digit = static_cast<unsigned>((k >> shift) & kRadixMask);
-            const unsigned dst = dst_base[digit] + (static_cast<unsigned>(at) - run_start[digit]);
-            keys_out[dst] = k;
-            idx_out[dst] = sidx[at];
-            if constexpr (GATHER) pos_out[dst] = pos_in[sidx[at]];
+    for (int k = 0; k < ITEMS; ++k) {
+        if (dt + k >= count) break;
+        const bool from_a = a < na && (b >= nb || sk[a] <= sk[na + b]);
+        const int at = from_a ? a++ : na + b++;
+        ok[k] = sk[at];
+        oi[k] = si[at];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k)
+        if (dt + k < count) {
+            sk[dt + k] = ok[k];
+            si[dt + k] = oi[k];
+        }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+        const int i = k * THREADS + tid;
+        if (i < count) {
+            const unsigned from = si[i];
+            keys_out[o0 + i] = sk[i];
+            idx_out[o0 + i] = from;
+            if constexpr (GATHER) pos_out[o0 + i] = pos[from];
         }
     }
 }
@@ -1697,15 +1657,12 @@ struct BHState {
     float* bounds_partial = nullptr;
     unsigned long long* keys[2] = {nullptr, nullptr};
     unsigned* idx[2] = {nullptr, nullptr};
-    unsigned* hist = nullptr;
-    size_t hist_elems = 0;
     float4* pos_sorted = nullptr;
     int2* child = nullptr;  // radix-tree nodes: encoded (left, right) children
     int* first = nullptr;
     int* last = nullptr;
     int* info = nullptr;    // level | kKeptBit
     ChildBlock* blocks = nullptr;
-    unsigned* digit_totals = nullptr;  // sort: keys per digit of the current pass
     size_t chunk_elems = 0;
     DD* prefix = nullptr;            // [4][n + 1] double-double prefix sums
     DD* mass_chunk = nullptr;        // [4][nchunks]
@@ -1736,20 +1693,17 @@ void bh_release(BHState* b) {
     bh_free(b->keys[1]);
     bh_free(b->idx[0]);
     bh_free(b->idx[1]);
-    bh_free(b->hist);
     bh_free(b->pos_sorted);
     bh_free(b->child);
     bh_free(b->first);
     bh_free(b->last);
     bh_free(b->info);
     bh_free(b->blocks);
-    bh_free(b->digit_totals);
     bh_free(b->prefix);
     bh_free(b->mass_chunk);
     bh_free(b->com);
     bh_free(b->thr);
     b->cap = 0;
-    b->hist_elems = 0;
     b->built = false;
 }
 
@@ -1880,16 +1834,12 @@ nbody_status bh_resize(BHState* b, size_t n, nbody_sim* s) {
     NB_TRY(bh_alloc(b->keys[1], n));
     NB_TRY(bh_alloc(b->idx[0], n));
     NB_TRY(bh_alloc(b->idx[1], n));
-    const size_t nb = sort_max_tiles(n);
-    NB_TRY(bh_alloc(b->hist, kRadixBins * nb));
-    b->hist_elems = kRadixBins * nb;
     NB_TRY(bh_alloc(b->pos_sorted, n));
     NB_TRY(bh_alloc(b->child, m));
     NB_TRY(bh_alloc(b->first, m));
     NB_TRY(bh_alloc(b->last, m));
     NB_TRY(bh_alloc(b->info, m));
     NB_TRY(bh_alloc(b->blocks, m));
-    NB_TRY(bh_alloc(b->digit_totals, kRadixBins));
     NB_TRY(bh_alloc(b->prefix, 4 * (n + 1)));
     NB_TRY(bh_alloc(b->mass_chunk, 4 * static_cast<size_t>(std::max(kMassFusedChunks, blocks_for(n + 1, kMassChunk)))));
     NB_TRY(bh_alloc(b->com, m));
@@ -1915,29 +1865,33 @@ nbody_status bh_set_theta(nbody_sim* s) {
     return NBODY_OK;
 }
 
-// The kRadixPasses LSD passes over the keys in tiles of 256 x ITEMS (the last pass
-// also gathers the sorted positions); the sorted buffer is b->sorted_buf.
-template <int ITEMS>
-void radix_sort_passes(BHState* b, int n, const float4* pos, hipStream_t st) {
-    const int nb = blocks_for(n, kSortThreads * ITEMS);
+// Merges of at most this many keys in total take small workgroups (512 x 2
+// outputs: more of them, each done sooner), larger ones 1,024 x 4 (a quarter
+// of the searches, longer contiguous runs).  Tree build, us, 512 x 2 /
+// 1,024 x 2 / 512 x 4 / 1,024 x 4: 131 / 132 / 137 / 143 at 200,003, 295 / 289 /
+// 293 / 301 at 1,048,576, 1,127 / 1,062 / 1,049 / 1,019 at 4,194,304.
+constexpr int kSmallMerge = 1 << 20;
+
+template <int THREADS, int ITEMS>
+void merge_runs(BHState* b, int n, const float4* pos, hipStream_t st) {
     int cur = 0;
-    for (int pass = 0; pass < kRadixPasses; ++pass) {
-        const int shift = kRadixBits * pass;
-        // Above kFusedScanTiles tiles the tile offsets within each digit and
-        // the digits' totals come from a separate scan of the counts.
-        const bool fused = nb <= kFusedScanTiles;
-        hipLaunchKernelGGL(radix_hist_kernel<ITEMS>, dim3(nb), dim3(kSortThreads), 0, st, b->keys[cur], n, shift, b->hist, nb);
-        if (!fused)
-            hipLaunchKernelGGL(radix_rowscan_kernel, dim3(kRadixBins), dim3(kScanThreads2), 0, st, b->hist, nb,
-                               b->digit_totals);
-        // the last pass also writes the sorted positions
-        auto scatter = pass < kRadixPasses - 1 ? (fused ? radix_scatter_kernel<true, false, ITEMS> : radix_scatter_kernel<false, false, ITEMS>)
-                                : (fused ? radix_scatter_kernel<true, true, ITEMS> : radix_scatter_kernel<false, true, ITEMS>);
-        hipLaunchKernelGGL(scatter, dim3(nb), dim3(kSortThreads), 0, st, b->keys[cur], b->idx[cur], b->keys[cur ^ 1],
-                           b->idx[cur ^ 1], n, shift, b->hist, b->digit_totals, nb, pos, b->pos_sorted);
+    for (int run = kTileKeys; run < n; run *= 2) {
+        const auto merge =
+            2LL * run >= n ? merge_kernel<THREADS, ITEMS, true> : merge_kernel<THREADS, ITEMS, false>;
+        hipLaunchKernelGGL(merge, dim3(blocks_for(n, THREADS * ITEMS)), dim3(THREADS), 0, st, b->keys[cur],
+                           b->idx[cur], b->keys[cur ^ 1], b->idx[cur ^ 1], n, run, pos, b->pos_sorted);
         cur ^= 1;
     }
     b->sorted_buf = cur;
+}
+
+// Keys and order by sorted tiles and merges; the sorted buffer is b->sorted_buf.
+void merge_sort(BHState* b, int n, const float4* pos, hipStream_t st) {
+    const auto tiles = n <= kTileKeys ? tile_sort_kernel<true> : tile_sort_kernel<false>;
+    hipLaunchKernelGGL(tiles, dim3(blocks_for(n, kTileKeys)), dim3(kTileThreads), 0, st, pos, n, b->root, b->keys[0],
+                       b->idx[0], b->counters, b->pos_sorted);
+    if (n <= kSmallMerge) merge_runs<512, 2>(b, n, pos, st);
+    else merge_runs<1024, 4>(b, n, pos, st);
 }
 
 // Keys, sort, tree, masses: everything before the traversal.
@@ -1951,13 +1905,7 @@ static nbody_status bh_build(nbody_sim* s, BHState* b) {
         hipLaunchKernelGGL(dynamic_root_kernel, dim3(1), dim3(256), 0, st, b->bounds_partial, nbb, b->root,
                            theta_below(s->cfg.theta), b->thr);
     }
-    hipLaunchKernelGGL(keys_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, st, pos, n, b->root, b->keys[0],
-                       b->idx[0], b->counters);
-    switch (sort_items(static_cast<size_t>(n))) {
-    case 2: radix_sort_passes<2>(b, n, pos, st); break;
-    case 4: radix_sort_passes<4>(b, n, pos, st); break;
-    default: radix_sort_passes<8>(b, n, pos, st); break;
-    }
+    merge_sort(b, n, pos, st);
     const unsigned long long* keys = b->keys[b->sorted_buf];
     const unsigned* order = b->idx[b->sorted_buf];
     const int m = n - 1;

@@ -1,4 +1,4 @@
-// Barnes-Hut pipeline on the device: bounds, Morton keys, radix sort,
+// Barnes-Hut pipeline on the device: bounds, Morton keys, merge sort,
 // binary radix tree, octree cells, FP64 mass/centre-of-mass, traversal.
 #pragma once
 
