@@ -29,9 +29,10 @@
 //                    every cell writes one 192-byte record of its children
 //                    (at most eight, in key order): sources, opening
 //                    thresholds and codes, all the traversal reads of it;
-//  6. traversal      one lane per particle in Morton order; a wave walks the
-//                    octree with one stack in LDS of (cell, lanes) entries,
-//                    up to eight cells per step of the walk.
+//  6. traversal      groups of 16 to 64 particles in Morton order, one lane per
+//                    particle; one to eight wavefronts walk the octree for a
+//                    group with one stack in LDS of (cell, lanes) entries, each
+//                    taking up to eight cells per step of the walk.
 //                    Each lane makes the reference's own decision at each cell
 //                    (Octree::CalculateForce, Octree.cpp:107-145): approximate
 //                    with the cell's monopole iff side / |p - COM| < theta,
@@ -78,9 +79,7 @@ namespace {
 
 constexpr int kLevels = 21;
 constexpr int kBucketLevel = kLevels;
-constexpr int kTravThreads = 64;  // one wavefront per workgroup: the finest tail
-constexpr int kTravWaves = kTravThreads / 64;
-// Pending (cell, lanes) entries per wave.  Popping one cell at a time (a
+// Pending (cell, lanes) entries of a wavefront that walks alone.  Popping one cell at a time (a
 // depth-first walk) needs at most 7 * 21 + 1 entries above the cell it starts
 // from: seven pending siblings per level below it and the last cell's eight
 // children.  A batch of k cells replaces them by at most 8k children, so a
@@ -88,6 +87,10 @@ constexpr int kTravWaves = kTravThreads / 64;
 // cannot overflow (the checked push that reports overflow is a safeguard).
 constexpr int kStackCap = 288;
 constexpr int kDfsReserve = 7 * 22;
+// A stack that several wavefronts share replaces up to 8 x waves cells at once:
+// room for that while up to 134 are pending (as many as one wavefront's stack
+// holds below the reserve), the same reserve above.
+constexpr int stack_cap(int waves) { return waves == 1 ? kStackCap : 56 * waves + 134 + kDfsReserve; }
 constexpr int kEmpty = -1;
 
 // Child encoding: >= 0 internal node; <= -2 particle at sorted position (-c - 2).
@@ -1293,36 +1296,47 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
     return ((k / C) * kXcds + x) * C + k % C;
 }
 
-// 72 VGPRs (70 for law P): seven waves per SIMD by registers, while the
-// workgroup limit keeps 24 one-wave workgroups per CU (six per SIMD)
-// resident.  The box's six bounds stay in vector registers: held in scalar
-// registers they were spilled and reloaded every batch (2.3% slower).
-//
-// G particles per wavefront (64, 32, 16 or 8).  Below 64 the lanes hold the
+// G particles per group (64, 32 or 16).  Below 64 a wavefront's lanes hold the
 // particles 64 / G times over: every copy takes part in the walk alike (masks
 // have G bits), and in the list each copy, a slot, evaluates its share of the
-// entries; the slots' sums are added at the end.  A small system is then more
-// and shorter wavefronts.
-template <int LAW, int G>
-__global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __restrict__ pos_sorted,
-                                                                const ChildBlock* __restrict__ blocks,
-                                                                const int* __restrict__ node_first,
-                                                                const int* __restrict__ node_last, TravArgs A) {
+// entries; the slots' sums are added at the end.
+//
+// W wavefronts per group (a workgroup).  With W > 1 they share the walk: one
+// stack, of whose top 8 W cells wavefront w takes every W-th, then all of them
+// push their opened children, the first wavefront's on top.  Each keeps a list
+// and sums of its own; the sums are added in order at the end.  Two barriers a
+// step, and no cell is visited twice: N = 32,768 (theta 0.6) 138 us with 8
+// groups of particles and walks per 64, 81 us with 4 wavefronts to 32; dealing a
+// step's cells out in runs of eight instead of round robin left the later
+// wavefronts idle while the stack is short (90 us).
+//
+// At most 72 VGPRs for W > 1 (seven waves per SIMD): 83 are taken freely, five
+// waves, 3% to 7% slower with G = 16 and 32.  With W = 1 72 (70 for law P),
+// while the workgroup limit keeps 24 one-wave workgroups per CU (six per SIMD)
+// resident.  The box's six bounds stay in vector registers: held in scalar
+// registers they were spilled and reloaded every batch (2.3% slower).
+template <int LAW, int G, int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W > 1 ? 7 : 6))) void traverse_kernel(
+    const float4* __restrict__ pos_sorted, const ChildBlock* __restrict__ blocks, const int* __restrict__ node_first,
+    const int* __restrict__ node_last, TravArgs A) {
     // The walk runs at raised wave priority and drops it while the list is
     // evaluated: a SIMD then issues the walk's dependent loads and decisions
     // ahead of other wavefronts' list arithmetic, which fills the walk's
     // memory waits (traversal -1% at N = 4M, -3% at 1M; priority 3 gained
     // less, the opposite assignment nothing).
     __builtin_amdgcn_s_setprio(1);
-    __shared__ int stk_node[kTravWaves][kStackCap];
-    __shared__ uint2 stk_mask[kTravWaves][kStackCap];
-    __shared__ float4 lsrc[kTravWaves][kListCap];
-    __shared__ __align__(16) float lk[kTravWaves][kListCap];
-    __shared__ uint2 lmask[kTravWaves][kListCap];
-    __shared__ unsigned long long red[3][kTravWaves];
+    constexpr int kCap = stack_cap(W);
+    __shared__ int stk_node[kCap];
+    __shared__ uint2 stk_mask[kCap];
+    __shared__ float4 lsrc[W][kListCap];
+    __shared__ __align__(16) float lk[W][kListCap];
+    __shared__ uint2 lmask[W][kListCap];
+    __shared__ unsigned long long red[3][W];
+    __shared__ int wave_pushed[W];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: list and stack addresses in SGPRs
     constexpr int SLOTS = 64 / G;
+    constexpr bool kScalar = G == 64 && W == 1;  // the tested cells' blocks in scalar registers
     constexpr unsigned long long kGroup = G == 64 ? ~0ull : (1ull << (G & 63)) - 1ull;  // the particles' mask bits
     const int mine = lane & (G - 1), slot = lane / G;
     const int blk = xcd_block<G>(blockIdx.x, gridDim.x);
@@ -1386,6 +1400,18 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
         return (l >= 0 && l < G) ? (m & ~(1ULL << l)) : m;
     };
 
+    // A level-21 cell: identical keys, every particle of the range, pair by pair.
+    auto bucket = [&](int flagged, unsigned lo32, unsigned hi32) {
+        const int node = flagged & ~kBucketFlag;
+        const unsigned long long mask = (static_cast<unsigned long long>(hi32) << 32) | lo32;
+        const int f = node_first[node], l = node_last[node];
+        for (int q = f; q <= l; ++q) {
+            if (cnt > kListCap - 4) flush();
+            const unsigned long long m = without_self(mask, q);
+            if (m) append(pos_sorted[q], m);
+        }
+    };
+
     // The wave's bounding box (lanes past n hold the last particle, inside it).
     // A child cell whose nearest point of the box is beyond its threshold is
     // approximated by every lane, one whose farthest point is within it is
@@ -1418,12 +1444,12 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
         const float dx = me.x - c.x, dy = me.y - c.y, dz = me.z - c.z;
         const float r2 = (dx * dx + dy * dy) + dz * dz;
         const unsigned long long am = __builtin_amdgcn_ballot_w64(!(r2 < A.thr[root_level])) & all;
-        if (am) append(c, am);
+        if (am && wave == 0) append(c, am);
         const unsigned long long om = all & ~am;
         if (om) {
-            if (lane == 0) {
-                stk_node[wave][0] = root_level >= kBucketLevel ? kBucketFlag : 0;
-                stk_mask[wave][0] = make_uint2(static_cast<unsigned>(om), static_cast<unsigned>(om >> 32));
+            if (tid == 0) {
+                stk_node[0] = root_level >= kBucketLevel ? kBucketFlag : 0;
+                stk_mask[0] = make_uint2(static_cast<unsigned>(om), static_cast<unsigned>(om >> 32));
             }
             sp = 1;
         }
@@ -1431,48 +1457,68 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
     // Lane 8j + s holds child s of the batch's j-th cell (j = 0 the top of
     // the stack) in the write phase.
     const int grp = lane >> 3;
+    if constexpr (W > 1) __syncthreads();
     while (sp > 0) {
-        __builtin_amdgcn_wave_barrier();
-        // The batch: up to eight cells from the top of the stack, as many as
-        // the stack has room to replace by their children (each cell nets at
-        // most seven more entries) while keeping the depth-first reserve, at
-        // least one, and no bucket among them.  Group j reads entry sp-1-j
-        // (groups beyond the batch repeat its last entry).
-        const int kmax = min(min(8, sp), max((kStackCap - kDfsReserve - sp) / 7, 1));
-        const int e = sp - 1 - min(grp, kmax - 1);
-        const int vcell = stk_node[wave][e];
-        const uint2 vm = stk_mask[wave][e];
-        const unsigned long long bk = __builtin_amdgcn_ballot_w64((vcell & kBucketFlag) != 0);
-        int k = bk ? min(kmax, static_cast<int>(__builtin_ctzll(bk)) >> 3) : kmax;
-        if (k == 0) {
-            // identical keys: every particle of the range, pair by pair
-            --sp;
-            ++opened;
-            const int node = __builtin_amdgcn_readfirstlane(vcell) & ~kBucketFlag;
-            const unsigned lo32 = __builtin_amdgcn_readfirstlane(vm.x);
-            const unsigned hi32 = __builtin_amdgcn_readfirstlane(vm.y);
-            const unsigned long long mask = (static_cast<unsigned long long>(hi32) << 32) | lo32;
-            const int f = node_first[node], l = node_last[node];
-            for (int q = f; q <= l; ++q) {
-                if (cnt > kListCap - 4) flush();
-                const unsigned long long m = without_self(mask, q);
-                if (m) append(pos_sorted[q], m);
+        int vcell, k, all_k = 0;
+        uint2 vm;
+        bool in_batch;
+        if constexpr (W == 1) {
+            __builtin_amdgcn_wave_barrier();
+            // The batch: up to eight cells from the top of the stack, as many as
+            // the stack has room to replace by their children (each cell nets at
+            // most seven more entries) while keeping the depth-first reserve, at
+            // least one, and no bucket among them.  Group j reads entry sp-1-j
+            // (groups beyond the batch repeat its last entry).
+            const int kmax = min(min(8, sp), max((kStackCap - kDfsReserve - sp) / 7, 1));
+            const int e = sp - 1 - min(grp, kmax - 1);
+            vcell = stk_node[e];
+            vm = stk_mask[e];
+            const unsigned long long bk = __builtin_amdgcn_ballot_w64((vcell & kBucketFlag) != 0);
+            k = bk ? min(kmax, static_cast<int>(__builtin_ctzll(bk)) >> 3) : kmax;
+            if (k == 0) {
+                // identical keys: every particle of the range, pair by pair
+                --sp;
+                ++opened;
+                bucket(__builtin_amdgcn_readfirstlane(vcell), __builtin_amdgcn_readfirstlane(vm.x),
+                       __builtin_amdgcn_readfirstlane(vm.y));
+                continue;
             }
-            continue;
+            // Up to eight list entries per cell: a smaller batch when at least
+            // four cells fit, else evaluate the list first.
+            if (cnt > kListCap - 8 * k) {
+                const int fit = (kListCap - cnt) >> 3;
+                if (fit >= 4) k = fit;
+                else flush();
+            }
+            opened += static_cast<unsigned long long>(k);
+            in_batch = grp < k;
+        } else {
+            // The same rule for the workgroup's batch, of which every W-th cell
+            // is this wavefront's; a bucket is expanded by the wavefront that
+            // holds it.  The list takes the share's children whole.
+            all_k = min(min(8 * W, sp), max((kCap - kDfsReserve - sp) / 7, 1));
+            const int share = W * grp + wave;
+            in_batch = share < all_k;
+            const int e = sp - 1 - min(share, all_k - 1);
+            vcell = stk_node[e];
+            vm = stk_mask[e];
+            k = (all_k - wave + W - 1) / W;
+            opened += static_cast<unsigned long long>(k);
+            unsigned long long bk = __builtin_amdgcn_ballot_w64(in_batch && (vcell & kBucketFlag) != 0);
+            while (bk) {
+                const int l = static_cast<int>(__builtin_ctzll(bk)) & ~7;
+                bk &= ~(0xffull << l);
+                bucket(__builtin_amdgcn_readlane(vcell, l), __builtin_amdgcn_readlane(static_cast<int>(vm.x), l),
+                       __builtin_amdgcn_readlane(static_cast<int>(vm.y), l));
+            }
+            in_batch = in_batch && (vcell & kBucketFlag) == 0;
+            if (cnt > kListCap - 8 * k) flush();
         }
-        // Up to eight list entries per cell: a smaller batch when at least
-        // four cells fit, else evaluate the list first.
-        if (cnt > kListCap - 8 * k) {
-            const int fit = (kListCap - cnt) >> 3;
-            if (fit >= 4) k = fit;
-            else flush();
-        }
-        opened += static_cast<unsigned long long>(k);
-        const int base = sp - k;
+        const int base = sp - (W == 1 ? k : all_k);
+        const unsigned long long batch = __builtin_amdgcn_ballot_w64(in_batch);
         // Lane 8j + s reads child s of cell j (lanes beyond the batch read the
         // top cell's block and take no part), issued before the decisions.
-        const int top = __builtin_amdgcn_readfirstlane(vcell);  // all lanes active: group 0
-        const bool in_batch = grp < k;
+        const int top = W == 1 ? __builtin_amdgcn_readfirstlane(vcell) : 0;  // all lanes active: group 0
         const ChildBlock* VB = blocks + (in_batch ? vcell : top);
         const float4 vsrc = VB->src[lane & 7];
         const float vthr = VB->thr[lane & 7];
@@ -1493,8 +1539,7 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
         }
         // child cells of the batch that need the lane-by-lane test
         const unsigned long long tested =
-            __builtin_amdgcn_ballot_w64(vcode >= 0 && !open_all && !accept_all) &
-            (k == 8 ? ~0ull : ((1ull << (8 * k)) - 1ull));
+            __builtin_amdgcn_ballot_w64(vcode >= 0 && !open_all && !accept_all) & batch;
         // Decisions, cell by cell, for the tested children only (a cell none
         // of whose children is tested is skipped).  The block's centres of
         // mass and thresholds in scalar registers at once (the empty asm
@@ -1507,10 +1552,10 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
         // every lane (the lanes' masks start as all lanes).
         ge_lo = open_all ? 0u : ~0u;
         ge_hi = open_all ? 0u : ~0u;
-        if constexpr (G < 64) {
-            // From the registers of the lane that holds the child: with few
-            // wavefronts per SIMD a scalar load of each block would be waited
-            // for in full, cell after cell.
+        if constexpr (!kScalar) {
+            // From the registers of the lane that holds the child: where the
+            // walk's length is what counts, a scalar load of each block would
+            // be waited for in full, cell after cell.
             for (unsigned long long todo = tested; todo != 0ull; todo &= todo - 1ull) {
                 const int l = static_cast<int>(__builtin_ctzll(todo));
                 const float dx = me.x - read_lane(vsrc.x, l), dy = me.y - read_lane(vsrc.y, l),
@@ -1520,7 +1565,7 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
                 if (ge != ~0ull) write_lane64(ge_lo, ge_hi, ge, l);
             }
         }
-        for (int j = 0; G == 64 && j < k; ++j) {
+        for (int j = 0; kScalar && j < k; ++j) {
             const unsigned tj = static_cast<unsigned>(tested >> (8 * j)) & 0xffu;
             if (tj == 0u) continue;  // every child cell of cell j has its box verdict
             const int code = __builtin_amdgcn_readlane(vcell, j * 8);
@@ -1551,7 +1596,6 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
         // particle every lane of the mask but the particle's own) and opening
         // lanes om (none for a particle).
         const unsigned long long mask = (static_cast<unsigned long long>(vm.y) << 32) | vm.x;
-        const unsigned long long batch = k == 8 ? ~0ull : ((1ull << (8 * k)) - 1ull);
         const bool child = in_batch && vcode != kEmpty;
         const unsigned long long children = __builtin_amdgcn_ballot_w64(vcode != kEmpty) & batch;
         const bool leaf = vcode < 0;
@@ -1575,16 +1619,31 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
         const bool ws = child && om != 0ull;  // a cell: a particle's ge is all lanes
         const unsigned long long has_s = __builtin_amdgcn_ballot_w64(om != 0ull) & children;
         const int pushed = __popcll(has_s);
-        const int last = base + pushed - 1;
-        if (last < kStackCap) {
+        int last = base + pushed - 1;
+        int next = base + pushed;
+        if constexpr (W > 1) {
+            // the first wavefront's children on top, as its cells were
+            if (lane == 0) wave_pushed[wave] = pushed;
+            __syncthreads();  // and every share has been read
+            next = base;
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const int c = wave_pushed[w];
+                next += c;
+                if (w > wave) last += c;
+            }
+            next = __builtin_amdgcn_readfirstlane(next);
+            last = __builtin_amdgcn_readfirstlane(last);
+        }
+        if (next <= kCap) {
             if (ws) {
                 const int at = last - static_cast<int>(__builtin_amdgcn_mbcnt_hi(
                                           static_cast<unsigned>(has_s >> 32),
                                           __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(has_s), 0u)));
-                stk_node[wave][at] = vcode;
-                stk_mask[wave][at] = make_uint2(static_cast<unsigned>(om), static_cast<unsigned>(om >> 32));
+                stk_node[at] = vcode;
+                stk_mask[at] = make_uint2(static_cast<unsigned>(om), static_cast<unsigned>(om >> 32));
             }
-            sp = base + pushed;
+            sp = next;
         } else {
             // not reached (the depth-first reserve): the entries beyond the
             // capacity would be lost and reported
@@ -1592,14 +1651,15 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
                 const int at = last - static_cast<int>(__builtin_amdgcn_mbcnt_hi(
                                           static_cast<unsigned>(has_s >> 32),
                                           __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(has_s), 0u)));
-                if (at < kStackCap) {
-                    stk_node[wave][at] = vcode;
-                    stk_mask[wave][at] = make_uint2(static_cast<unsigned>(om), static_cast<unsigned>(om >> 32));
+                if (at < kCap) {
+                    stk_node[at] = vcode;
+                    stk_mask[at] = make_uint2(static_cast<unsigned>(om), static_cast<unsigned>(om >> 32));
                 }
             }
-            sp = kStackCap;
+            sp = kCap;
             overflowed = true;
         }
+        if constexpr (W > 1) __syncthreads();
     }
     if (overflowed && lane == 0) atomicOr(A.overflow, 1u);
     if (cnt) flush();
@@ -1616,7 +1676,26 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
             kahan_add(sx, cx, -qx), kahan_add(sy, cy, -qy), kahan_add(sz, cz, -qz);
         }
     }
-    if (valid && slot == 0) {
+    if constexpr (W > 1) {
+        // the wavefronts' sums likewise, through the first's list
+        float* out = reinterpret_cast<float*>(lsrc[wave]);
+        static_assert(sizeof(lsrc[0]) >= 6 * G * sizeof(float), "a wavefront's sums fit its list");
+        __builtin_amdgcn_wave_barrier();
+        if (lane < G) {
+            out[lane] = sx, out[G + lane] = sy, out[2 * G + lane] = sz;
+            out[3 * G + lane] = cx, out[4 * G + lane] = cy, out[5 * G + lane] = cz;
+        }
+        __syncthreads();
+        if (wave == 0 && lane < G) {
+            for (int w = 1; w < W; ++w) {
+                const float* in = reinterpret_cast<const float*>(lsrc[w]);
+                kahan_add(sx, cx, in[lane]), kahan_add(sy, cy, in[G + lane]), kahan_add(sz, cz, in[2 * G + lane]);
+                kahan_add(sx, cx, -in[3 * G + lane]), kahan_add(sy, cy, -in[4 * G + lane]);
+                kahan_add(sz, cz, -in[5 * G + lane]);
+            }
+        }
+    }
+    if (wave == 0 && valid && slot == 0) {
         const unsigned p = A.order[t];
         // back from scaled units (a power of two: exact)
         const float ax = sx * A.sc.out, ay = sy * A.sc.out, az = sz * A.sc.out;
@@ -1642,7 +1721,7 @@ __global__ __launch_bounds__(kTravThreads) void traverse_kernel(const float4* __
     __syncthreads();
     if (tid < 3) {
         unsigned long long tot = 0;
-        for (int w = 0; w < kTravWaves; ++w) tot += red[tid][w];
+        for (int w = 0; w < W; ++w) tot += red[tid][w];
         atomicAdd(A.walk + tid, tot);
     }
 }
@@ -1725,19 +1804,47 @@ inline int mass_rows(int n) {
     return kMassPer;
 }
 
-// Particles per wavefront of the traversal.  Few particles make short
-// wavefronts and many of them (a walk over few cells, the list shared by the
-// slots) but more walks in all, so the smallest systems take eight, and 64 pay
-// off from about a million on.  Force pass, ms, with 64 / 32 / 16 / 8:
-//   Plummer sphere, theta 0.6:    16,384  0.256 / 0.168 / 0.123 / 0.099
-//                                 32,768  0.293 / 0.187 / 0.144 / 0.138
-//                                 65,536  0.331 / 0.209 / 0.169 / 0.203
-//                                131,072  0.326 / 0.234 / 0.269 / 0.316
-//   two-disc encounter, 0.5:     524,288  0.858 / 0.708 / 0.853 / 1.120
-//                              1,048,576  1.353 / 1.434 / 1.719 / 2.354
-// Where systems share the device the total work counts, so the next larger
-// count is taken where it costs one alone little (32,768).
-inline int trav_group(int n) { return n <= 24576 ? 8 : n <= 98304 ? 16 : n <= 786432 ? 32 : 64; }
+// Particles per group of the traversal and wavefronts that share a group's walk.
+// One wavefront after another waits for its cells, decides, and waits again, so
+// a system with few groups is bound by the longest walk: several wavefronts to a
+// group shorten it, and more of them the fewer groups there are.  Small groups
+// make more and shorter walks, but more in all.  Force pass, us:
+//                                 16x8   32x8   32x4   64x8   64x4   64x2   64x1
+//   Plummer, theta 0.6:   4,000     30     36     47     47     74    115
+//                         8,192     38     39     52     53     80
+//                        16,384     63     50     63     60     94
+//                        32,768    106     83     81     83    104    162    293
+//                        65,536           142    125    134    131           331
+//                       131,072                  192    226    210    222    333
+//   encounter, 0.5:     262,144                  354    379    339    425    556
+//                       524,288                  700    715    620    676    862
+//              0.6:   1,048,576                               988    933    979
+//              0.5:   2,097,152                 2954   3133   2557   2465   2573
+//              0.8:   4,194,304                 3324   3896   2743   2439   2291
+// (One wavefront to a group of 8, 16 or 32: 53 at 4,000, 138 at 32,768, 234 at
+// 131,072, 309 at 200,003, where 64x4 takes 264.)
+struct TravShape {
+    int group, waves;
+};
+
+inline TravShape trav_shape(int n) {
+    if (n <= 12288) return {16, 8};
+    if (n <= 24576) return {32, 8};
+    if (n <= 163840) return {32, 4};
+    if (n <= 786432) return {64, 4};
+    if (n <= 2621440) return {64, 2};
+    return {64, 1};
+}
+
+using TraverseFn = void (*)(const float4*, const ChildBlock*, const int*, const int*, TravArgs);
+
+template <int LAW>
+TraverseFn traverse_fn(TravShape s) {
+    if (s.group == 16) return traverse_kernel<LAW, 16, 8>;
+    if (s.group == 32) return s.waves == 8 ? traverse_kernel<LAW, 32, 8> : traverse_kernel<LAW, 32, 4>;
+    return s.waves == 4 ? traverse_kernel<LAW, 64, 4> : s.waves == 2 ? traverse_kernel<LAW, 64, 2>
+                                                                     : traverse_kernel<LAW, 64, 1>;
+}
 
 float theta_below(double theta) {
     float t = static_cast<float>(theta);
@@ -1987,14 +2094,10 @@ nbody_status bh_step(nbody_sim* s, float dt, bool kick, hipEvent_t ev_b, hipEven
     A.dt = dt;
     A.dts = static_cast<float>(static_cast<double>(dt) / s->cfg.scale);
     if (ev_b) NB_HIP(hipEventRecord(ev_b, st));
-    const int group = trav_group(n);
-    const bool r = s->cfg.law == NBODY_LAW_R;
-    const auto fn = group == 8    ? (r ? traverse_kernel<NBODY_LAW_R, 8> : traverse_kernel<NBODY_LAW_P, 8>)
-                    : group == 16 ? (r ? traverse_kernel<NBODY_LAW_R, 16> : traverse_kernel<NBODY_LAW_P, 16>)
-                    : group == 32 ? (r ? traverse_kernel<NBODY_LAW_R, 32> : traverse_kernel<NBODY_LAW_P, 32>)
-                                  : (r ? traverse_kernel<NBODY_LAW_R, 64> : traverse_kernel<NBODY_LAW_P, 64>);
-    hipLaunchKernelGGL(fn, dim3(blocks_for(n, group)), dim3(kTravThreads), 0, st, b->pos_sorted, b->blocks, b->first,
-                       b->last, A);
+    const TravShape shape = trav_shape(n);
+    const auto fn = s->cfg.law == NBODY_LAW_R ? traverse_fn<NBODY_LAW_R>(shape) : traverse_fn<NBODY_LAW_P>(shape);
+    hipLaunchKernelGGL(fn, dim3(blocks_for(n, shape.group)), dim3(64 * shape.waves), 0, st, b->pos_sorted, b->blocks,
+                       b->first, b->last, A);
     NB_HIP(hipGetLastError());
     if (ev_e) NB_HIP(hipEventRecord(ev_e, st));
     hipLaunchKernelGGL(publish_counters_kernel, dim3(1), dim3(64), 0, st, b->counters, b->walk, b->host_ctr);
