@@ -354,8 +354,8 @@ typedef struct nbody_batch_info {
 } nbody_batch_info;
 
 /* cfg->method must be NBODY_METHOD_DIRECT; capacity = arena size in particles
- * (each system takes its size rounded up to 256).  Steps of systems of 8,192
- * particles or more also use up to 1 GiB of device memory for partial sums,
+ * (each system takes its size rounded up to 256).  Steps of systems of more than
+ * 1,024 particles also use up to 1 GiB of device memory for partial sums,
  * allocated as they need it (without it, slower and rounded differently). */
 nbody_status nbody_batch_create(const nbody_config* cfg, size_t capacity, nbody_batch** out);
 nbody_status nbody_batch_destroy(nbody_batch* batch);
@@ -374,10 +374,10 @@ nbody_status nbody_batch_add_plummer(nbody_batch* batch, uint64_t seed, size_t n
 /* Advance every system nsteps kick-drift steps (asynchronous, one graph launch). */
 nbody_status nbody_batch_step(nbody_batch* batch, float dt, int32_t nsteps);
 
-/* The baseline: each system alone, one-sided single-system launches, waiting
- * for each system before the next.  split_small = 0: the plain launch (one
- * workgroup per 256 targets, all sources); 1: the single-system default,
- * which splits a small system's sources over more workgroups. */
+/* The baseline: each system alone, single-system launches, waiting for each
+ * system before the next.  split_small = 0: the sum that a batch step takes for
+ * the system's size (the same bits); 1: the one-sided launch that splits a small
+ * system's sources over more workgroups. */
 nbody_status nbody_batch_step_sequential(nbody_batch* batch, float dt, int32_t nsteps, int32_t split_small);
 
 nbody_status nbody_batch_synchronize(nbody_batch* batch);

@@ -9,12 +9,14 @@
 // core (direct_core.hpp) over its own system's sources, so a system's forces are
 // the same bits whether it runs alone or in any mix.
 //
-// Systems from 8,192 particles on take the sum over unordered pairs
+// Systems of more than 1,024 particles take the sum over unordered pairs
 // (direct_sym.hip) instead: a persistent kernel drains their tasks, then one adds
 // their rows of partial sums and kicks.  The rows lie in a buffer of at most
 // kRowsBytes; where a batch's systems need more, they are taken in groups, one
-// group's two kernels after the other's.  Which way a system takes, and its
-// tasks, depend on its size alone.
+// group's two kernels after the other's.  The smaller systems' items are drained
+// behind the last group's tasks; only a batch without any pairs has a kernel of
+// its own for them.  Which way a system takes, and its tasks, depend on its size
+// alone.
 //
 // The queue lives in device memory (items, their count, per-step counters), so
 // a captured hipGraph of k steps stays valid while systems join and leave: only
@@ -54,7 +56,7 @@ struct SysDesc {
 };
 
 // A task of the sum over unordered pairs: blocks a and a + d, run h of the
-// streamed one.
+// streamed one; with d < 0 the kTile targets of a one-sided system from a kTile on.
 struct SymTask {
     int sys, a, d, h;
 };
@@ -75,8 +77,13 @@ struct SymGroup {
 // stays with the one-sided sum.
 constexpr size_t kRowsBytes = size_t(1) << 30;
 
-// Below this the blocks with themselves, one-sided, are too large a part.
-constexpr size_t kSymMin = 8192;
+// A one-sided item is n pairs per lane, one after another: the batch waits for
+// its largest item.  A pair task is at most 1,024, so every padded size above
+// that takes them.  A step, us, with pairs from 1,280 / 2,049 / 8,192 on: 96
+// systems of 1,024 to 32,768 particles 2,669 / 2,677 / 2,807, 8 of 1,024 to 4,096
+// 83 / 102 / 180, 128 of 1,024 to 8,192 474 / 506 / 713, 256 of 1,500 to 1,600
+// 250 / 256 / 261; from 512 on 512 systems of 500 to 1,024 take 175 against 155.
+constexpr size_t kSymMin = 1280;
 
 SymPlan batch_sym_plan(size_t n_pad) {
     SymPlan p{};
@@ -128,6 +135,30 @@ __device__ __forceinline__ void batch_kick(const BatchLaunch& B, int r, float4 x
     B.acc[r] = make_float4(ax, ay, az, 0.f);
 }
 
+// One item of a one-sided system: K x BLOCK targets from `ibase` on over all of
+// its sources.
+template <int LAW, int K, int BLOCK>
+__device__ __forceinline__ void one_sided_item(const BatchLaunch& B, const SysDesc& d, int ibase,
+                                               core::SrcTile* tiles) {
+    const int tid = threadIdx.x;
+    const float4* src = B.pos_in + d.off;
+    float xi[K], yi[K], zi[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int i = min(ibase + tid + k * BLOCK, d.n_pad - 1);
+        const float4 q = src[i];
+        xi[k] = q.x * d.sc.inv_len;
+        yi[k] = q.y * d.sc.inv_len;
+        zi[k] = q.z * d.sc.inv_len;
+    }
+    float sx[K], sy[K], sz[K];
+    core::block_forces<LAW, K, BLOCK>(tiles, src, 0, d.n_pad, d.sc, xi, yi, zi, sx, sy, sz);
+    for (int k = 0; k < K; ++k) {  // K is 1 or 2: fully unrolled without a pragma
+        const int i = ibase + tid + k * BLOCK;
+        if (i < d.n) batch_kick(B, d.off + i, src[i], sx[k] * d.sc.out, sy[k] * d.sc.out, sz[k] * d.sc.out);
+    }
+}
+
 // The barriers around the item fetch also separate one item's last reads of
 // the LDS tiles from the next item's first writes.
 template <int LAW, int K, int BLOCK>
@@ -143,37 +174,23 @@ __global__ __launch_bounds__(BLOCK) void batch_step_kernel(BatchLaunch B, unsign
         __syncthreads();
         if (it >= n_items) break;
         const WorkItem w = B.items[it];
-        const SysDesc d = B.sys[w.sys];
-        const float4* src = B.pos_in + d.off;
-        float xi[K], yi[K], zi[K];
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            const int i = min(w.ibase + tid + k * BLOCK, d.n_pad - 1);
-            const float4 q = src[i];
-            xi[k] = q.x * d.sc.inv_len;
-            yi[k] = q.y * d.sc.inv_len;
-            zi[k] = q.z * d.sc.inv_len;
-        }
-        float sx[K], sy[K], sz[K];
-        core::block_forces<LAW, K, BLOCK>(tiles, src, 0, d.n_pad, d.sc, xi, yi, zi, sx, sy, sz);
-        for (int k = 0; k < K; ++k) {  // K is 1 or 2: fully unrolled without a pragma
-            const int i = w.ibase + tid + k * BLOCK;
-            if (i < d.n) {
-                batch_kick(B, d.off + i, src[i], sx[k] * d.sc.out, sy[k] * d.sc.out, sz[k] * d.sc.out);
-            }
-        }
+        one_sided_item<LAW, K, BLOCK>(B, B.sys[w.sys], w.ibase, tiles);
     }
 }
 
 // The tasks of one group, largest systems first, from a counter.  Every branch is
-// uniform over the workgroup.  Bound by the pair arithmetic's issue: 96 systems
-// of 1,024 to 32,768 particles, five steps and their reads, 21.9 ms, 29.0 ms with
-// every system one-sided; a burst of 16 served requests 66.6 -> 50.8 ms.
+// uniform over the workgroup.  Bound by the pair arithmetic's issue: a step of 96
+// systems of 1,024 to 32,768 particles 2.67 ms (5.6e12 interactions/s), 3.24 ms
+// with the systems below 8,192 one-sided in a kernel of their own, 4.9 ms with
+// every system one-sided.
 template <int LAW>
 __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(6))) void batch_sym_kernel(BatchLaunch B,
                                                                                                  int group,
                                                                                                  unsigned* counter) {
-    __shared__ core::SymShared S;
+    __shared__ union {
+        core::SymShared pairs;
+        core::SrcTile tiles[2];
+    } S;
     __shared__ int item_sh;
     const SymGroup G = B.groups[group];
     for (;;) {
@@ -184,17 +201,21 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(6))) void
         if (it >= G.task1) break;
         const SymTask w = B.tasks[it];
         const SysDesc D = B.sys[w.sys];
+        if (w.d < 0) {
+            one_sided_item<LAW, 1, kTile>(B, D, w.a * kTile, S.tiles);
+            continue;
+        }
         const core::SymArgs A{B.pos_in + D.off, B.rows + D.rows, D.n_pad, D.sym, D.sc};
         const int H = D.sym.nsb / 2;
         if (w.d == 0) {
-            if (D.gm_equal > 0.f) core::sym_task<LAW, false, true>(A, S, w.a, w.a, w.h, w.h, 0);
-            else core::sym_task<LAW, false, false>(A, S, w.a, w.a, w.h, w.h, 0);
+            if (D.gm_equal > 0.f) core::sym_task<LAW, false, true>(A, S.pairs, w.a, w.a, w.h, w.h, 0);
+            else core::sym_task<LAW, false, false>(A, S.pairs, w.a, w.a, w.h, w.h, 0);
         } else {
             int b = w.a + w.d;
             if (b >= D.sym.nsb) b -= D.sym.nsb;
             const int rowi = w.d * D.sym.split + w.h, rowj = (H + 1) * D.sym.split + w.d - 1;
-            if (D.gm_equal > 0.f) core::sym_task<LAW, true, true>(A, S, w.a, b, w.h, rowi, rowj);
-            else core::sym_task<LAW, true, false>(A, S, w.a, b, w.h, rowi, rowj);
+            if (D.gm_equal > 0.f) core::sym_task<LAW, true, true>(A, S.pairs, w.a, b, w.h, rowi, rowj);
+            else core::sym_task<LAW, true, false>(A, S.pairs, w.a, b, w.h, rowi, rowj);
         }
     }
 }
@@ -381,6 +402,11 @@ void arena_free(nbody_batch* b, size_t off, size_t len) {
     }
 }
 
+// Every particle's G m in the pair arithmetic's scaled units if all are equal, else 0.
+float scaled_gm(const nbody_batch* b, const nbody_batch::Sys& y) {
+    return y.gm_equal * (b->cfg.law == NBODY_LAW_R ? 1.0f / y.sc.mass_k : y.sc.mass_k);
+}
+
 // Rebuild the work-item list (largest systems first) and upload it.
 nbody_status rebuild_items(nbody_batch* b) {
     if (!b->items_dirty) return NBODY_OK;
@@ -398,12 +424,12 @@ nbody_status rebuild_items(nbody_batch* b) {
     uint64_t inter = 0;
     for (size_t s = 0; s < b->systems.size(); ++s) {
         const auto& y = b->systems[s];
-        const float gm = y.gm_equal * (b->cfg.law == NBODY_LAW_R ? 1.0f / y.sc.mass_k : y.sc.mass_k);
-        descs[s] = SysDesc{static_cast<int>(y.off), static_cast<int>(y.n), static_cast<int>(y.n_pad), gm, y.sc, {}, 0};
+        descs[s] = SysDesc{static_cast<int>(y.off), static_cast<int>(y.n), static_cast<int>(y.n_pad), scaled_gm(b, y),
+                           y.sc, {}, 0};
     }
     // Groups of systems, largest first, whose rows fit the buffer together.
     size_t rows = 0, rows_max = 0;
-    std::vector<int> in_group;
+    std::vector<int> in_group, one_sided;
     auto close_group = [&] {
         if (in_group.empty()) return;
         SymGroup g{static_cast<int>(tasks.size()), 0, static_cast<int>(sums.size()), 0};
@@ -435,10 +461,19 @@ nbody_status rebuild_items(nbody_batch* b) {
             rows += need;
             in_group.push_back(s);
         } else {
-            for (size_t i = 0; i < y.n_pad; i += per) items.push_back(WorkItem{s, static_cast<int>(i)});
+            one_sided.push_back(s);
         }
     }
     close_group();
+    // With the last group's tasks, behind them; without any, a kernel of their own.
+    for (int s : one_sided) {
+        const int n_pad = static_cast<int>(b->systems[s].n_pad);
+        if (groups.empty())
+            for (int i = 0; i < n_pad; i += per) items.push_back(WorkItem{s, i});
+        else
+            for (int i = 0; i < n_pad; i += kTile) tasks.push_back(SymTask{s, i / kTile, -1, 0});
+    }
+    if (!groups.empty()) groups.back().task1 = static_cast<int>(tasks.size());
     if (rows_max > b->rows_cap) {
         const nbody_status st = ensure_dev(reinterpret_cast<void**>(&b->d_rows), b->rows_cap, rows_max, sizeof(float),
                                            b->stream, kRowsBytes / sizeof(float));
@@ -803,14 +838,18 @@ nbody_status nbody_batch_step_sequential(nbody_batch* b, float dt, int32_t nstep
     if (nsteps == 0) return NBODY_OK;
     NB_HIP(hipEventRecord(b->ev[0], b->stream));
     // Each galaxy alone, one launch per step of the single-system kernel,
-    // waiting for each galaxy before the next: either the plain launch (one
-    // workgroup per 256 targets over all sources) or, with split_small, the
-    // single-system default that splits the sources of a small system over
-    // more workgroups and adds a reduction launch.
+    // waiting for each galaxy before the next: either the sum that the batch
+    // takes for its size (one workgroup per 256 targets over all sources, or its
+    // pairs and their rows) or, with split_small, the one-sided launch that
+    // splits the sources of a small system over more workgroups and adds a
+    // reduction launch.
     for (const auto& y : b->systems) {
         if (!y.live) continue;
         DirectShape shape = split_small ? direct_default_shape(static_cast<int>(y.n_pad)) : DirectShape{1, 256, 1};
-        const size_t split = static_cast<size_t>(direct_effective_split(shape, static_cast<int>(y.n_pad)));
+        // the rows' buffer holds any one system's (rebuild_items)
+        const SymPlan P = split_small || b->no_rows ? SymPlan{} : batch_sym_plan(y.n_pad);
+        const size_t split =
+            P.nsb > 0 ? 0 : static_cast<size_t>(direct_effective_split(shape, static_cast<int>(y.n_pad)));
         if (split * y.n_pad > b->part_elems) {
             NB_HIP(hipStreamSynchronize(b->stream));
             if (b->part) (void)hipFree(b->part);
@@ -825,14 +864,16 @@ nbody_status nbody_batch_step_sequential(nbody_batch* b, float dt, int32_t nstep
             L.pos_out = b->pos[parity ^ 1] + y.off;
             L.vel = b->vel + y.off;
             L.acc = b->acc + y.off;
-            L.part = b->part;
+            L.part = P.nsb > 0 ? reinterpret_cast<float4*>(b->d_rows) : b->part;
+            L.gm_equal = scaled_gm(b, y);
             L.n = static_cast<int>(y.n);
             L.n_pad = static_cast<int>(y.n_pad);
             L.law = b->cfg.law;
             L.sc = y.sc;
             L.dt = dt;
             L.dts = static_cast<float>(static_cast<double>(dt) / b->cfg.scale);
-            NB_HIP(direct_step(L, shape, true, b->stream, nullptr, nullptr));
+            NB_HIP(P.nsb > 0 ? sym_step(L, P, true, b->stream, nullptr, nullptr)
+                             : direct_step(L, shape, true, b->stream, nullptr, nullptr));
             parity ^= 1;
         }
         // Steps of one galaxy leave its positions in buffer cur ^ (nsteps & 1);
