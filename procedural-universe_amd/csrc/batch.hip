@@ -181,8 +181,7 @@ __global__ __launch_bounds__(BLOCK) void batch_step_kernel(BatchLaunch B, unsign
 // The tasks of one group, largest systems first, from a counter.  Every branch is
 // uniform over the workgroup.  Bound by the pair arithmetic's issue: a step of 96
 // systems of 1,024 to 32,768 particles 2.67 ms (5.6e12 interactions/s), 3.24 ms
-// with the systems below 8,192 one-sided in a kernel of their own, 4.9 ms with
-// every system one-sided.
+// with the systems below 8,192 one-sided in a kernel of their own.
 template <int LAW>
 __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(6))) void batch_sym_kernel(BatchLaunch B,
                                                                                                  int group,

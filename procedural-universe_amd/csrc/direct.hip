@@ -238,50 +238,75 @@ __global__ __launch_bounds__(256) void field_kernel(const float4* __restrict__ s
     }
 }
 
-// The same with the sources shared out twice, for few points: a workgroup
-// holds 64 points (every wavefront the same ones, wave w a quarter of each
-// source tile) and takes the tiles of one chunk, [blockIdx.y * jchunk, +jchunk).
-// part[chunk * m + i] receives the chunk's sums in scaled units.
+// The same with the sources shared out three times, for few points: a workgroup
+// holds 64 points and takes the tiles of one chunk, [blockIdx.y * jchunk,
+// +jchunk); each half of it takes half of the chunk's tiles, and wave w of the half
+// a quarter of each.  part[chunk * m + i] receives the chunk's sums in scaled
+// units.
 //
-// Bound by the pair arithmetic once the chip is full: 4,096 points from
-// 262,144 sources take 0.376 ms with the copies and the sum (2.9e12 pairs/s)
-// on 64 x 16 workgroups, 8.60 ms on the 16 that one workgroup per 256 points
-// over all sources makes.
+// Bound by the pair arithmetic once the chip is full: 65,536 points from 262,144
+// sources 4.9 ms (3.5e12 pairs/s), 5.5 with 256 threads to a workgroup (the
+// partial sums allow 1,024 workgroups, half the waves that the chip holds); with
+// 1,024 threads 4.8, but 100 points take 57 us against 47.  4,096 points 0.36 ms
+// with the copies and the sum, 0.39 with 256 threads, 8.60 ms on the 16
+// workgroups that one per 256 points over all sources makes.
+constexpr int kFieldParts = 2;
+constexpr int kFieldThreads = 256 * kFieldParts;
+
 template <int LAW>
-__global__ __launch_bounds__(256) void field_slice_kernel(const float4* __restrict__ src, int n_src_pad,
+__global__ __launch_bounds__(kFieldThreads) __attribute__((amdgpu_waves_per_eu(8))) void field_slice_kernel(const float4* __restrict__ src, int n_src_pad,
                                                           const float* __restrict__ pts, int m, DirectScale sc,
                                                           int jchunk, float4* __restrict__ part) {
-    __shared__ core::SrcTile tiles[2];
-    __shared__ core::SliceSums sums;
+    __shared__ core::SrcTile tiles[kFieldParts][2];
+    __shared__ core::WaveSums<kFieldThreads / 64> sums;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int i = blockIdx.x * 64 + lane;
     const size_t p = 3 * static_cast<size_t>(min(i, m - 1));
     float xi[1] = {pts[p] * sc.inv_len}, yi[1] = {pts[p + 1] * sc.inv_len}, zi[1] = {pts[p + 2] * sc.inv_len};
     float sx[1], sy[1], sz[1], cx[1], cy[1], cz[1];
     const int j0 = blockIdx.y * jchunk, j1 = min(j0 + jchunk, n_src_pad);
-    core::block_forces_comp<LAW, 1, 256, 4>(tiles, src, j0, j1, sc, xi, yi, zi, sx, sy, sz, cx, cy, cz);
+    const int turns = ((j1 - j0) / kTile + kFieldParts - 1) / kFieldParts;
+    const int part_id = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / 256);
+    const int p0 = j0 + part_id * turns * kTile, p1 = min(p0 + turns * kTile, j1);
+    core::block_forces_comp<LAW, 1, 256, 4, kFieldParts>(tiles[part_id], src, p0, p1, sc, xi, yi, zi, sx, sy, sz, cx,
+                                                         cy, cz, turns);
     float s[3] = {sx[0], sy[0], sz[0]}, c[3] = {cx[0], cy[0], cz[0]};
     core::add_slices(sums, wave, lane, s, c);
     if (wave == 0 && i < m) part[static_cast<size_t>(blockIdx.y) * m + i] = make_float4(s[0], s[1], s[2], 0.f);
 }
 
-// Adds the chunks' sums of each point in chunk order (compensated) and scales
-// them back.
+// Adds the chunks' sums of each point (compensated, in a fixed order) and scales
+// them back.  A workgroup takes 16 points, the 16 threads of each every 16th
+// chunk: with one thread to a point the 1,024 chunks of a single point among
+// 262,144 sources took 0.1 ms of its 0.143.
 __global__ __launch_bounds__(256) void field_sum_kernel(const float4* __restrict__ part, int split, int m,
                                                         DirectScale sc, float* __restrict__ out) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= m) return;
-    float sx = 0.f, sy = 0.f, sz = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;
-    for (int s = 0; s < split; ++s) {
-        const float4 p = part[static_cast<size_t>(s) * m + i];
-        kahan_add(sx, cx, p.x);
-        kahan_add(sy, cy, p.y);
-        kahan_add(sz, cz, p.z);
+    __shared__ float sums[6][16][16];
+    const int pt = threadIdx.x & 15, row = threadIdx.x >> 4;
+    const int i = blockIdx.x * 16 + pt;
+    float s[3] = {0.f, 0.f, 0.f}, c[3] = {0.f, 0.f, 0.f};
+    if (i < m) {
+#pragma unroll 4
+        for (int k = row; k < split; k += 16) {
+            const float4 p = part[static_cast<size_t>(k) * m + i];
+            kahan_add(s[0], c[0], p.x);
+            kahan_add(s[1], c[1], p.y);
+            kahan_add(s[2], c[2], p.z);
+        }
     }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) sums[a][row][pt] = s[a], sums[3 + a][row][pt] = c[a];
+    __syncthreads();
+    if (row != 0 || i >= m) return;
     float* o = out + 3 * static_cast<size_t>(i);
-    o[0] = sx * sc.out;
-    o[1] = sy * sc.out;
-    o[2] = sz * sc.out;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        for (int r = 1; r < min(16, split); ++r) {
+            kahan_add(s[a], c[a], sums[a][r][pt]);
+            kahan_add(s[a], c[a], -sums[3 + a][r][pt]);
+        }
+        o[a] = s[a] * sc.out;
+    }
 }
 
 // Chunks the field's sources are split into (0: field_kernel, no partial
@@ -410,10 +435,10 @@ hipError_t direct_field(const float4* src, int n_src_pad, const float* pts, int 
     const int tiles = n_src_pad / kTile;
     const int jchunk = ((tiles + split - 1) / split) * kTile;
     hipLaunchKernelGGL((r ? field_slice_kernel<NBODY_LAW_R> : field_slice_kernel<NBODY_LAW_P>),
-                       dim3((m + 63) / 64, split), dim3(256), 0, stream, src, n_src_pad, pts, m, sc, jchunk, part);
+                       dim3((m + 63) / 64, split), dim3(kFieldThreads), 0, stream, src, n_src_pad, pts, m, sc, jchunk, part);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(field_sum_kernel, dim3((m + 255) / 256), dim3(256), 0, stream, part, split, m, sc, out);
+    hipLaunchKernelGGL(field_sum_kernel, dim3((m + 15) / 16), dim3(256), 0, stream, part, split, m, sc, out);
     return hipGetLastError();
 }
 

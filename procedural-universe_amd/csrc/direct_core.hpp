@@ -160,18 +160,25 @@ __device__ __forceinline__ void stage_source(const float4 s, const DirectScale& 
 // wavefronts (wave w takes the w-th of SLICES equal runs of the tile), so the
 // lanes of different waves may hold the same targets; the caller adds the
 // waves' sums.  (cx, cy, cz) receive the sums' compensations.
-template <int LAW, int K, int BLOCK, int SLICES>
+//
+// PARTS > 1: the workgroup is PARTS times BLOCK threads, each part with sources
+// and LDS buffers of its own; every part makes `turns` turns (as many as the
+// longest has tiles), those past its last tile over massless sources.
+template <int LAW, int K, int BLOCK, int SLICES, int PARTS = 1>
 __device__ __forceinline__ void block_forces_comp(SrcTile* tiles, const float4* __restrict__ src, const int j0,
                                                   const int j1, const DirectScale& sc, const float (&xi)[K],
                                                   const float (&yi)[K], const float (&zi)[K], float (&sx)[K],
                                                   float (&sy)[K], float (&sz)[K], float (&cx)[K], float (&cy)[K],
-                                                  float (&cz)[K]) {
+                                                  float (&cz)[K], const int turns) {
     static_assert(kTile % BLOCK == 0, "tile must be a multiple of the block");
     static_assert(SLICES == 1 || SLICES == BLOCK / 64, "one slice of the tile per wavefront");
     constexpr int kSlice = kTile / SLICES;
-    const int s0 = SLICES == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6) * kSlice;
     constexpr int PER = kTile / BLOCK;
-    const int tid = threadIdx.x;
+    const int tid = PARTS == 1 ? static_cast<int>(threadIdx.x) : static_cast<int>(threadIdx.x) % BLOCK;
+    const int s0 = SLICES == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6) * kSlice;
+    auto load = [&](int jt, int l) {
+        return PARTS == 1 || jt < j1 ? src[jt + tid + l * BLOCK] : make_float4(0.f, 0.f, 0.f, 0.f);
+    };
     const float tiny = in_vgpr(__FLT_MIN__);
     const float soft = in_vgpr(sc.soft);
 #pragma unroll
@@ -181,17 +188,17 @@ __device__ __forceinline__ void block_forces_comp(SrcTile* tiles, const float4* 
     }
     float4 pre[PER];
 #pragma unroll
-    for (int l = 0; l < PER; ++l) pre[l] = src[j0 + tid + l * BLOCK];
+    for (int l = 0; l < PER; ++l) pre[l] = load(j0, l);
 #pragma unroll
     for (int l = 0; l < PER; ++l) stage_source<LAW>(pre[l], sc, tiles[0].p[tid + l * BLOCK], tiles[0].k[tid + l * BLOCK]);
     __syncthreads();
 
     int buf = 0;
-    for (int jt = j0; jt < j1; jt += kTile) {
-        const bool more = jt + kTile < j1;
+    for (int turn = 0, jt = j0; turn < turns; ++turn, jt += kTile) {
+        const bool more = turn + 1 < turns;
         if (more) {
 #pragma unroll
-            for (int l = 0; l < PER; ++l) pre[l] = src[jt + kTile + tid + l * BLOCK];
+            for (int l = 0; l < PER; ++l) pre[l] = load(jt + kTile, l);
         }
         const SrcTile& T = tiles[buf];
 
@@ -262,18 +269,21 @@ __device__ __forceinline__ void block_forces(SrcTile* tiles, const float4* __res
                                              const DirectScale& sc, const float (&xi)[K], const float (&yi)[K],
                                              const float (&zi)[K], float (&sx)[K], float (&sy)[K], float (&sz)[K]) {
     float cx[K], cy[K], cz[K];
-    block_forces_comp<LAW, K, BLOCK, 1>(tiles, src, j0, j1, sc, xi, yi, zi, sx, sy, sz, cx, cy, cz);
+    block_forces_comp<LAW, K, BLOCK, 1>(tiles, src, j0, j1, sc, xi, yi, zi, sx, sy, sz, cx, cy, cz, (j1 - j0) / kTile);
 }
 
 // The waves' compensated sums (s, c: Kahan's sum and compensation) of the same
 // 64 targets, added in wave order into wave 0's, compensations included (four
 // sums rounded apart cost a third more error than one).  Every thread of the
 // workgroup must call it; only wave 0 returns the totals, in s.
-struct SliceSums {
-    float s[3][3][64], c[3][3][64];
+template <int WAVES>
+struct WaveSums {
+    float s[WAVES - 1][3][64], c[WAVES - 1][3][64];
 };
+using SliceSums = WaveSums<4>;
 
-__device__ __forceinline__ void add_slices(SliceSums& S, int wave, int lane, float (&s)[3], float (&c)[3]) {
+template <int WAVES>
+__device__ __forceinline__ void add_slices(WaveSums<WAVES>& S, int wave, int lane, float (&s)[3], float (&c)[3]) {
     if (wave > 0) {
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
@@ -284,7 +294,7 @@ __device__ __forceinline__ void add_slices(SliceSums& S, int wave, int lane, flo
     __syncthreads();
     if (wave == 0) {
 #pragma unroll
-        for (int w = 0; w < 3; ++w)
+        for (int w = 0; w < WAVES - 1; ++w)
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
                 kahan_add(s[a], c[a], S.s[w][a][lane]);
