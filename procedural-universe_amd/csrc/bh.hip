@@ -928,6 +928,38 @@ __device__ void mass_reduce_block(const MassArgs& A, int block) {
     }
 }
 
+// Small systems (n < ITEMS x kMassThreads): the whole exclusive prefix of quantity
+// q by one workgroup, ITEMS consecutive elements per thread.
+template <int ITEMS>
+__device__ void mass_scan_block(const MassArgs& A, int q) {
+    __shared__ DD wsum[kMassWaves];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, k0 = threadIdx.x * ITEMS;
+    DD* out = A.prefix + static_cast<size_t>(q) * (static_cast<size_t>(A.n) + 1);
+    double v[ITEMS];
+#pragma unroll
+    for (int e = 0; e < ITEMS; ++e) {
+        const int k = min(k0 + e, A.n - 1);
+        const float4 p = A.pos_sorted[k];
+        const double m = A.mass[A.order[k]];
+        const double x = q == 0 ? 1.0 : q == 1 ? p.x : q == 2 ? p.y : p.z;
+        v[e] = k0 + e < A.n ? m * x : 0.0;
+    }
+    DD sum{v[0], 0.0};
+#pragma unroll
+    for (int e = 1; e < ITEMS; ++e) sum = dd_add(sum, DD{v[e], 0.0});
+    const DD incl = wave_scan_dd(sum, lane);
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    DD p{0.0, 0.0};
+    for (int w = 0; w < wave; ++w) p = dd_add(p, wsum[w]);
+    p = dd_add(p, wave_exclusive(incl, lane));
+#pragma unroll
+    for (int e = 0; e < ITEMS; ++e) {
+        if (k0 + e <= A.n) out[k0 + e] = p;
+        p = dd_add(p, DD{v[e], 0.0});
+    }
+}
+
 // The radix tree's nodes and the chunk sums of the mass prefix are
 // independent: one launch, the first A.nchunks workgroups reduce chunks and
 // the others build nodes (neither half reads what the other writes).
@@ -936,6 +968,19 @@ __global__ __launch_bounds__(256) void tree_mass_kernel(TreeArgs T, MassArgs A) 
     build_priority();
     if (static_cast<int>(blockIdx.x) < A.nchunks) mass_reduce_block(A, blockIdx.x);
     else radix_tree_block(T, blockIdx.x - A.nchunks);
+}
+
+// Systems small enough for one workgroup per quantity: the whole prefix in place
+// of the chunk sums (the first four workgroups), beside the tree, which takes
+// longer, and no second launch.  Tree build, us, with the chunk sums and the
+// prefix pass / with ITEMS = 16: 51 / 43 at 500 particles, 56 / 50 at 1,000, 72 /
+// 64 at 4,000; ITEMS = 32 gains 4 at 5,000 and nothing at 8,000, where the scan
+// takes longer than the tree.
+template <int ITEMS>
+__global__ __launch_bounds__(256) void tree_scan_kernel(TreeArgs T, MassArgs A) {
+    build_priority();
+    if (blockIdx.x < 4) mass_scan_block<ITEMS>(A, blockIdx.x);
+    else radix_tree_block(T, blockIdx.x - 4);
 }
 
 // Exclusive scan of the chunk sums (workgroup q scans quantity q).
@@ -2023,12 +2068,17 @@ static nbody_status bh_build(nbody_sim* s, BHState* b) {
     // the sorted masses go to the sort's other key buffer, idle until the next step's keys
     double* mass_sorted = reinterpret_cast<double*>(b->keys[b->sorted_buf ^ 1]);
     MassArgs M{b->pos_sorted, order, s->mass_dev, mass_sorted, n, b->prefix, b->mass_chunk, mchunks, mrows};
-    hipLaunchKernelGGL(tree_mass_kernel, dim3(mchunks + tree_blocks), dim3(256), 0, st, T, M);
-    if (mchunks <= kMassFusedChunks) {
-        hipLaunchKernelGGL(mass_prefix_kernel<true>, dim3(mchunks), dim3(kMassThreads), 0, st, M);
+    if (n < 24 * kMassThreads) {
+        const auto scan = n < 16 * kMassThreads ? tree_scan_kernel<16> : tree_scan_kernel<24>;
+        hipLaunchKernelGGL(scan, dim3(4 + tree_blocks), dim3(256), 0, st, T, M);
     } else {
-        hipLaunchKernelGGL(mass_chunks_kernel, dim3(4), dim3(kMassThreads), 0, st, M);
-        hipLaunchKernelGGL(mass_prefix_kernel<false>, dim3(mchunks), dim3(kMassThreads), 0, st, M);
+        hipLaunchKernelGGL(tree_mass_kernel, dim3(mchunks + tree_blocks), dim3(256), 0, st, T, M);
+        if (mchunks <= kMassFusedChunks) {
+            hipLaunchKernelGGL(mass_prefix_kernel<true>, dim3(mchunks), dim3(kMassThreads), 0, st, M);
+        } else {
+            hipLaunchKernelGGL(mass_chunks_kernel, dim3(4), dim3(kMassThreads), 0, st, M);
+            hipLaunchKernelGGL(mass_prefix_kernel<false>, dim3(mchunks), dim3(kMassThreads), 0, st, M);
+        }
     }
     hipLaunchKernelGGL(cell_com_kernel, dim3(blocks_for(m, 256)), dim3(256), 0, st, b->prefix, n, b->first, b->last,
                        b->info, m, s->cfg.G, b->com);
