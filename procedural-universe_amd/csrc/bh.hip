@@ -15,7 +15,7 @@
 //                    of the root size in integers, so keys equal the CPU's bit
 //                    for bit and the cells are the reference's half-open cubes;
 //  3. sort           merge sort of (key, index): the keys are formed and sorted
-//                    in LDS in tiles of 4,096, then pairs of sorted runs are
+//                    in LDS in tiles, then pairs of sorted runs are
 //                    merged, the earlier run first among equal keys, so the
 //                    order is stable and equals std::stable_sort of the keys;
 //  4. radix tree     binary radix tree over the sorted keys (Karras 2012);
@@ -328,40 +328,39 @@ __global__ void publish_counters_kernel(const unsigned* __restrict__ counters,
 // ---- 3. sort -----------------------------------------------------------------
 //
 // A merge sort, the index carried with the key: one launch forms the keys and
-// sorts tiles of 4,096 in LDS, and each further launch merges pairs of sorted
-// runs, the earlier run first among equal keys; the last one also writes the
-// sorted positions.  In a small system a launch is the cost (about 5 us however
-// little it does), in a large one the bytes: a merge reads and writes each key
-// once.  Eight radix passes of histogram, row scan and scatter, which this
-// replaced, took 17 to 24 launches and read the keys twice a pass.  Tree
-// build, us, radix / merge: 86 / 56 at 1,000 particles, 104 / 72 at 4,000,
-// 130 / 93 at 32,768, 172 / 131 at 200,003, 366 / 291 at 1,048,576,
-// 1,108 / 1,019 at 4,194,304, 4,450 / 4,287 at 16,777,216.
+// sorts tiles of 2,048 or 4,096 in LDS, and each further launch merges pairs of
+// sorted runs, the earlier run first among equal keys; the last one also writes
+// the sorted positions.  In a small system a launch is the cost (about 5 us
+// however little it does), in a large one the bytes: a merge reads and writes
+// each key once (4.7 TB/s at 4,194,304).  Eight radix passes of histogram, row
+// scan and scatter, which this replaced, took 17 to 24 launches and read the keys
+// twice a pass.  Tree build, us, radix / merge: 86 / 55 at 1,000 particles, 104 /
+// 69 at 4,000, 130 / 91 at 32,768, 172 / 130 at 200,003, 366 / 293 at 1,048,576,
+// 1,108 / 1,024 at 4,194,304, 17,793 / 17,784 at 67,108,864.
 //
 // The tile kernel is bound by one compute unit's arithmetic and LDS while there
-// are few tiles (28 us: keys 4.5, nine rounds of merging 1.3 to 2.2 each).
-// Eight keys per thread, four take the same time and sixteen 11 us more; the
-// same eight digit passes with ballots, all in LDS, took 37 us.
+// are few tiles (28 us for 4,096: keys 4.5, nine rounds of merging 1.3 to 2.2
+// each).  Eight keys per thread, four take the same time and sixteen 11 us more;
+// eight digit passes with ballots, all in LDS, took 37 us.
 constexpr int kTileItems = 8;
-constexpr int kTileThreads = 512;
-constexpr int kTileKeys = kTileThreads * kTileItems;
 
 // A tile's place in LDS: one key skipped in every 32, so that threads reading
 // four consecutive keys each do not meet in the same banks.
 __device__ constexpr int tile_at(int i) { return i + (i >> 5); }
 
-template <bool GATHER>
-__global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(const float4* __restrict__ pos, int n,
-                                                                 const RootParams* __restrict__ Rp,
-                                                                 unsigned long long* __restrict__ keys,
-                                                                 unsigned* __restrict__ idx,
-                                                                 unsigned* __restrict__ outside,
-                                                                 float4* __restrict__ pos_out) {
+template <int KEYS, bool GATHER>
+__global__ __launch_bounds__(KEYS / kTileItems) void tile_sort_kernel(const float4* __restrict__ pos, int n,
+                                                                      const RootParams* __restrict__ Rp,
+                                                                      unsigned long long* __restrict__ keys,
+                                                                      unsigned* __restrict__ idx,
+                                                                      unsigned* __restrict__ outside,
+                                                                      float4* __restrict__ pos_out) {
+    constexpr int kThreads = KEYS / kTileItems;
     build_priority();
-    __shared__ unsigned long long sk[tile_at(kTileKeys)];
-    __shared__ unsigned short sl[tile_at(kTileKeys)];
+    __shared__ unsigned long long sk[tile_at(KEYS)];
+    __shared__ unsigned short sl[tile_at(KEYS)];
     const int tid = threadIdx.x;
-    const int base = blockIdx.x * kTileKeys, count = min(kTileKeys, n - base);
+    const int base = blockIdx.x * KEYS, count = min(KEYS, n - base);
     const int mine = tid * kTileItems;  // this thread's keys, and its outputs of every merge
     const RootParams R = *Rp;
     const double inv_odd = 1.0 / static_cast<double>(R.odd);
@@ -369,7 +368,7 @@ __global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(const float4* _
     unsigned loc[kTileItems];
 #pragma unroll
     for (int k = 0; k < kTileItems; ++k) {
-        const int i = k * kTileThreads + tid;
+        const int i = k * kThreads + tid;
         unsigned long long v = ~0ULL;  // past the end: after every key
         if (i < count) {
             bool out;
@@ -441,7 +440,7 @@ __global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(const float4* _
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kTileItems; ++k) {
-        const int i = k * kTileThreads + tid;
+        const int i = k * kThreads + tid;
         if (i < count) {
             const unsigned from = static_cast<unsigned>(base) + sl[tile_at(i)];
             keys[base + i] = sk[tile_at(i)];
@@ -484,7 +483,6 @@ __global__ __launch_bounds__(THREADS) void merge_kernel(const unsigned long long
                                                         const float4* __restrict__ pos,
                                                         float4* __restrict__ pos_out) {
     constexpr int kMergeKeys = THREADS * ITEMS;
-    static_assert(2 * kTileKeys % kMergeKeys == 0, "a workgroup's outputs belong to one pair");
     build_priority();
     __shared__ unsigned long long sk[kMergeKeys];
     __shared__ unsigned si[kMergeKeys];
@@ -2017,17 +2015,27 @@ nbody_status bh_set_theta(nbody_sim* s) {
     return NBODY_OK;
 }
 
-// Merges of at most this many keys in total take small workgroups (512 x 2
-// outputs: more of them, each done sooner), larger ones 1,024 x 4 (a quarter
-// of the searches, longer contiguous runs).  Tree build, us, 512 x 2 /
-// 1,024 x 2 / 512 x 4 / 1,024 x 4: 131 / 132 / 137 / 143 at 200,003, 295 / 289 /
-// 293 / 301 at 1,048,576, 1,127 / 1,062 / 1,049 / 1,019 at 4,194,304.
-constexpr int kSmallMerge = 1 << 20;
-
-template <int THREADS, int ITEMS>
-void merge_runs(BHState* b, int n, const float4* pos, hipStream_t st) {
+// Keys and order by tiles of TILE keys and their merges, THREADS x ITEMS outputs a
+// workgroup; the sorted buffer is b->sorted_buf.
+//
+// Small tiles spread over more compute units and, where systems share the device,
+// find room on them sooner (16 served requests 45.4 -> 45.0 ms); large systems
+// save a merge with large ones.  Tree build, us, 1,024 / 2,048 / 4,096: 62 / 60 /
+// 64 at 4,000 particles, 93 / 91 / 94 at 32,768, 132 / 130 / 131 at 200,003, 307 /
+// 298 / 293 at 1,048,576; 1,041 / 1,024 at 4,194,304 with the last two.  Merges by
+// small workgroups (512 x 2 outputs: more of them, each done sooner) up to
+// 1,048,576, by 1,024 x 4 beyond (a quarter of the searches, longer contiguous
+// runs): 131 / 132 / 137 / 143 at 200,003 with 512 x 2 / 1,024 x 2 / 512 x 4 /
+// 1,024 x 4, 295 / 289 / 293 / 301 at 1,048,576, 1,127 / 1,062 / 1,049 / 1,019 at
+// 4,194,304.
+template <int TILE, int THREADS, int ITEMS>
+void sort_runs(BHState* b, int n, const float4* pos, hipStream_t st) {
+    static_assert(2 * TILE % (THREADS * ITEMS) == 0, "a workgroup's outputs belong to one pair");
+    const auto tiles = n <= TILE ? tile_sort_kernel<TILE, true> : tile_sort_kernel<TILE, false>;
+    hipLaunchKernelGGL(tiles, dim3(blocks_for(n, TILE)), dim3(TILE / kTileItems), 0, st, pos, n, b->root, b->keys[0],
+                       b->idx[0], b->counters, b->pos_sorted);
     int cur = 0;
-    for (int run = kTileKeys; run < n; run *= 2) {
+    for (int run = TILE; run < n; run *= 2) {
         const auto merge =
             2LL * run >= n ? merge_kernel<THREADS, ITEMS, true> : merge_kernel<THREADS, ITEMS, false>;
         hipLaunchKernelGGL(merge, dim3(blocks_for(n, THREADS * ITEMS)), dim3(THREADS), 0, st, b->keys[cur],
@@ -2035,15 +2043,6 @@ void merge_runs(BHState* b, int n, const float4* pos, hipStream_t st) {
         cur ^= 1;
     }
     b->sorted_buf = cur;
-}
-
-// Keys and order by sorted tiles and merges; the sorted buffer is b->sorted_buf.
-void merge_sort(BHState* b, int n, const float4* pos, hipStream_t st) {
-    const auto tiles = n <= kTileKeys ? tile_sort_kernel<true> : tile_sort_kernel<false>;
-    hipLaunchKernelGGL(tiles, dim3(blocks_for(n, kTileKeys)), dim3(kTileThreads), 0, st, pos, n, b->root, b->keys[0],
-                       b->idx[0], b->counters, b->pos_sorted);
-    if (n <= kSmallMerge) merge_runs<512, 2>(b, n, pos, st);
-    else merge_runs<1024, 4>(b, n, pos, st);
 }
 
 // Keys, sort, tree, masses: everything before the traversal.
@@ -2057,7 +2056,9 @@ static nbody_status bh_build(nbody_sim* s, BHState* b) {
         hipLaunchKernelGGL(dynamic_root_kernel, dim3(1), dim3(256), 0, st, b->bounds_partial, nbb, b->root,
                            theta_below(s->cfg.theta), b->thr);
     }
-    merge_sort(b, n, pos, st);
+    if (n <= 1 << 19) sort_runs<2048, 512, 2>(b, n, pos, st);
+    else if (n <= 1 << 20) sort_runs<4096, 512, 2>(b, n, pos, st);
+    else sort_runs<4096, 1024, 4>(b, n, pos, st);
     const unsigned long long* keys = b->keys[b->sorted_buf];
     const unsigned* order = b->idx[b->sorted_buf];
     const int m = n - 1;
