@@ -30,13 +30,13 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 PKG_DIR = os.path.join(ROOT, "procedural-universe_amd")
 
 FP32_PEAK_TFLOPS = 157.3   # MI355X FP32 vector peak (AMD public spec)
-# HBM-side bytes per launch of the fused direct kernel at N = 2^20 with the
-# default shape, from rocprofv3 FETCH_SIZE and WRITE_SIZE scaled by a 256 MiB
-# copy (profiles/direct_force_n1m_law_r_traffic.md).
+# HBM-side bytes per step of the sum over unordered pairs at N = 2^20 (both
+# kernels), from rocprofv3 FETCH_SIZE and WRITE_SIZE scaled by a 256 MiB copy
+# (profiles/direct_force_n1m_law_r_traffic.md).
 DIRECT_1M_TRAFFIC_BYTES = 2.1835e9
-# The same launch's SQ counters (profiles/direct_force_n1m_law_r_counters.md):
-# VALU instructions per pair, VALU instructions issued per SIMD per cycle and
-# rocprof's VALUBusy, at the 2.265 GHz the launch ran at.
+# The force launch's SQ counters (profiles/direct_force_n1m_law_r_counters.md):
+# VALU instructions per interaction (two to a pair), VALU instructions issued per
+# SIMD per cycle and the clock that the launch ran at.
 DIRECT_1M_VALU = {"valu_instructions_per_pair": 13.30, "rsq_per_pair": 1.004, "valu_issue_per_simd_per_clock": 0.326,
                   "valu_lane_ops_per_clock_per_cu": 83.5, "valu_busy_pct": 140, "lds_wait_pct_of_wave_time": 1.0,
                   "clock_ghz": 2.265, "source": "rocprofv3 --pmc, profiles/direct_force_n1m_law_r_counters.md"}
@@ -155,15 +155,15 @@ def bench_batch(pu, args):
             "ic_seconds": t_ic,
         },
         "baseline": {
-            "kind": "sequential per-galaxy plain launches (same kernel and arena, one workgroup per 256 targets, "
+            "kind": "sequential per-galaxy launches (the batch's own sum and arena, one galaxy at a time, "
             "synchronised per galaxy)",
             "steps": seq_steps,
             "value": seq_value,
             "unit": "interactions/s",
             "speedup": value / seq_value,
             "tuned_single_system": {
-                "kind": "sequential per-galaxy launches of the single-system default (sources split over more "
-                "workgroups for small systems, plus a reduction launch)",
+                "kind": "sequential per-galaxy one-sided launches (sources split over more workgroups for small "
+                "systems, plus a reduction launch)",
                 "value": seq[True],
                 "speedup": value / seq[True],
             },
@@ -715,6 +715,8 @@ def main():
     sim.synchronize()
     elapsed = time.perf_counter() - t0
     timing = sim.timing()
+    # the shape that the sum over unordered pairs reports
+    pairs = n >= 16384 and (timing.i_per_lane, timing.block) == (4, 256)
 
     e1 = None if args.no_energy else sim.diagnostics()
 
@@ -757,16 +759,18 @@ def main():
             "unit": "TFLOP/s",
             "frac": achieved_tflops / FP32_PEAK_TFLOPS,
             "traffic": DIRECT_1M_TRAFFIC_BYTES
-            if (n == 1 << 20 and timing.i_per_lane == 1 and timing.block == 256 and timing.split == 1)
+            if (n == 1 << 20 and pairs)
             else None,
             "traffic_source": "rocprofv3 FETCH_SIZE x2.0 + WRITE_SIZE x1.0 (256 MiB copy calibration), "
             "profiles/direct_force_n1m_law_r_traffic.md",
             "algorithmic_bytes": 80.0 * n,
-            "kernel": "direct_force_kernel (fused kick-drift)",
+            "kernel": "sym_force_kernel + sym_reduce_kernel (unordered pairs, kick-drift)"
+            if pairs
+            else "direct_force_kernel or small_step_kernel (one-sided, fused kick-drift)",
             "kernel_ms": force_ms,
             "flop_per_interaction": FLOP_PER_INTERACTION,
             "valu_counters": DIRECT_1M_VALU
-            if (n == 1 << 20 and timing.i_per_lane == 1 and timing.block == 256 and timing.split == 1)
+            if (n == 1 << 20 and pairs)
             else None,
         },
     }

@@ -287,8 +287,9 @@ typedef struct nbody_bh_stats {
     uint64_t interactions;    /* cell + particle interactions since the last nbody_step began   */
     uint32_t outside_root;    /* particles clamped into a fixed root (the reference drops them) */
     uint32_t stack_overflow;  /* nonzero if a traversal stack overflowed (forces invalid)        */
-    uint64_t list_entries;    /* sources evaluated by a whole wavefront (64 lanes, some masked)  */
-    uint64_t cells_opened;    /* cells whose children a wavefront examined                       */
+    uint64_t list_entries;    /* sources evaluated, each by a whole group of particles, some of  */
+                              /* them masked (64 of Morton order; 16 or 32 in small systems)     */
+    uint64_t cells_opened;    /* cells whose children were examined for a group                  */
 } nbody_bh_stats;
 
 /* Counters of the Barnes-Hut steps since the last nbody_step began, or of the

@@ -30,7 +30,7 @@ nbody_status bh_fixed_root(const nbody_config* c, void* out_params);
 // Counters of the steps since the last reset.
 struct BHCounters {
     unsigned long long interactions;  // lanes x list entries they take part in
-    unsigned long long entries;       // list entries (sources evaluated by a whole wave)
+    unsigned long long entries;       // list entries (sources evaluated by a whole group)
     unsigned long long opened;        // cells opened (stack pops)
     unsigned outside;                 // particles clamped into a fixed root
     unsigned overflow;                // nonzero if a traversal stack overflowed

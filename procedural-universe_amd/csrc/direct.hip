@@ -1,5 +1,10 @@
 // Direct-sum gravity on gfx950: O(N^2) pair forces with LDS j-tiles.
 //
+// A step of fewer than 16,384 particles is one launch (small_step_kernel below),
+// a larger one takes every unordered pair once (direct_sym.hip).  The one-sided
+// sum described here, direct_force_kernel, runs where the launch is tuned by hand,
+// where the rows of the pair sums find no room, and as the batch's baseline.
+//
 // Replaces the reference's BruteForceCPU::Exec/Update
 // (src/Sim/BruteForceCPU.cpp:25-73) and the D3D11 pair of compute shaders
 // (shaders/Compute/Gravity.csh:28-48, Update.csh:22-36), written from the

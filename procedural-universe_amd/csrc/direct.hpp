@@ -64,7 +64,9 @@ bool direct_shape_valid(const DirectShape& s);
 // Effective number of j-chunks for a shape at this size (never an empty chunk).
 int direct_effective_split(const DirectShape& s, int n_pad);
 
-// Heuristic shape: enough workgroups to cover all CUs several times.
+// The one-sided launch's shape (systems whose launch is tuned or whose pair rows
+// find no room, and the batch baseline): enough workgroups to cover all CUs
+// several times.
 DirectShape direct_default_shape(int n_pad);
 
 // One force evaluation.  kick = true advances positions/velocities (kick then

@@ -1,5 +1,5 @@
-"""Batch systems of 8,192 particles and more take the sum over unordered pairs:
-both sides of that size, one and several blocks' remainders, both cuts of the
+"""Batch systems that take the sum over unordered pairs: around 8,192 particles,
+one and several blocks' remainders, both cuts of the
 streamed blocks, equal and unequal masses, both laws; alone and in the mix bit
 for bit, against FP64, and with systems joining and leaving so that groups,
 tasks and the rows' buffer are laid out anew.
