@@ -8,9 +8,8 @@
 // + 0.5 per interaction.  Measured, one step of N = 2^20: one-sided 288 ms
 // (3.8e12 interactions/s), 193 ms (5.7e12) here, 177 ms (6.2e12) with equal
 // masses; N = 65,536: 1.25, 0.79, 0.72 ms; N = 20,011 (law P): 0.151, 0.120,
-// 0.108 ms.  Still bound by issue: 0.32 VALU instructions per SIMD per cycle
-// were measured at N = 524,288, where the same step in a register-only loop
-// reaches 0.34.
+// 0.108 ms.  Still bound by issue: 0.389 VALU instructions per SIMD per cycle at
+// N = 2^20 (2.13 GHz under this load), 0.326 one-sided.
 //
 // Layout.  A wavefront holds 256 resident particles, four per lane, with their
 // sums in registers, and streams sets of 64 particles past them: at step s
