@@ -1189,6 +1189,15 @@ using core::kahan_add;
 // moves only the address and the lane mask.
 constexpr int kListCap = 96;
 
+// Two wavefronts with a group of 64 have a list each for 32 of its particles (see
+// traverse_kernel), evaluated when a step leaves kOwnFlush entries or more in it; a
+// step adds at most 64 per wavefront.  More room before the evaluation costs
+// workgroups per CU: 5.10, 5.23, 5.41 ms at 4,194,304 with 16, 32, 64.
+template <int G, int W>
+constexpr bool own_lists = G == 64 && W == 2;
+constexpr int kOwnFlush = 16;
+constexpr int kOwnCap = 64 * 2 + kOwnFlush;
+
 // Margins of the box verdicts: 64 FP32 ulps, above the 16 that the rounding of
 // a lane's squared distance and of the box's nearest and farthest squared
 // distances can add up to.
@@ -1242,25 +1251,30 @@ __device__ __forceinline__ void write_entry(float4* lsrc, float* lk, uint2* lmas
 // SLOTS > 1 (a wave of 64 / SLOTS particles): slot s evaluates the s-th of every
 // SLOTS groups of four; the caller has padded the list to whole rounds of
 // 4 x SLOTS entries.  `lane` is then the lane's particle.
-template <int LAW, int SLOTS>
-__device__ __forceinline__ void flush_list(const float4* lsrc, const float* lk, const uint2* lmask, int cnt, int lane,
-                                           int slot, float px, float py, float pz, float soft, float& sx, float& sy,
+template <int LAW, int SLOTS, int WORDS>
+__device__ __forceinline__ void flush_list(const float4* lsrc, const float* lk, const unsigned* words, int cnt,
+                                           int lane, int slot, float px, float py, float pz, float soft, float& sx, float& sy,
                                            float& sz, float& cx, float& cy, float& cz) {
     const float tiny = core::in_vgpr(__FLT_MIN__);
     float ax = 0.f, ay = 0.f, az = 0.f;
-    // the lane's word of every entry's mask
-    const unsigned* words = reinterpret_cast<const unsigned*>(lmask) + (lane >> 5);
+    if constexpr (WORDS == 2) words += lane >> 5;  // the lane's word of every entry's mask
     if constexpr (SLOTS > 1) {
         lsrc += 4 * slot;
         lk += 4 * slot;
-        words += 8 * slot;
+        words += 4 * WORDS * slot;
     }
     const int cnt4 = SLOTS == 1 ? cnt & ~3 : cnt;
     for (int e = 0; e < cnt4; e += 4 * SLOTS) {
         float4 src[4];
         float dx[4], dy[4], dz[4], q[4];
-        const float4 k4 = *reinterpret_cast<const float4*>(lk + e);
-        const float kg[4] = {k4.x, k4.y, k4.z, k4.w};
+        float kg[4];
+        if constexpr (WORDS == 2) {
+            const float4 k4 = *reinterpret_cast<const float4*>(lk + e);
+            kg[0] = k4.x, kg[1] = k4.y, kg[2] = k4.z, kg[3] = k4.w;
+        } else {  // from any entry on
+#pragma unroll
+            for (int g = 0; g < 4; ++g) kg[g] = lk[e + g];
+        }
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             src[g] = lsrc[e + g];
@@ -1285,7 +1299,7 @@ __device__ __forceinline__ void flush_list(const float4* lsrc, const float* lk, 
             } else {
                 f = (src[g].w * q[g]) * (q[g] * q[g]);
             }
-            f = lane_masked(f, words[(e + g) * 2], lane);
+            f = lane_masked(f, words[(e + g) * WORDS], lane);
             ax = __builtin_fmaf(dx[g], f, ax);
             ay = __builtin_fmaf(dy[g], f, ay);
             az = __builtin_fmaf(dz[g], f, az);
@@ -1312,7 +1326,7 @@ __device__ __forceinline__ void flush_list(const float4* lsrc, const float* lk, 
         } else {
             f = (src.w * q) * (q * q);
         }
-        f = lane_masked(f, words[e * 2], lane);
+        f = lane_masked(f, words[e * WORDS], lane);
         ax = __builtin_fmaf(dx, f, ax);
         ay = __builtin_fmaf(dy, f, ay);
         az = __builtin_fmaf(dz, f, az);
@@ -1353,13 +1367,28 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
 // step's cells out in runs of eight instead of round robin left the later
 // wavefronts idle while the stack is short (90 us).
 //
+// Own lists (G = 64, W = 2).  An entry of the group's list is evaluated by all its
+// lanes, of which 46% use it (N = 4,194,304, theta 0.5); a list per half group has
+// 17% fewer rows in all, and the walk is still the whole group's.  Wavefront w
+// keeps the list of particles [32 w, 32 w + 32): both decide for all 64, each
+// child's entry goes to the lists that its mask reaches (each wavefront's counts
+// through LDS, at the barrier that the pushes have), and each wavefront evaluates its own
+// list two entries at a time.  11% fewer VALU instructions, 5.47 -> 5.10 ms at
+// 4,194,304 (law P 5.29 -> 4.80), 2.51 -> 2.34 at 2,097,152, 0.91 -> 0.83 at
+// 1,048,576.  Quarter lists of four wavefronts save 29% of the rows, but their
+// space and registers leave four or five waves per SIMD: 0.68 ms against 0.62 at
+// 524,288.  79 VGPRs and 12.2 KB to a workgroup: six waves per SIMD; held to
+// seven ten registers spill (5.44).  Blocks in scalar registers, as one
+// wavefront has them: 5.18 ms without.
+//
 // At most 72 VGPRs for W > 1 (seven waves per SIMD): 83 are taken freely, five
 // waves, 3% to 7% slower with G = 16 and 32.  With W = 1 72 (70 for law P),
 // while the workgroup limit keeps 24 one-wave workgroups per CU (six per SIMD)
 // resident.  The box's six bounds stay in vector registers: held in scalar
 // registers they were spilled and reloaded every batch (2.3% slower).
 template <int LAW, int G, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W > 1 ? 7 : 6))) void traverse_kernel(
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W > 1 && !own_lists<G, W> ? 7 : 6)))
+void traverse_kernel(
     const float4* __restrict__ pos_sorted, const ChildBlock* __restrict__ blocks, const int* __restrict__ node_first,
     const int* __restrict__ node_last, TravArgs A) {
     // The walk runs at raised wave priority and drops it while the list is
@@ -1371,15 +1400,24 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W > 1 ? 
     constexpr int kCap = stack_cap(W);
     __shared__ int stk_node[kCap];
     __shared__ uint2 stk_mask[kCap];
-    __shared__ float4 lsrc[W][kListCap];
-    __shared__ __align__(16) float lk[W][kListCap];
-    __shared__ uint2 lmask[W][kListCap];
+    constexpr bool OWN = own_lists<G, W>;
+    constexpr int P = OWN ? G / W : G;                 // the particles a wavefront's list is for
+    constexpr int EVAL = 64 / P;                       // slots of its evaluation
+    constexpr int kRound = 4 * EVAL;                   // entries a round of it takes
+    constexpr unsigned kOwn = P >= 32 ? ~0u : (1u << (P & 31)) - 1u;  // their bits, shifted down
+    constexpr int kCapL = OWN ? kOwnCap : kListCap;
+    constexpr int kCapAll = OWN ? kCapL + kRound : kListCap;  // own lists: a round beside the list
+    __shared__ float4 lsrc[W][kCapAll];
+    __shared__ __align__(16) float lk[W][kCapAll];
+    __shared__ std::conditional_t<OWN, unsigned, uint2> lmask[W][kCapAll];
     __shared__ unsigned long long red[3][W];
     __shared__ int wave_pushed[W];
+    __shared__ unsigned wave_listed[W];  // own lists: entries for each, 16 bits a count
+    static_assert(!OWN || (kCapL >= 64 * W + kOwnFlush - 1 && kOwnFlush >= kRound), "a step's entries fit");
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: list and stack addresses in SGPRs
     constexpr int SLOTS = 64 / G;
-    constexpr bool kScalar = G == 64 && W == 1;  // the tested cells' blocks in scalar registers
+    constexpr bool kScalar = G == 64 && (W == 1 || own_lists<G, W>);  // the tested cells' blocks in scalar registers
     constexpr unsigned long long kGroup = G == 64 ? ~0ull : (1ull << (G & 63)) - 1ull;  // the particles' mask bits
     const int mine = lane & (G - 1), slot = lane / G;
     const int blk = xcd_block<G>(blockIdx.x, gridDim.x);
@@ -1388,7 +1426,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W > 1 ? 
     const bool valid = t < A.n;
     const float4 me = pos_sorted[valid ? t : A.n - 1];
     // the particle in the pair arithmetic's scaled units (the decisions use me)
-    const float mx = me.x * A.sc.inv_len, my = me.y * A.sc.inv_len, mz = me.z * A.sc.inv_len;
+    const int own_base = OWN ? wave_base + wave * P : wave_base;
+    const int emine = OWN ? lane & (P - 1) : mine, eslot = OWN ? lane / P : slot;
+    float4 ev = me;
+    if constexpr (OWN) ev = pos_sorted[min(own_base + emine, A.n - 1)];
+    const float mx = ev.x * A.sc.inv_len, my = ev.y * A.sc.inv_len, mz = ev.z * A.sc.inv_len;
     const float soft = core::in_vgpr(A.sc.soft);
     float sx = 0.f, sy = 0.f, sz = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;
     // wave-uniform counters and list length
@@ -1404,38 +1446,75 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W > 1 ? 
     // its opening threshold, in lane 8j + s; lanes of particle children and
     // lanes beyond the batch's children are not used
     unsigned ge_lo = 0u, ge_hi = 0u;
+    int len[W] = {};  // own lists: entries in each (uniform over the workgroup)
+
+    // Own lists: entry `at` of this wavefront's, and the evaluation of the whole
+    // rounds [from, to).
+    auto put = [&](int w, int at, const float4 p, float k, unsigned m) {
+        if constexpr (OWN) lsrc[w][at] = p, lk[w][at] = k, lmask[w][at] = m;
+    };
+    auto evaluate = [&](int from, int to) {
+        if constexpr (OWN) {
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_s_setprio(0);
+            flush_list<LAW, EVAL, 1>(lsrc[wave] + from, lk[wave] + from, lmask[wave] + from, to - from, emine, eslot, mx,
+                                     my, mz, soft, sx, sy, sz, cx, cy, cz);
+            __builtin_amdgcn_s_setprio(1);
+            __builtin_amdgcn_wave_barrier();
+            lane_total += lane_count;
+            lane_count = 0;
+        }
+    };
+    // One round beside the list: lane i's source (G m in w) for the own
+    // particles of mask m, empty masks beyond the sources.
+    auto round_alone = [&](const float4 src, unsigned m) {
+        if constexpr (OWN) {
+            if (lane < kRound) {
+                float4 p;
+                float k;
+                core::stage_factored<LAW>(make_float4(src.x, src.y, src.z, core::mass_factor<LAW>(src.w, A.sc)), A.sc,
+                                          p, k);
+                put(wave, kCapL + lane, p, k, m);
+                lane_count += __popc(m);
+            }
+            evaluate(kCapL, kCapL + kRound);
+        }
+    };
 
     // Append a source (x, y, z, G m) held in scalar registers (written by lane 0).
     auto append = [&](const float4 src, unsigned long long mask) {
-        if (lane == 0)
-            write_entry<LAW>(lsrc[wave], lk[wave], lmask[wave], cnt,
-                             make_float4(src.x, src.y, src.z, core::mass_factor<LAW>(src.w, A.sc)), mask, A.sc);
+        if constexpr (!OWN)
+            if (lane == 0)
+                write_entry<LAW>(lsrc[wave], lk[wave], lmask[wave], cnt,
+                                 make_float4(src.x, src.y, src.z, core::mass_factor<LAW>(src.w, A.sc)), mask, A.sc);
         count += static_cast<unsigned long long>(__popcll(mask));
         ++cnt;
     };
     auto flush = [&]() {
-        entries += static_cast<unsigned long long>(cnt);
-        int total = __builtin_amdgcn_readfirstlane(cnt);
-        __builtin_amdgcn_wave_barrier();
-        if constexpr (SLOTS > 1) {
-            // whole rounds of four entries per slot: empty masks, finite sources
-            const int whole = (total + 4 * SLOTS - 1) & ~(4 * SLOTS - 1);
-            if (total + lane < whole) {
-                lsrc[wave][total + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
-                lk[wave][total + lane] = 0.f;
-                lmask[wave][total + lane] = make_uint2(0u, 0u);
-            }
-            total = whole;
+        if constexpr (!OWN) {
+            entries += static_cast<unsigned long long>(cnt);
+            int total = __builtin_amdgcn_readfirstlane(cnt);
             __builtin_amdgcn_wave_barrier();
+            if constexpr (SLOTS > 1) {
+                // whole rounds of four entries per slot: empty masks, finite sources
+                const int whole = (total + 4 * SLOTS - 1) & ~(4 * SLOTS - 1);
+                if (total + lane < whole) {
+                    lsrc[wave][total + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+                    lk[wave][total + lane] = 0.f;
+                    lmask[wave][total + lane] = make_uint2(0u, 0u);
+                }
+                total = whole;
+                __builtin_amdgcn_wave_barrier();
+            }
+            __builtin_amdgcn_s_setprio(0);  // the list at normal priority, the walk raised (kernel start)
+            flush_list<LAW, SLOTS, 2>(lsrc[wave], lk[wave], reinterpret_cast<const unsigned*>(lmask[wave]), total, mine,
+                                      slot, mx, my, mz, soft, sx, sy, sz, cx, cy, cz);
+            __builtin_amdgcn_s_setprio(1);
+            __builtin_amdgcn_wave_barrier();
+            cnt = 0;
+            lane_total += lane_count;
+            lane_count = 0;
         }
-        __builtin_amdgcn_s_setprio(0);  // the list at normal priority, the walk raised (kernel start)
-        flush_list<LAW, SLOTS>(lsrc[wave], lk[wave], lmask[wave], total, mine, slot, mx, my, mz, soft, sx, sy, sz, cx,
-                               cy, cz);
-        __builtin_amdgcn_s_setprio(1);
-        __builtin_amdgcn_wave_barrier();
-        cnt = 0;
-        lane_total += lane_count;
-        lane_count = 0;
     };
     // the lanes of a particle's own position never interact with it
     auto without_self = [&](unsigned long long m, int q) {
@@ -1448,6 +1527,16 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W > 1 ? 
         const int node = flagged & ~kBucketFlag;
         const unsigned long long mask = (static_cast<unsigned long long>(hi32) << 32) | lo32;
         const int f = node_first[node], l = node_last[node];
+        if constexpr (OWN) {  // every wavefront for its own particles
+            const unsigned m = static_cast<unsigned>(mask >> (wave * P)) & kOwn;
+            for (int q0 = f; q0 <= l; q0 += kRound) {
+                const int q = q0 + lane, o = q - own_base;
+                const unsigned not_self = o >= 0 && o < P ? ~(1u << o) : ~0u;
+                round_alone(pos_sorted[min(q, l)], q <= l ? m & not_self : 0u);
+            }
+            if (wave == 0) entries += static_cast<unsigned long long>(l - f + 1);
+            return;
+        }
         for (int q = f; q <= l; ++q) {
             if (cnt > kListCap - 4) flush();
             const unsigned long long m = without_self(mask, q);
@@ -1487,7 +1576,12 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W > 1 ? 
         const float dx = me.x - c.x, dy = me.y - c.y, dz = me.z - c.z;
         const float r2 = (dx * dx + dy * dy) + dz * dz;
         const unsigned long long am = __builtin_amdgcn_ballot_w64(!(r2 < A.thr[root_level])) & all;
-        if (am && wave == 0) append(c, am);
+        if constexpr (OWN) {
+            if (am) round_alone(c, lane == 0 ? static_cast<unsigned>(am >> (wave * P)) & kOwn : 0u);
+            if (am && wave == 0) ++entries;
+        } else {
+            if (am && wave == 0) append(c, am);
+        }
         const unsigned long long om = all & ~am;
         if (om) {
             if (tid == 0) {
@@ -1548,6 +1642,18 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W > 1 ? 
             k = (all_k - wave + W - 1) / W;
             opened += static_cast<unsigned long long>(k);
             unsigned long long bk = __builtin_amdgcn_ballot_w64(in_batch && (vcell & kBucketFlag) != 0);
+            if constexpr (OWN) {
+                // the whole batch's buckets, by every wavefront for its own particles
+                bk = __builtin_amdgcn_ballot_w64((stk_node[sp - 1 - min(lane, all_k - 1)] & kBucketFlag) != 0 &&
+                                                 lane < all_k);
+                while (bk) {
+                    const int at = sp - 1 - static_cast<int>(__builtin_ctzll(bk));
+                    bk &= bk - 1ull;
+                    bucket(__builtin_amdgcn_readfirstlane(stk_node[at]),
+                           __builtin_amdgcn_readfirstlane(stk_mask[at].x),
+                           __builtin_amdgcn_readfirstlane(stk_mask[at].y));
+                }
+            }
             while (bk) {
                 const int l = static_cast<int>(__builtin_ctzll(bk)) & ~7;
                 bk &= ~(0xffull << l);
@@ -1555,7 +1661,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W > 1 ? 
                        __builtin_amdgcn_readlane(static_cast<int>(vm.y), l));
             }
             in_batch = in_batch && (vcell & kBucketFlag) == 0;
-            if (cnt > kListCap - 8 * k) flush();
+            if constexpr (!OWN)
+                if (cnt > kListCap - 8 * k) flush();
         }
         const int base = sp - (W == 1 ? k : all_k);
         const unsigned long long batch = __builtin_amdgcn_ballot_w64(in_batch);
@@ -1650,13 +1757,25 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W > 1 ? 
         // List entries, in lane order, written by the children's lanes.
         const bool wl = child && am != 0ull;
         const unsigned long long has_l = __builtin_amdgcn_ballot_w64(am != 0ull) & children;
-        if (wl) {
+        // own lists: the child's mask in each, and which children have one
+        unsigned long long has_part[W];
+        if constexpr (OWN) {
+            entries += static_cast<unsigned long long>(__popcll(has_l));
+            if (wl) lane_count += __popcll(am);
+            unsigned counts = 0u;
+#pragma unroll
+            for (int q = 0; q < W; ++q) {
+                has_part[q] = __builtin_amdgcn_ballot_w64((static_cast<unsigned>(am >> (q * P)) & kOwn) != 0u) & children;
+                counts |= static_cast<unsigned>(__popcll(has_part[q])) << (16 * q);
+            }
+            if (lane == 0) wave_listed[wave] = counts;
+        } else if (wl) {
             const int at = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
                 static_cast<unsigned>(has_l >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(has_l), cnt)));
             write_entry<LAW>(lsrc[wave], lk[wave], lmask[wave], at, vsrc, am, A.sc);
             lane_count += __popcll(am);
         }
-        cnt += __popcll(has_l);
+        if constexpr (!OWN) cnt += __popcll(has_l);
         // Opened cells onto the stack in place of the batch, in reverse lane
         // order: the top cell's first opened child ends on top.
         const bool ws = child && om != 0ull;  // a cell: a particle's ge is all lanes
@@ -1702,24 +1821,72 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W > 1 ? 
             sp = kCap;
             overflowed = true;
         }
-        if constexpr (W > 1) __syncthreads();
+        if constexpr (OWN) {
+            // The step's entries into the lists, in the order of the wavefronts
+            // and lanes.
+            unsigned before = 0, sum = 0;
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const unsigned c = wave_listed[w];
+                sum += c;
+                if (w < wave) before += c;
+            }
+            sum = __builtin_amdgcn_readfirstlane(sum);
+            before = __builtin_amdgcn_readfirstlane(before);
+            float4 p;
+            float k;
+            core::stage_factored<LAW>(vsrc, A.sc, p, k);
+#pragma unroll
+            for (int q = 0; q < W; ++q) {
+                const unsigned long long has = has_part[q];
+                const int at = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                    static_cast<unsigned>(has >> 32),
+                    __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(has), len[q] + (before >> (16 * q) & 0xffffu))));
+                const unsigned part = static_cast<unsigned>(am >> (q * P)) & kOwn;
+                if (child && part != 0u) put(q, at, p, k, part);
+                len[q] += static_cast<int>(sum >> (16 * q) & 0xffffu);
+            }
+            __syncthreads();
+            int left = 0, full = 0;
+#pragma unroll
+            for (int q = 0; q < W; ++q)
+                if (len[q] >= kOwnFlush) {
+                    const int l = len[q] & (kRound - 1);  // stay, at the list's start
+                    if (q == wave) left = l, full = len[q];
+                    len[q] = l;
+                }
+            if (left < full) evaluate(left, full);
+        } else if constexpr (W > 1) {
+            __syncthreads();
+        }
     }
     if (overflowed && lane == 0) atomicOr(A.overflow, 1u);
-    if (cnt) flush();
+    if constexpr (OWN) {
+        int rest = 0;
+#pragma unroll
+        for (int q = 0; q < W; ++q)
+            if (q == wave) rest = len[q];
+        const int whole = (rest + kRound - 1) & ~(kRound - 1);
+        if (rest + lane < whole) put(wave, rest + lane, make_float4(0.f, 0.f, 0.f, 0.f), 0.f, 0u);
+        if (whole) evaluate(0, whole);
+        lane_total += lane_count;
+    } else {
+        if (cnt) flush();
+    }
     for (int off = 32; off > 0; off >>= 1) lane_total += __shfl_xor(lane_total, off);
     count += lane_total;
 
-    if constexpr (SLOTS > 1) {
+    if constexpr (EVAL > 1) {
         // the slots' sums, compensations included, in a fixed order
 #pragma unroll
-        for (int off = G; off < 64; off <<= 1) {
+        for (int off = P; off < 64; off <<= 1) {
             const float ox = __shfl_xor(sx, off), oy = __shfl_xor(sy, off), oz = __shfl_xor(sz, off);
             const float qx = __shfl_xor(cx, off), qy = __shfl_xor(cy, off), qz = __shfl_xor(cz, off);
             kahan_add(sx, cx, ox), kahan_add(sy, cy, oy), kahan_add(sz, cz, oz);
             kahan_add(sx, cx, -qx), kahan_add(sy, cy, -qy), kahan_add(sz, cz, -qz);
         }
     }
-    if constexpr (W > 1) {
+    if constexpr (W > 1 && !OWN) {
         // the wavefronts' sums likewise, through the first's list
         float* out = reinterpret_cast<float*>(lsrc[wave]);
         static_assert(sizeof(lsrc[0]) >= 6 * G * sizeof(float), "a wavefront's sums fit its list");
@@ -1738,8 +1905,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W > 1 ? 
             }
         }
     }
-    if (wave == 0 && valid && slot == 0) {
-        const unsigned p = A.order[t];
+    const int to = OWN ? own_base + lane : t;
+    if (OWN ? lane < P && to < A.n : wave == 0 && valid && slot == 0) {
+        const unsigned p = A.order[to];
         // back from scaled units (a power of two: exact)
         const float ax = sx * A.sc.out, ay = sy * A.sc.out, az = sz * A.sc.out;
         A.acc[p] = make_float4(ax, ay, az, 0.f);
@@ -1851,19 +2019,27 @@ inline int mass_rows(int n) {
 // One wavefront after another waits for its cells, decides, and waits again, so
 // a system with few groups is bound by the longest walk: several wavefronts to a
 // group shorten it, and more of them the fewer groups there are.  Small groups
-// make more and shorter walks, but more in all.  Force pass, us:
+// make more and shorter walks, but more in all.  Force pass, us (64x2 with a list
+// per half group):
 //                                 16x8   32x8   32x4   64x8   64x4   64x2   64x1
-//   Plummer, theta 0.6:   4,000     30     36     47     47     74    115
+//   Plummer, theta 0.6:   4,000     30     36     47     47     74
 //                         8,192     38     39     52     53     80
 //                        16,384     63     50     63     60     94
-//                        32,768    106     83     81     83    104    162    293
-//                        65,536           142    125    134    131           331
-//                       131,072                  192    226    210    222    333
-//   encounter, 0.5:     262,144                  354    379    339    425    556
-//                       524,288                  700    715    620    676    862
-//              0.6:   1,048,576                               988    933    979
-//              0.5:   2,097,152                 2954   3133   2557   2465   2573
-//              0.8:   4,194,304                 3324   3896   2743   2439   2291
+//                        32,768    106     83     81     83    104    165    293
+//                        65,536           142    125    134    131    185    331
+//                       131,072                  192    226    193    205    333
+//                       393,216                                475    461
+//   encounter, 0.5:     262,144                  354    379    339           556
+//                       300,000                                373    398
+//                       524,288                  700    715    620    629    862
+//              0.6:   1,048,576                               988    825    979
+//              0.5:   2,097,152                 2954   3133   2557   2334   2573
+//              0.5:   4,194,304                                      5099   5466
+//              0.8:   4,194,304                 3324   3896   2743   2212   2244
+//              2.0:   4,194,304                                       880    866
+//              0.7:   8,388,608                                      5620   5837
+//   Plummer,   0.5:  16,777,216                                     27142  28379
+//              1.0:  16,777,216                                      8144   7989
 // (One wavefront to a group of 8, 16 or 32: 53 at 4,000, 138 at 32,768, 234 at
 // 131,072, 309 at 200,003, where 64x4 takes 264.)
 struct TravShape {
@@ -1874,8 +2050,8 @@ inline TravShape trav_shape(int n) {
     if (n <= 12288) return {16, 8};
     if (n <= 24576) return {32, 8};
     if (n <= 163840) return {32, 4};
-    if (n <= 786432) return {64, 4};
-    if (n <= 2621440) return {64, 2};
+    if (n <= 393216) return {64, 4};
+    if (n <= 8388608) return {64, 2};
     return {64, 1};
 }
 
