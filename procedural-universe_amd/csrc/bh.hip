@@ -1189,14 +1189,13 @@ using core::kahan_add;
 // moves only the address and the lane mask.
 constexpr int kListCap = 96;
 
-// Two wavefronts with a group of 64 have a list each for 32 of its particles (see
-// traverse_kernel), evaluated when a step leaves kOwnFlush entries or more in it; a
-// step adds at most 64 per wavefront.  More room before the evaluation costs
-// workgroups per CU: 5.10, 5.23, 5.41 ms at 4,194,304 with 16, 32, 64.
+// Two or four wavefronts with a group of 64 keep a list for each half of its
+// particles (see traverse_kernel), evaluated when a step leaves kOwnFlush entries or
+// more in it; a step adds at most 64 per wavefront.  More room before the evaluation
+// costs workgroups per CU: 5.10, 5.23, 5.41 ms at 4,194,304 with 16, 32, 64.
 template <int G, int W>
-constexpr bool own_lists = G == 64 && W == 2;
+constexpr bool own_lists = G == 64 && (W == 2 || W == 4);
 constexpr int kOwnFlush = 16;
-constexpr int kOwnCap = 64 * 2 + kOwnFlush;
 
 // Margins of the box verdicts: 64 FP32 ulps, above the 16 that the rounding of
 // a lane's squared distance and of the box's nearest and farthest squared
@@ -1367,19 +1366,20 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
 // step's cells out in runs of eight instead of round robin left the later
 // wavefronts idle while the stack is short (90 us).
 //
-// Own lists (G = 64, W = 2).  An entry of the group's list is evaluated by all its
-// lanes, of which 46% use it (N = 4,194,304, theta 0.5); a list per half group has
-// 17% fewer rows in all, and the walk is still the whole group's.  Wavefront w
-// keeps the list of particles [32 w, 32 w + 32): both decide for all 64, each
-// child's entry goes to the lists that its mask reaches (each wavefront's counts
-// through LDS, at the barrier that the pushes have), and each wavefront evaluates its own
-// list two entries at a time.  11% fewer VALU instructions, 5.47 -> 5.10 ms at
-// 4,194,304 (law P 5.29 -> 4.80), 2.51 -> 2.34 at 2,097,152, 0.91 -> 0.83 at
-// 1,048,576.  Quarter lists of four wavefronts save 29% of the rows, but their
-// space and registers leave four or five waves per SIMD: 0.68 ms against 0.62 at
-// 524,288.  79 VGPRs and 12.2 KB to a workgroup: six waves per SIMD; held to
+// Own lists (G = 64, W = 2 or 4).  An entry of the group's list is evaluated by all
+// its lanes, of which 46% use it (N = 4,194,304, theta 0.5); a list per half group
+// has 17% fewer rows in all, and the walk is still the whole group's.  List h is
+// for particles [32 h, 32 h + 32): every wavefront decides for all 64, each child's
+// entry goes to the lists that its mask reaches (every wavefront's counts through
+// LDS, at the barrier that the pushes have), and list h is evaluated by the
+// wavefronts w with w mod 2 = h, two entries at a time each.  11% fewer VALU
+// instructions: 5.47 -> 5.10 ms at 4,194,304 (law P 5.29 -> 4.80), 2.51 -> 2.34 at
+// 2,097,152, 0.91 -> 0.83 at 1,048,576; with four wavefronts 0.264 -> 0.243 at
+// 200,003 (law P), 0.124 -> 0.117 at 65,536.  Quarter lists of four wavefronts save
+// 29% of the rows, but their space and registers leave four or five waves per
+// SIMD: 0.68 ms against 0.62 at 524,288.  80 VGPRs, six waves per SIMD; held to
 // seven ten registers spill (5.44).  Blocks in scalar registers, as one
-// wavefront has them: 5.18 ms without.
+// wavefront has them: 5.18 ms without, law P at 200,003 0.252.
 //
 // At most 72 VGPRs for W > 1 (seven waves per SIMD): 83 are taken freely, five
 // waves, 3% to 7% slower with G = 16 and 32.  With W = 1 72 (70 for law P),
@@ -1401,19 +1401,20 @@ void traverse_kernel(
     __shared__ int stk_node[kCap];
     __shared__ uint2 stk_mask[kCap];
     constexpr bool OWN = own_lists<G, W>;
-    constexpr int P = OWN ? G / W : G;                 // the particles a wavefront's list is for
-    constexpr int EVAL = 64 / P;                       // slots of its evaluation
-    constexpr int kRound = 4 * EVAL;                   // entries a round of it takes
+    constexpr int P = OWN ? G / 2 : G;                          // the particles a list is for
+    constexpr int LISTS = OWN ? 2 : W;
+    constexpr int EVAL = 64 / P;                                // slots of a wavefront's evaluation
+    constexpr int kRound = OWN ? 4 * W : 4 * EVAL;              // entries a round of all the list's wavefronts takes
     constexpr unsigned kOwn = P >= 32 ? ~0u : (1u << (P & 31)) - 1u;  // their bits, shifted down
-    constexpr int kCapL = OWN ? kOwnCap : kListCap;
-    constexpr int kCapAll = OWN ? kCapL + kRound : kListCap;  // own lists: a round beside the list
-    __shared__ float4 lsrc[W][kCapAll];
-    __shared__ __align__(16) float lk[W][kCapAll];
-    __shared__ std::conditional_t<OWN, unsigned, uint2> lmask[W][kCapAll];
+    constexpr int kCapL = OWN ? 64 * W + kOwnFlush : kListCap;
+    constexpr int kCapAll = OWN ? kCapL + W / 2 * kRound : kListCap;  // own lists: a round for each wavefront beside it
+    __shared__ float4 lsrc[LISTS][kCapAll];
+    __shared__ __align__(16) float lk[LISTS][kCapAll];
+    __shared__ std::conditional_t<OWN, unsigned, uint2> lmask[LISTS][kCapAll];
     __shared__ unsigned long long red[3][W];
     __shared__ int wave_pushed[W];
     __shared__ unsigned wave_listed[W];  // own lists: entries for each, 16 bits a count
-    static_assert(!OWN || (kCapL >= 64 * W + kOwnFlush - 1 && kOwnFlush >= kRound), "a step's entries fit");
+    static_assert(!OWN || kOwnFlush >= kRound, "what stays in a list is less than a round");
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: list and stack addresses in SGPRs
     constexpr int SLOTS = 64 / G;
@@ -1426,8 +1427,10 @@ void traverse_kernel(
     const bool valid = t < A.n;
     const float4 me = pos_sorted[valid ? t : A.n - 1];
     // the particle in the pair arithmetic's scaled units (the decisions use me)
-    const int own_base = OWN ? wave_base + wave * P : wave_base;
-    const int emine = OWN ? lane & (P - 1) : mine, eslot = OWN ? lane / P : slot;
+    // the wavefront's list, and which of the list's wavefronts it is
+    const int half = OWN && W > 2 ? wave & 1 : wave, share_of = OWN && W > 2 ? wave >> 1 : 0;
+    const int own_base = OWN ? wave_base + half * P : wave_base;
+    const int emine = OWN ? lane & (P - 1) : mine, eslot = OWN ? share_of * EVAL + lane / P : slot;
     float4 ev = me;
     if constexpr (OWN) ev = pos_sorted[min(own_base + emine, A.n - 1)];
     const float mx = ev.x * A.sc.inv_len, my = ev.y * A.sc.inv_len, mz = ev.z * A.sc.inv_len;
@@ -1446,7 +1449,7 @@ void traverse_kernel(
     // its opening threshold, in lane 8j + s; lanes of particle children and
     // lanes beyond the batch's children are not used
     unsigned ge_lo = 0u, ge_hi = 0u;
-    int len[W] = {};  // own lists: entries in each (uniform over the workgroup)
+    int len[LISTS] = {};  // own lists: entries in each (uniform over the workgroup)
 
     // Own lists: entry `at` of this wavefront's, and the evaluation of the whole
     // rounds [from, to).
@@ -1457,8 +1460,8 @@ void traverse_kernel(
         if constexpr (OWN) {
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_s_setprio(0);
-            flush_list<LAW, EVAL, 1>(lsrc[wave] + from, lk[wave] + from, lmask[wave] + from, to - from, emine, eslot, mx,
-                                     my, mz, soft, sx, sy, sz, cx, cy, cz);
+            flush_list<LAW, kRound / 4, 1>(lsrc[half] + from, lk[half] + from, lmask[half] + from, to - from, emine,
+                                           eslot, mx, my, mz, soft, sx, sy, sz, cx, cy, cz);
             __builtin_amdgcn_s_setprio(1);
             __builtin_amdgcn_wave_barrier();
             lane_total += lane_count;
@@ -1474,10 +1477,10 @@ void traverse_kernel(
                 float k;
                 core::stage_factored<LAW>(make_float4(src.x, src.y, src.z, core::mass_factor<LAW>(src.w, A.sc)), A.sc,
                                           p, k);
-                put(wave, kCapL + lane, p, k, m);
-                lane_count += __popc(m);
+                put(half, kCapL + share_of * kRound + lane, p, k, m);
+                if (share_of == 0) lane_count += __popc(m);
             }
-            evaluate(kCapL, kCapL + kRound);
+            evaluate(kCapL + share_of * kRound, kCapL + (share_of + 1) * kRound);
         }
     };
 
@@ -1528,7 +1531,7 @@ void traverse_kernel(
         const unsigned long long mask = (static_cast<unsigned long long>(hi32) << 32) | lo32;
         const int f = node_first[node], l = node_last[node];
         if constexpr (OWN) {  // every wavefront for its own particles
-            const unsigned m = static_cast<unsigned>(mask >> (wave * P)) & kOwn;
+            const unsigned m = static_cast<unsigned>(mask >> (half * P)) & kOwn;
             for (int q0 = f; q0 <= l; q0 += kRound) {
                 const int q = q0 + lane, o = q - own_base;
                 const unsigned not_self = o >= 0 && o < P ? ~(1u << o) : ~0u;
@@ -1577,7 +1580,7 @@ void traverse_kernel(
         const float r2 = (dx * dx + dy * dy) + dz * dz;
         const unsigned long long am = __builtin_amdgcn_ballot_w64(!(r2 < A.thr[root_level])) & all;
         if constexpr (OWN) {
-            if (am) round_alone(c, lane == 0 ? static_cast<unsigned>(am >> (wave * P)) & kOwn : 0u);
+            if (am) round_alone(c, lane == 0 ? static_cast<unsigned>(am >> (half * P)) & kOwn : 0u);
             if (am && wave == 0) ++entries;
         } else {
             if (am && wave == 0) append(c, am);
@@ -1758,13 +1761,13 @@ void traverse_kernel(
         const bool wl = child && am != 0ull;
         const unsigned long long has_l = __builtin_amdgcn_ballot_w64(am != 0ull) & children;
         // own lists: the child's mask in each, and which children have one
-        unsigned long long has_part[W];
+        unsigned long long has_part[LISTS];
         if constexpr (OWN) {
             entries += static_cast<unsigned long long>(__popcll(has_l));
             if (wl) lane_count += __popcll(am);
             unsigned counts = 0u;
 #pragma unroll
-            for (int q = 0; q < W; ++q) {
+            for (int q = 0; q < LISTS; ++q) {
                 has_part[q] = __builtin_amdgcn_ballot_w64((static_cast<unsigned>(am >> (q * P)) & kOwn) != 0u) & children;
                 counts |= static_cast<unsigned>(__popcll(has_part[q])) << (16 * q);
             }
@@ -1837,7 +1840,7 @@ void traverse_kernel(
             float k;
             core::stage_factored<LAW>(vsrc, A.sc, p, k);
 #pragma unroll
-            for (int q = 0; q < W; ++q) {
+            for (int q = 0; q < LISTS; ++q) {
                 const unsigned long long has = has_part[q];
                 const int at = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
                     static_cast<unsigned>(has >> 32),
@@ -1849,10 +1852,10 @@ void traverse_kernel(
             __syncthreads();
             int left = 0, full = 0;
 #pragma unroll
-            for (int q = 0; q < W; ++q)
+            for (int q = 0; q < LISTS; ++q)
                 if (len[q] >= kOwnFlush) {
                     const int l = len[q] & (kRound - 1);  // stay, at the list's start
-                    if (q == wave) left = l, full = len[q];
+                    if (q == half) left = l, full = len[q];
                     len[q] = l;
                 }
             if (left < full) evaluate(left, full);
@@ -1862,12 +1865,10 @@ void traverse_kernel(
     }
     if (overflowed && lane == 0) atomicOr(A.overflow, 1u);
     if constexpr (OWN) {
-        int rest = 0;
-#pragma unroll
-        for (int q = 0; q < W; ++q)
-            if (q == wave) rest = len[q];
+        const int rest = half == 0 ? len[0] : len[1];
         const int whole = (rest + kRound - 1) & ~(kRound - 1);
-        if (rest + lane < whole) put(wave, rest + lane, make_float4(0.f, 0.f, 0.f, 0.f), 0.f, 0u);
+        if (share_of == 0 && rest + lane < whole) put(half, rest + lane, make_float4(0.f, 0.f, 0.f, 0.f), 0.f, 0u);
+        if constexpr (W > 2) __syncthreads();
         if (whole) evaluate(0, whole);
         lane_total += lane_count;
     } else {
@@ -1884,6 +1885,23 @@ void traverse_kernel(
             const float qx = __shfl_xor(cx, off), qy = __shfl_xor(cy, off), qz = __shfl_xor(cz, off);
             kahan_add(sx, cx, ox), kahan_add(sy, cy, oy), kahan_add(sz, cz, oz);
             kahan_add(sx, cx, -qx), kahan_add(sy, cy, -qy), kahan_add(sz, cz, -qz);
+        }
+    }
+    if constexpr (OWN && W > 2) {
+        // the sums of the wavefronts of one list, through it
+        static_assert(W == 4, "two wavefronts to a list");
+        float* out = reinterpret_cast<float*>(lsrc[half]);
+        static_assert(sizeof(lsrc[0]) >= 6 * P * sizeof(float), "a wavefront's sums fit a list");
+        __syncthreads();  // both have evaluated it
+        if (share_of == 1 && lane < P) {
+            out[lane] = sx, out[P + lane] = sy, out[2 * P + lane] = sz;
+            out[3 * P + lane] = cx, out[4 * P + lane] = cy, out[5 * P + lane] = cz;
+        }
+        __syncthreads();
+        if (share_of == 0 && lane < P) {
+            kahan_add(sx, cx, out[lane]), kahan_add(sy, cy, out[P + lane]), kahan_add(sz, cz, out[2 * P + lane]);
+            kahan_add(sx, cx, -out[3 * P + lane]), kahan_add(sy, cy, -out[4 * P + lane]);
+            kahan_add(sz, cz, -out[5 * P + lane]);
         }
     }
     if constexpr (W > 1 && !OWN) {
@@ -1906,7 +1924,7 @@ void traverse_kernel(
         }
     }
     const int to = OWN ? own_base + lane : t;
-    if (OWN ? lane < P && to < A.n : wave == 0 && valid && slot == 0) {
+    if (OWN ? share_of == 0 && lane < P && to < A.n : wave == 0 && valid && slot == 0) {
         const unsigned p = A.order[to];
         // back from scaled units (a power of two: exact)
         const float ax = sx * A.sc.out, ay = sy * A.sc.out, az = sz * A.sc.out;
@@ -2019,29 +2037,35 @@ inline int mass_rows(int n) {
 // One wavefront after another waits for its cells, decides, and waits again, so
 // a system with few groups is bound by the longest walk: several wavefronts to a
 // group shorten it, and more of them the fewer groups there are.  Small groups
-// make more and shorter walks, but more in all.  Force pass, us (64x2 with a list
-// per half group):
-//                                 16x8   32x8   32x4   64x8   64x4   64x2   64x1
-//   Plummer, theta 0.6:   4,000     30     36     47     47     74
-//                         8,192     38     39     52     53     80
-//                        16,384     63     50     63     60     94
-//                        32,768    106     83     81     83    104    165    293
-//                        65,536           142    125    134    131    185    331
-//                       131,072                  192    226    193    205    333
-//                       393,216                                475    461
-//   encounter, 0.5:     262,144                  354    379    339           556
-//                       300,000                                373    398
-//                       524,288                  700    715    620    629    862
-//              0.6:   1,048,576                               988    825    979
-//              0.5:   2,097,152                 2954   3133   2557   2334   2573
-//              0.5:   4,194,304                                      5099   5466
-//              0.8:   4,194,304                 3324   3896   2743   2212   2244
-//              2.0:   4,194,304                                       880    866
-//              0.7:   8,388,608                                      5620   5837
-//   Plummer,   0.5:  16,777,216                                     27142  28379
-//              1.0:  16,777,216                                      8144   7989
+// make more and shorter walks, but more in all.  Force pass, us (64x4 and 64x2 with
+// a list per half group; in brackets with one for the group):
+//                                 16x8   32x8   32x4   64x8        64x4         64x2   64x1
+//   Plummer, theta 0.6:   4,000     30     36     47     47        (74)
+//                         8,192     38     39     52     53        (80)
+//                        16,384     63     50     63     60        (94)
+//                        32,768    106     83     81     83    97 (104)   165 (162)     293
+//                        65,536           142    124    134   117 (131)         185     331
+//                        98,304                  157          146
+//                       131,072                  194    226   195 (210)   205 (222)     333
+//                       163,840                  235          226
+//                       393,216                                     (475)         461
+//   encounter, 0.5:      65,536                  116          127
+//                        98,304                  152          134
+//                       200,003                               267 (275)
+//                       262,144                  354    379         (339)               556
+//                       393,216                               503 (517)
+//                       524,288                  700    715   614 (634)   634 (676)     862
+//                       786,432                               920 (931)         850
+//              0.6:   1,048,576                                     (988)   825 (891)   979
+//              0.5:   2,097,152                 2954   3133        (2557) 2334 (2495)  2573
+//                     4,194,304                                           5099 (5529)  5466
+//              0.8:   4,194,304                 3324   3896        (2743) 2212 (2439)  2244
+//              2.0:   4,194,304                                                   880   866
+//              0.7:   8,388,608                                                  5620  5837
+//   Plummer,   0.5:  16,777,216                                                 27142 28379
+//              1.0:  16,777,216                                                  8144  7989
 // (One wavefront to a group of 8, 16 or 32: 53 at 4,000, 138 at 32,768, 234 at
-// 131,072, 309 at 200,003, where 64x4 takes 264.)
+// 131,072, 309 at 200,003.)
 struct TravShape {
     int group, waves;
 };
@@ -2049,8 +2073,8 @@ struct TravShape {
 inline TravShape trav_shape(int n) {
     if (n <= 12288) return {16, 8};
     if (n <= 24576) return {32, 8};
-    if (n <= 163840) return {32, 4};
-    if (n <= 393216) return {64, 4};
+    if (n <= 65536) return {32, 4};
+    if (n <= 524288) return {64, 4};
     if (n <= 8388608) return {64, 2};
     return {64, 1};
 }

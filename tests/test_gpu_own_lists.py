@@ -1,5 +1,5 @@
-"""Walks of two wavefronts with a list each for half of the group: both ends of
-their range of sizes, a last group of one particle, both laws, and coincident
+"""Walks of four or two wavefronts with a list for each half of the group: the ends
+of their ranges of sizes, a last group of one particle, both laws, and coincident
 particles.
 
 Bounds as for the other shapes of the walk: interaction counts against the
@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
 SOFT = 4e-4
 
 
-@pytest.mark.parametrize("n,theta", [(393216, 0.9), (393217, 0.9), (400003, 0.7), (600000, 1.0), (3000001, 2.0)])
+@pytest.mark.parametrize("n,theta", [(65536, 0.6), (65537, 0.6), (200003, 0.6), (393216, 0.9), (393217, 0.9),
+                                     (400003, 0.7), (524288, 0.9), (524289, 0.9), (600000, 1.0), (3000001, 2.0)])
 def test_half_lists_against_the_octree(gpu, oracle, n, theta):
     pu = gpu
     pos, _, mass = pu.ic_plummer(n, 0x5EED0700 + n)
@@ -35,11 +36,12 @@ def test_half_lists_against_the_octree(gpu, oracle, n, theta):
     assert np.count_nonzero(rel_err_rows(a, F / mass[:, None]) >= 1e-5) <= 1e-3 * n
 
 
-@pytest.mark.parametrize("points,law", [(40000, "R"), (40000, "P"), (393216, "R"), (393216, "P")])
-def test_half_lists_at_theta_zero(gpu, points, law):
-    """Buckets of coincident particles with 40,000 points, every pair counted."""
+@pytest.mark.parametrize("n,points,law", [(65537, 7000, "R"), (65537, 65536, "P"), (70000, 3, "R"),
+                                          (393217, 40000, "R"), (393217, 40000, "P"), (393217, 393216, "R"),
+                                          (524289, 50000, "P"), (524289, 524288, "R")])
+def test_half_lists_at_theta_zero(gpu, n, points, law):
+    """Every pair counted; with fewer points than particles, buckets."""
     pu = gpu
-    n = 393217
     rng = np.random.default_rng(points)
     sites = rng.normal(size=(points, 3))
     which = rng.integers(0, points, n - 1) if points < n - 1 else np.arange(points)
