@@ -30,7 +30,6 @@
 #include <cstring>
 #include <map>
 #include <new>
-#include <tuple>
 #include <vector>
 
 #include "common.hpp"
@@ -319,13 +318,33 @@ struct nbody_batch {
     nbody_batch_tuning tuning{1, 256, 8, {0, 0, 0, 0, 0}, 0.0};
 
     bool use_graph = true;
+    // What a captured graph's launches hold besides their (steps, dt, launch
+    // shape): the buffers, the number of groups and whether the one-sided kernel
+    // is among them.  Everything else they read from the device.
+    struct Held {
+        const void *items = nullptr, *sys = nullptr, *tasks = nullptr, *sums = nullptr, *groups = nullptr,
+                   *rows = nullptr, *counters = nullptr;
+        int n_groups = 0;
+        bool one_sided = false;
+        bool operator==(const Held& o) const {
+            return items == o.items && sys == o.sys && tasks == o.tasks && sums == o.sums && groups == o.groups &&
+                   rows == o.rows && counters == o.counters && n_groups == o.n_groups && one_sided == o.one_sided;
+        }
+    };
+    Held held() const {
+        return Held{d_items, d_sys, d_tasks, d_sums, d_groups, d_rows, d_counters, n_groups, n_items > 0};
+    }
+
     // One captured graph per position-buffer parity (a step of an odd number
-    // of steps flips it), each for one (steps, dt, launch shape).
+    // of steps flips it), each for one (steps, dt, launch shape).  A graph is
+    // replayed only where it would be captured the same again, whichever call
+    // laid the items out anew since.
     struct Graph {
         hipGraphExec_t exec = nullptr;
         int steps = -1;
         float dt = 0.f;
         int k = 0, block = 0, wg = 0;
+        Held held;
     };
     Graph graph[2];
 
@@ -493,7 +512,6 @@ nbody_status rebuild_items(nbody_batch* b) {
             NB_HIP(hipMemcpyAsync(*dev, host.data(), host.size() * elem, hipMemcpyHostToDevice, b->stream));
         return NBODY_OK;
     };
-    // The graph holds these pointers: a reallocation invalidates it.
     NB_TRY(upload(&b->d_items, b->items_cap, items));
     NB_TRY(upload(&b->d_sys, b->sys_cap, descs));
     NB_TRY(upload(&b->d_tasks, b->tasks_cap, tasks));
@@ -764,19 +782,11 @@ nbody_status nbody_batch_step(nbody_batch* b, float dt, int32_t nsteps) {
     b->last_interactions = 0;
     b->timed = false;
     if (nsteps == 0) return NBODY_OK;
-    // What a captured graph holds besides its own (steps, dt, launch shape).
-    const auto held = [b] {
-        return std::make_tuple(b->d_items, b->d_sys, b->d_tasks, b->d_sums, b->d_groups, b->d_rows, b->n_groups,
-                               b->n_items > 0);
-    };
-    const auto before = held();
     NB_TRY(rebuild_items(b));
-    if (held() != before) drop_graph(b);
     if (b->n_items == 0 && b->n_tasks == 0) return NBODY_OK;
     const int counters = counters_per_step(b) * nsteps;
     if (counters > b->counters_cap) {
-        drop_graph(b);
-        NB_HIP(hipStreamSynchronize(b->stream));  // plain launches may still use the counters
+        NB_HIP(hipStreamSynchronize(b->stream));  // launches in flight may still use the counters
         if (b->d_counters) (void)hipFree(b->d_counters);
         b->d_counters = nullptr;
         b->counters_cap = 0;
@@ -787,7 +797,7 @@ nbody_status nbody_batch_step(nbody_batch* b, float dt, int32_t nsteps) {
     if (b->use_graph) {
         auto& G = b->graph[b->cur];
         const bool reuse = G.exec && G.steps == nsteps && G.dt == dt && G.k == b->tuning.i_per_lane &&
-                           G.block == b->tuning.block && G.wg == b->tuning.wg_per_cu;
+                           G.block == b->tuning.block && G.wg == b->tuning.wg_per_cu && G.held == b->held();
         if (!reuse) {
             if (G.exec) {
                 // its last launch may still be queued on the stream
@@ -812,6 +822,7 @@ nbody_status nbody_batch_step(nbody_batch* b, float dt, int32_t nsteps) {
             G.k = b->tuning.i_per_lane;
             G.block = b->tuning.block;
             G.wg = b->tuning.wg_per_cu;
+            G.held = b->held();
         }
         NB_HIP(hipGraphLaunch(G.exec, b->stream));
     } else {
