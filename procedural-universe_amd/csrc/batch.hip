@@ -219,6 +219,7 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(6))) void
 }
 
 // Adds the rows of one group's systems, 64 particles a workgroup at a time.
+template <int LAW>
 __global__ __launch_bounds__(256) void batch_sum_kernel(BatchLaunch B, int group) {
     __shared__ core::SliceSums sums;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -231,7 +232,9 @@ __global__ __launch_bounds__(256) void batch_sum_kernel(BatchLaunch B, int group
         core::sum_rows(B.rows + D.rows, D.sym, D.n_pad, i, sums, wave, lane, s);
         if (wave == 0 && i < D.n) {
             const float out = D.gm_equal > 0.f ? D.gm_equal * D.sc.out : D.sc.out;
-            batch_kick(B, D.off + i, B.pos_in[D.off + i], s[0] * out, s[1] * out, s[2] * out);
+            const float4 x = B.pos_in[D.off + i];
+            core::sums_of_a_lost_particle<LAW>(x, D.sc, s);
+            batch_kick(B, D.off + i, x, s[0] * out, s[1] * out, s[2] * out);
         }
         __syncthreads();  // the sums are read before the next item's
     }
@@ -569,13 +572,14 @@ nbody_status enqueue_steps(nbody_batch* b, float dt, int nsteps) {
     hipLaunchKernelGGL(fill_u32_kernel, dim3((counters + 255) / 256), dim3(256), 0, b->stream, b->d_counters, counters, 0u);
     const dim3 grid(static_cast<unsigned>(b->tuning.wg_per_cu * b->cus));
     const auto sym = b->cfg.law == NBODY_LAW_R ? batch_sym_kernel<NBODY_LAW_R> : batch_sym_kernel<NBODY_LAW_P>;
+    const auto sum = b->cfg.law == NBODY_LAW_R ? batch_sum_kernel<NBODY_LAW_R> : batch_sum_kernel<NBODY_LAW_P>;
     int parity = b->cur;
     for (int s = 0; s < nsteps; ++s) {
         const BatchLaunch L = launch_for(b, parity, dt);
         unsigned* counter = b->d_counters + static_cast<size_t>(s) * per;
         for (int g = 0; g < b->n_groups; ++g) {
             hipLaunchKernelGGL(sym, dim3(6 * b->cus), dim3(kTile), 0, b->stream, L, g, counter + 1 + g);
-            hipLaunchKernelGGL(batch_sum_kernel, dim3(8 * b->cus), dim3(256), 0, b->stream, L, g);
+            hipLaunchKernelGGL(sum, dim3(8 * b->cus), dim3(256), 0, b->stream, L, g);
         }
         if (b->n_items > 0) hipLaunchKernelGGL(fn, grid, dim3(b->tuning.block), 0, b->stream, L, counter);
         parity ^= 1;

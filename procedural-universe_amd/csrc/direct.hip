@@ -147,15 +147,24 @@ __global__ __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(8
         const float4 p = j < L.n_pad ? L.src[j] : make_float4(0.f, 0.f, 0.f, 0.f);
         return make_float4(p.x * L.sc.inv_len, p.y * L.sc.inv_len, p.z * L.sc.inv_len, p.w * inv_c);
     };
+    // a source: under law R a massless one far away, as core::stage_source does
+    // (it pulls nothing, even from a position that is not finite)
+    auto source = [&](int j) {
+        float4 q = scaled(j);
+        if constexpr (LAW == NBODY_LAW_R) {
+            if (!(q.w > 0.f)) q.x = q.y = q.z = 0x1p100f;
+        }
+        return q;
+    };
     const float4 me = scaled(min(i, L.n_pad - 1));
     float s[3] = {0.f, 0.f, 0.f}, c[3] = {0.f, 0.f, 0.f};
-    tile[0][tid] = scaled(tid);
+    tile[0][tid] = source(tid);
     __syncthreads();
     int buf = 0;
     for (int jt = 0; jt < L.n_pad; jt += kSmallThreads) {
         const bool more = jt + kSmallThreads < L.n_pad;
         float4 next;
-        if (more) next = scaled(jt + kSmallThreads + tid);
+        if (more) next = source(jt + kSmallThreads + tid);
         float ax = 0.f, ay = 0.f, az = 0.f;
 #pragma unroll 2
         for (int g = 0; g < PER; g += 4) {

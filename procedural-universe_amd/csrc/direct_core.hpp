@@ -142,6 +142,29 @@ __device__ __forceinline__ void stage_factored(const float4 s, const DirectScale
     }
 }
 
+// A massless particle of law R pulls nothing, wherever it is: where its position in
+// scaled units q is not finite, the kernels whose streamed records are targets
+// too place it at (2^100, 2^100, 2^100), from where its pairs are exactly 0
+// (direct_core's own staging does so with every massless source).
+__device__ __forceinline__ bool finite3(const float4 q) {
+    return q.x * 0.f + q.y * 0.f + q.z * 0.f == 0.f;
+}
+
+// Its own acceleration is then what the pair arithmetic gives from where it is: 0
+// along a finite coordinate and NaN along an infinite one, NaN if any is NaN.
+// x: the particle's record (any mass); s: its sums.
+template <int LAW>
+__device__ __forceinline__ void sums_of_a_lost_particle(const float4 x, const DirectScale& sc, float (&s)[3]) {
+    if constexpr (LAW == NBODY_LAW_R) {
+        const float4 q = make_float4(x.x * sc.inv_len, x.y * sc.inv_len, x.z * sc.inv_len, 0.f);
+        if (x.w > 0.f || finite3(q)) return;
+        const float f = __builtin_amdgcn_rsqf(q.x * q.x + q.y * q.y + q.z * q.z);
+        s[0] = q.x * f;
+        s[1] = q.y * f;
+        s[2] = q.z * f;
+    }
+}
+
 // The staged record of a source (x, y, z, G m) of this system.
 template <int LAW>
 __device__ __forceinline__ void stage_source(const float4 s, const DirectScale& sc, float4& p, float& k) {

@@ -72,6 +72,7 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(6))) void
 
 // Adds each particle's rows, 64 particles a workgroup, scales the sums back and
 // kicks and drifts (kick != 0) or stores the acceleration only.
+template <int LAW>
 __global__ __launch_bounds__(256) void sym_reduce_kernel(DirectLaunch L, SymPlan P, int kick) {
     __shared__ core::SliceSums sums;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -79,12 +80,14 @@ __global__ __launch_bounds__(256) void sym_reduce_kernel(DirectLaunch L, SymPlan
     float s[3];
     core::sum_rows(reinterpret_cast<const float*>(L.part), P, L.n_pad, i, sums, wave, lane, s);
     if (wave != 0 || i >= L.n) return;
+    float4 x = L.src[i];
+    core::sums_of_a_lost_particle<LAW>(x, L.sc, s);
     // equal masses: the rows are sums without the mass, in scaled units
     const float out = L.gm_equal > 0.f ? L.gm_equal * L.sc.out : L.sc.out;
     const float ax = s[0] * out, ay = s[1] * out, az = s[2] * out;
     L.acc[i] = make_float4(ax, ay, az, 0.f);
     if (!kick) return;
-    float4 v = L.vel[i], x = L.src[i];
+    float4 v = L.vel[i];
     v.x = __builtin_fmaf(ax, L.dt, v.x);
     v.y = __builtin_fmaf(ay, L.dt, v.y);
     v.z = __builtin_fmaf(az, L.dt, v.z);
@@ -133,7 +136,7 @@ hipError_t sym_step(const DirectLaunch& L, const SymPlan& P, bool kick, hipStrea
     hipLaunchKernelGGL(fn, grid, dim3(kTile), 0, stream, A);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (ev_e && (e = hipEventRecord(ev_e, stream)) != hipSuccess) return e;
-    hipLaunchKernelGGL(sym_reduce_kernel, dim3(L.n_pad / 64), dim3(256), 0, stream, L, P, kick ? 1 : 0);
+    hipLaunchKernelGGL((r ? sym_reduce_kernel<NBODY_LAW_R> : sym_reduce_kernel<NBODY_LAW_P>), dim3(L.n_pad / 64), dim3(256), 0, stream, L, P, kick ? 1 : 0);
     return hipGetLastError();
 }
 

@@ -36,13 +36,16 @@ struct SymArgs {
 // A particle in scaled units: (x', y', z', G m / c).  With EQ the masses do not
 // enter the pairs, so a massless one (the padding) is placed at
 // (2^100, 2^100, 2^100): its squared distances are +inf and their reciprocal
-// square roots 0.
+// square roots 0; so is, under law R, a massless particle that has no finite
+// position (sums_of_a_lost_particle).
 template <int LAW, bool EQ>
 __device__ __forceinline__ float4 scaled(const float4 p, const DirectScale& sc) {
     float4 q = make_float4(p.x * sc.inv_len, p.y * sc.inv_len, p.z * sc.inv_len,
                            p.w * (LAW == NBODY_LAW_R ? 1.0f / sc.mass_k : sc.mass_k));
     if constexpr (EQ) {
         if (!(p.w > 0.f)) q.x = q.y = q.z = 0x1p100f;
+    } else if constexpr (LAW == NBODY_LAW_R) {
+        if (!(p.w > 0.f) && !finite3(q)) q.x = q.y = q.z = 0x1p100f;
     }
     return q;
 }
