@@ -210,13 +210,15 @@ void set_scale(nbody_sim* s, double extent) {
     s->dscale = direct_scale_for(s->cfg.law, s->cfg.softening, extent, s->max_gm);
 }
 
-// Whether every particle has the same positive G m (in FP32, as the records
-// hold it); mass: n FP64 masses.
+// Whether every particle has the same positive G m and whether one has none (in
+// FP32, as the records hold it); mass: n FP64 masses.
 void set_equal(nbody_sim* s, const std::vector<double>& mass) {
     const float first = s->n ? static_cast<float>(s->cfg.G * mass[0]) : 0.f;
     bool equal = first > 0.f && std::isfinite(first);
     for (size_t i = 1; i < s->n && equal; ++i) equal = static_cast<float>(s->cfg.G * mass[i]) == first;
     s->gm_equal = equal ? first : 0.f;
+    s->massless = std::any_of(mass.begin(), mass.begin() + s->n,
+                              [&](double m) { return !(static_cast<float>(s->cfg.G * m) > 0.f); });
 }
 
 // Masses must be finite and >= 0 (the direct sum folds G m into a square).
@@ -305,6 +307,7 @@ DirectLaunch launch_for(nbody_sim* s, float dt) {
     L.law = s->cfg.law;
     L.sc = s->dscale;
     L.gm_equal = s->gm_equal * (s->cfg.law == NBODY_LAW_R ? 1.0f / s->dscale.mass_k : s->dscale.mass_k);
+    L.massless = s->massless;
     L.dt = dt;
     L.dts = static_cast<float>(static_cast<double>(dt) / s->cfg.scale);
     return L;

@@ -54,6 +54,7 @@ struct DirectLaunch {
     int law;            // nbody_law
     DirectScale sc;     // the system's scaled units
     float gm_equal;     // sym_step: every real particle's G m in scaled units if all are equal, else 0
+    bool massless;      // small_step: some real particle has no mass
     float dt;           // kick step
     float dts;          // drift factor dt / scale
 };
