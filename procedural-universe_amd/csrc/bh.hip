@@ -1867,6 +1867,9 @@ void traverse_kernel(
     if constexpr (OWN) {
         const int rest = half == 0 ? len[0] : len[1];
         const int whole = (rest + kRound - 1) & ~(kRound - 1);
+        // the last step's evaluation, which began at the same entry, is over in
+        // every wavefront of the list before its end is padded
+        if constexpr (W > 2) __syncthreads();
         if (share_of == 0 && rest + lane < whole) put(half, rest + lane, make_float4(0.f, 0.f, 0.f, 0.f), 0.f, 0u);
         if constexpr (W > 2) __syncthreads();
         if (whole) evaluate(0, whole);
