@@ -175,7 +175,7 @@ nbody_status prepare_state(nbody_sim* s, size_t n) {
     if (s->sym.nsb > 0) {
         const size_t need = sym_part_records(s->sym, static_cast<int>(n_pad));
         if (need <= s->part_elems) return NBODY_OK;
-        // Its rows take up to 2 KB per particle: on a device too full for them
+        // Its rows take up to 3.1 KB per particle: on a device too full for them
         // the one-sided sum runs instead.
         const nbody_status st = grow_part(s, need);
         if (st != NBODY_ERR_OUT_OF_MEMORY) return st;
@@ -210,13 +210,10 @@ void set_scale(nbody_sim* s, double extent) {
     s->dscale = direct_scale_for(s->cfg.law, s->cfg.softening, extent, s->max_gm);
 }
 
-// Whether every particle has the same positive G m and whether one has none (in
-// FP32, as the records hold it); mass: n FP64 masses.
-void set_equal(nbody_sim* s, const std::vector<double>& mass) {
-    const float first = s->n ? static_cast<float>(s->cfg.G * mass[0]) : 0.f;
-    bool equal = first > 0.f && std::isfinite(first);
-    for (size_t i = 1; i < s->n && equal; ++i) equal = static_cast<float>(s->cfg.G * mass[i]) == first;
-    s->gm_equal = equal ? first : 0.f;
+// What the direct sum chooses by the masses (n in FP64): whether every particle
+// has the same positive G m and whether one has none.
+void set_masses(nbody_sim* s, const std::vector<double>& mass) {
+    s->gm_equal = equal_gm(s->cfg.G, mass.data(), s->n);
     s->massless = std::any_of(mass.begin(), mass.begin() + s->n,
                               [&](double m) { return !(static_cast<float>(s->cfg.G * m) > 0.f); });
 }
@@ -270,7 +267,7 @@ nbody_status upload_state(nbody_sim* s, const std::vector<float4>& pos, const st
         hg[i] = s->cfg.G * mass[i];
         s->max_gm = std::max(s->max_gm, std::fabs(hg[i]));
     }
-    set_equal(s, mass);
+    set_masses(s, mass);
     set_scale(s, extent_of(pos.data(), n));
     NB_HIP(hipMemcpyAsync(s->pos[0], hp.data(), n_pad * sizeof(float4), hipMemcpyHostToDevice, s->stream));
     NB_HIP(hipMemcpyAsync(s->pos[1], hp.data(), n_pad * sizeof(float4), hipMemcpyHostToDevice, s->stream));
@@ -306,7 +303,8 @@ DirectLaunch launch_for(nbody_sim* s, float dt) {
     L.n_pad = static_cast<int>(s->n_pad);
     L.law = s->cfg.law;
     L.sc = s->dscale;
-    L.gm_equal = s->gm_equal * (s->cfg.law == NBODY_LAW_R ? 1.0f / s->dscale.mass_k : s->dscale.mass_k);
+    L.equal = s->gm_equal > 0;
+    L.sums_out = sym_out(s->cfg.law, s->dscale, s->gm_equal);
     L.massless = s->massless;
     L.dt = dt;
     L.dts = static_cast<float>(static_cast<double>(dt) / s->cfg.scale);
@@ -476,7 +474,7 @@ nbody_status nbody_init_plummer(nbody_sim* s, uint64_t seed, size_t n, double a,
     const double m = total_mass / static_cast<double>(n);
     s->mass_host.assign(n, m);
     s->max_gm = std::fabs(s->cfg.G * m);
-    set_equal(s, s->mass_host);
+    set_masses(s, s->mass_host);
     set_scale(s, 40.0 * a);  // radii are cut at 20 a
     s->initialised = true;
     s->acc_valid = false;
@@ -553,7 +551,7 @@ nbody_status nbody_init_seeded(nbody_sim* s, int32_t seeder, uint64_t seed, size
     NB_HIP(hipStreamSynchronize(s->stream));
     s->max_gm = 0.0;
     for (double m : s->mass_host) s->max_gm = std::max(s->max_gm, std::fabs(s->cfg.G * m));
-    set_equal(s, s->mass_host);
+    set_masses(s, s->mass_host);
     set_scale(s, extent_of(pos_host.data(), n));
     s->initialised = true;
     s->acc_valid = false;

@@ -12,7 +12,7 @@
 // Systems of more than 1,024 particles take the sum over unordered pairs
 // (direct_sym.hip) instead: a persistent kernel drains their tasks, then one adds
 // their rows of partial sums and kicks.  The rows lie in a buffer of at most
-// kRowsBytes; where a batch's systems need more, they are taken in groups, one
+// kRowsRecords; where a batch's systems need more, they are taken in groups, one
 // group's two kernels after the other's.  The smaller systems' items are drained
 // behind the last group's tasks; only a batch without any pairs has a kernel of
 // its own for them.  Which way a system takes, and its tasks, depend on its size
@@ -48,10 +48,11 @@ struct SysDesc {
     int off;         // first record in the arena
     int n;           // real particles
     int n_pad;       // padded to kTile
-    float gm_equal;  // every particle's G m in scaled units if all are equal, else 0
+    int equal;       // every particle has the same positive G m
     DirectScale sc;  // the system's scaled units
+    SymOut out;      // its rows' sums back to accelerations
     SymPlan sym;     // nsb > 0: over unordered pairs
-    size_t rows;     // its partial sums in the rows buffer (floats)
+    size_t rows;     // its partial sums in the rows buffer (records)
 };
 
 // A task of the sum over unordered pairs: blocks a and a + d, run h of the
@@ -71,10 +72,10 @@ struct SymGroup {
     int sum0, sum1;
 };
 
-// Partial sums of at most this many bytes in flight (the 512 galaxies of up to
-// 65,536 particles need about 4 GB in all); a system that needs more alone
-// stays with the one-sided sum.
-constexpr size_t kRowsBytes = size_t(1) << 30;
+// Partial sums of at most this many records in flight, 1.33 GiB (the 512 galaxies
+// of up to 65,536 particles need about 5.4 GB in all); a system that needs more
+// alone, from about 247,000 particles on, stays with the one-sided sum.
+constexpr size_t kRowsRecords = (size_t(1) << 30) / 12;
 
 // A one-sided item is n pairs per lane, one after another: the batch waits for
 // its largest item.  A pair task is at most 1,024, so every padded size above
@@ -90,7 +91,7 @@ SymPlan batch_sym_plan(size_t n_pad) {
     p.block = 1024;
     p.nsb = static_cast<int>((n_pad + 1023) / 1024);
     p.split = p.nsb <= 16 ? 4 : 2;
-    if (sym_part_records(p, static_cast<int>(n_pad)) * sizeof(float4) > kRowsBytes) p = SymPlan{};
+    if (sym_part_records(p, static_cast<int>(n_pad)) > kRowsRecords) p = SymPlan{};
     return p;
 }
 
@@ -110,7 +111,7 @@ struct BatchLaunch {
     const SymTask* tasks;
     const SumItem* sums;
     const SymGroup* groups;
-    float* rows;
+    float4* rows;
     float dt;
     float dts;
 };
@@ -177,6 +178,21 @@ __global__ __launch_bounds__(BLOCK) void batch_step_kernel(BatchLaunch B, unsign
     }
 }
 
+// A value that is the same in every lane, in scalar registers (the compiler keeps
+// what it loads through a pointer of its own finding in vector registers, which
+// the pair loop has none to spare of).
+template <class T>
+__device__ __forceinline__ T scalar_copy(const T& v) {
+    static_assert(sizeof(T) % sizeof(int) == 0, "whole registers");
+    int w[sizeof(T) / sizeof(int)];
+    __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+    for (size_t i = 0; i < sizeof(T) / sizeof(int); ++i) w[i] = __builtin_amdgcn_readfirstlane(w[i]);
+    T r;
+    __builtin_memcpy(&r, w, sizeof(T));
+    return r;
+}
+
 // The tasks of one group, largest systems first, from a counter.  Every branch is
 // uniform over the workgroup.  Bound by the pair arithmetic's issue: a step of 96
 // systems of 1,024 to 32,768 particles 2.67 ms (5.6e12 interactions/s), 3.24 ms
@@ -197,8 +213,8 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(6))) void
         const int it = item_sh;
         __syncthreads();
         if (it >= G.task1) break;
-        const SymTask w = B.tasks[it];
-        const SysDesc D = B.sys[w.sys];
+        const SymTask w = scalar_copy(B.tasks[it]);
+        const SysDesc D = scalar_copy(B.sys[w.sys]);
         if (w.d < 0) {
             one_sided_item<LAW, 1, kTile>(B, D, w.a * kTile, S.tiles);
             continue;
@@ -206,13 +222,13 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(6))) void
         const core::SymArgs A{B.pos_in + D.off, B.rows + D.rows, D.n_pad, D.sym, D.sc};
         const int H = D.sym.nsb / 2;
         if (w.d == 0) {
-            if (D.gm_equal > 0.f) core::sym_task<LAW, false, true>(A, S.pairs, w.a, w.a, w.h, w.h, 0);
+            if (D.equal) core::sym_task<LAW, false, true>(A, S.pairs, w.a, w.a, w.h, w.h, 0);
             else core::sym_task<LAW, false, false>(A, S.pairs, w.a, w.a, w.h, w.h, 0);
         } else {
             int b = w.a + w.d;
             if (b >= D.sym.nsb) b -= D.sym.nsb;
             const int rowi = w.d * D.sym.split + w.h, rowj = (H + 1) * D.sym.split + w.d - 1;
-            if (D.gm_equal > 0.f) core::sym_task<LAW, true, true>(A, S.pairs, w.a, b, w.h, rowi, rowj);
+            if (D.equal) core::sym_task<LAW, true, true>(A, S.pairs, w.a, b, w.h, rowi, rowj);
             else core::sym_task<LAW, true, false>(A, S.pairs, w.a, b, w.h, rowi, rowj);
         }
     }
@@ -229,12 +245,11 @@ __global__ __launch_bounds__(256) void batch_sum_kernel(BatchLaunch B, int group
         const SysDesc D = B.sys[w.sys];
         const int i = w.i + lane;
         float s[3];
-        core::sum_rows(B.rows + D.rows, D.sym, D.n_pad, i, sums, wave, lane, s);
+        core::sum_rows(B.rows + D.rows, D.sym, D.n_pad, i, sums, wave, lane, D.out, s);
         if (wave == 0 && i < D.n) {
-            const float out = D.gm_equal > 0.f ? D.gm_equal * D.sc.out : D.sc.out;
             const float4 x = B.pos_in[D.off + i];
             core::sums_of_a_lost_particle<LAW>(x, D.sc, s);
-            batch_kick(B, D.off + i, x, s[0] * out, s[1] * out, s[2] * out);
+            batch_kick(B, D.off + i, x, s[0], s[1], s[2]);
         }
         __syncthreads();  // the sums are read before the next item's
     }
@@ -292,7 +307,7 @@ struct nbody_batch {
         size_t off = 0, n = 0, n_pad = 0;
         DirectScale sc{};
         double max_gm = 0.0;
-        float gm_equal = 0.f;  // FP32 G*m if every particle has the same positive one, else 0
+        double gm_equal = 0.0;  // G*m if every particle has the same positive one in FP32, else 0
     };
     std::vector<Sys> systems;  // index = id = descriptor slot
     std::vector<int> free_ids;
@@ -308,7 +323,7 @@ struct nbody_batch {
     size_t sums_cap = 0;
     SymGroup* d_groups = nullptr;
     size_t groups_cap = 0;
-    float* d_rows = nullptr;
+    float4* d_rows = nullptr;
     size_t rows_cap = 0;
     int n_tasks = 0, n_groups = 0;
     bool no_rows = false;  // the rows buffer could not be allocated
@@ -423,11 +438,6 @@ void arena_free(nbody_batch* b, size_t off, size_t len) {
     }
 }
 
-// Every particle's G m in the pair arithmetic's scaled units if all are equal, else 0.
-float scaled_gm(const nbody_batch* b, const nbody_batch::Sys& y) {
-    return y.gm_equal * (b->cfg.law == NBODY_LAW_R ? 1.0f / y.sc.mass_k : y.sc.mass_k);
-}
-
 // Rebuild the work-item list (largest systems first) and upload it.
 nbody_status rebuild_items(nbody_batch* b) {
     if (!b->items_dirty) return NBODY_OK;
@@ -445,8 +455,8 @@ nbody_status rebuild_items(nbody_batch* b) {
     uint64_t inter = 0;
     for (size_t s = 0; s < b->systems.size(); ++s) {
         const auto& y = b->systems[s];
-        descs[s] = SysDesc{static_cast<int>(y.off), static_cast<int>(y.n), static_cast<int>(y.n_pad), scaled_gm(b, y),
-                           y.sc, {}, 0};
+        descs[s] = SysDesc{static_cast<int>(y.off), static_cast<int>(y.n), static_cast<int>(y.n_pad), y.gm_equal > 0,
+                           y.sc, sym_out(b->cfg.law, y.sc, y.gm_equal), {}, 0};
     }
     // Groups of systems, largest first, whose rows fit the buffer together.
     size_t rows = 0, rows_max = 0;
@@ -475,8 +485,8 @@ nbody_status rebuild_items(nbody_batch* b) {
         inter += static_cast<uint64_t>(y.n) * y.n;
         const SymPlan P = b->no_rows ? SymPlan{} : batch_sym_plan(y.n_pad);
         if (P.nsb > 0) {
-            const size_t need = sym_part_records(P, static_cast<int>(y.n_pad)) * 4;
-            if ((rows + need) * sizeof(float) > kRowsBytes) close_group();
+            const size_t need = sym_part_records(P, static_cast<int>(y.n_pad));
+            if (rows + need > kRowsRecords) close_group();
             descs[s].sym = P;
             descs[s].rows = rows;
             rows += need;
@@ -496,8 +506,8 @@ nbody_status rebuild_items(nbody_batch* b) {
     }
     if (!groups.empty()) groups.back().task1 = static_cast<int>(tasks.size());
     if (rows_max > b->rows_cap) {
-        const nbody_status st = ensure_dev(reinterpret_cast<void**>(&b->d_rows), b->rows_cap, rows_max, sizeof(float),
-                                           b->stream, kRowsBytes / sizeof(float));
+        const nbody_status st = ensure_dev(reinterpret_cast<void**>(&b->d_rows), b->rows_cap, rows_max, sizeof(float4),
+                                           b->stream, kRowsRecords);
         if (st == NBODY_ERR_OUT_OF_MEMORY) {
             // A device too full for the rows: the one-sided sum for every
             // system, from now on.
@@ -667,13 +677,11 @@ nbody_status nbody_batch_add(nbody_batch* b, const float* pos3, const float* vel
     NB_TRY(arena_alloc(b, n_pad, &off));
     std::vector<float4> hp(n_pad, make_float4(0.f, 0.f, 0.f, 0.f)), hv(n_pad, make_float4(0.f, 0.f, 0.f, 0.f));
     double max_gm = 0.0;
-    const float gm0 = static_cast<float>(b->cfg.G * mass[0]);
-    bool equal = gm0 > 0.f && std::isfinite(gm0);
+    const double gm_equal = equal_gm(b->cfg.G, mass, n);
     float lo[3] = {pos3[0], pos3[1], pos3[2]}, hi[3] = {pos3[0], pos3[1], pos3[2]};
     for (size_t i = 0; i < n; ++i) {
         const double gm = b->cfg.G * mass[i];
         max_gm = std::max(max_gm, std::fabs(gm));
-        equal = equal && static_cast<float>(gm) == gm0;
         hp[i] = make_float4(pos3[3 * i], pos3[3 * i + 1], pos3[3 * i + 2], static_cast<float>(gm));
         if (vel3) hv[i] = make_float4(vel3[3 * i], vel3[3 * i + 1], vel3[3 * i + 2], 0.f);
         for (int c = 0; c < 3; ++c) {
@@ -708,7 +716,7 @@ nbody_status nbody_batch_add(nbody_batch* b, const float* pos3, const float* vel
     y.n = n;
     y.n_pad = n_pad;
     y.max_gm = max_gm;
-    y.gm_equal = equal ? gm0 : 0.f;
+    y.gm_equal = gm_equal;
     y.sc = direct_scale_for(b->cfg.law, b->cfg.softening, extent, max_gm);
     b->items_dirty = true;
     *id = slot;
@@ -752,8 +760,8 @@ nbody_status nbody_batch_add_plummer(nbody_batch* b, uint64_t seed, size_t n, do
     y.n = n;
     y.n_pad = n_pad;
     y.max_gm = std::fabs(b->cfg.G * total_mass / static_cast<double>(n));
-    const float gm = static_cast<float>(b->cfg.G * (total_mass / static_cast<double>(n)));
-    y.gm_equal = gm > 0.f && std::isfinite(gm) ? gm : 0.f;
+    const double m = total_mass / static_cast<double>(n);
+    y.gm_equal = equal_gm(b->cfg.G, &m, 1);
     // Plummer radii are cut at 20 a, so the sphere spans at most 40 a
     y.sc = direct_scale_for(b->cfg.law, b->cfg.softening, 40.0 * a, y.max_gm);
     b->items_dirty = true;
@@ -878,8 +886,9 @@ nbody_status nbody_batch_step_sequential(nbody_batch* b, float dt, int32_t nstep
             L.pos_out = b->pos[parity ^ 1] + y.off;
             L.vel = b->vel + y.off;
             L.acc = b->acc + y.off;
-            L.part = P.nsb > 0 ? reinterpret_cast<float4*>(b->d_rows) : b->part;
-            L.gm_equal = scaled_gm(b, y);
+            L.part = P.nsb > 0 ? b->d_rows : b->part;
+            L.equal = y.gm_equal > 0;
+            L.sums_out = sym_out(b->cfg.law, y.sc, y.gm_equal);
             L.n = static_cast<int>(y.n);
             L.n_pad = static_cast<int>(y.n_pad);
             L.law = b->cfg.law;

@@ -55,6 +55,15 @@ __device__ __forceinline__ void kahan_add(float& s, float& c, float x) {
     s = t;
 }
 
+// s + x, and in x what the rounding of it left out, whichever is larger (TwoSum).
+// kahan_add's three subtractions want the sum to be the larger one.
+__device__ __forceinline__ void add_keeping_rest(float& s, float& x) {
+    const float t = s + x;
+    const float z = t - s;
+    x = (s - (t - z)) + (x - z);
+    s = t;
+}
+
 // A uniform value held in a VGPR, so that the arithmetic using it keeps
 // all-VGPR operands (an SGPR operand halves the issue rate).
 __device__ __forceinline__ float in_vgpr(float x) {
@@ -298,7 +307,7 @@ __device__ __forceinline__ void block_forces(SrcTile* tiles, const float4* __res
 // The waves' compensated sums (s, c: Kahan's sum and compensation) of the same
 // 64 targets, added in wave order into wave 0's, compensations included (four
 // sums rounded apart cost a third more error than one).  Every thread of the
-// workgroup must call it; only wave 0 returns the totals, in s.
+// workgroup must call it; only wave 0 returns the totals, s - c.
 template <int WAVES>
 struct WaveSums {
     float s[WAVES - 1][3][64], c[WAVES - 1][3][64];
@@ -320,8 +329,9 @@ __device__ __forceinline__ void add_slices(WaveSums<WAVES>& S, int wave, int lan
         for (int w = 0; w < WAVES - 1; ++w)
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
-                kahan_add(s[a], c[a], S.s[w][a][lane]);
-                kahan_add(s[a], c[a], -S.c[w][a][lane]);
+                float x = S.s[w][a][lane];
+                add_keeping_rest(s[a], x);
+                c[a] += S.c[w][a][lane] - x;
             }
     }
 }

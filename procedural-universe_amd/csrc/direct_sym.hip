@@ -6,9 +6,9 @@
 // sides a law-R pair costs 17 (15 when all masses are equal) and one
 // v_rsq_f32, and 0.75 for moving the streamed sums from lane to lane: 8.9 (7.9)
 // + 0.5 per interaction.  Measured, one step of N = 2^20: one-sided 288 ms
-// (3.8e12 interactions/s), 193 ms (5.7e12) here, 177 ms (6.2e12) with equal
-// masses; N = 65,536: 1.25, 0.79, 0.72 ms; N = 20,011 (law P): 0.151, 0.120,
-// 0.108 ms.  Still bound by issue: 0.389 VALU instructions per SIMD per cycle at
+// (3.8e12 interactions/s), 197 ms (5.6e12) here, 180 ms (6.1e12) with equal
+// masses; N = 65,536: 1.25, 0.81, 0.74 ms; N = 20,011 (law P): 0.151, 0.123,
+// 0.111 ms.  Still bound by issue: 0.389 VALU instructions per SIMD per cycle at
 // N = 2^20 (2.13 GHz under this load), 0.326 one-sided.
 //
 // Layout.  A wavefront holds 256 resident particles, four per lane, with their
@@ -33,9 +33,14 @@
 // other task writes, and a second kernel adds each particle's rows in a fixed
 // order: no atomics, the same bits every run.
 //
-// Summation: FP32 sums of 256 pairs, added over the task (at most about 30
-// of them) and then, compensated, over the tasks.  RMS error against FP64 at
-// N = 2^20: 2.9e-8, one-sided 2.6e-8; at 65,536 3.4e-8 either way.
+// Summation: a resident's FP32 sums of 256 pairs (a streamed particle's of 1,024,
+// four at a time and in four parts) are added with compensation over the task
+// and then over the tasks: what the rounding of a resident's sum leaves out is where
+// its next tile starts, so that it takes no registers, and a row keeps it too.
+// RMS error against FP64, one-sided / here: N = 2^20 2.8e-8 / 2.7e-8 (a disc of unequal
+// masses), 3.1e-8 / 3.1e-8 (a sphere of equal ones), 2^21 2.7e-8 / 2.7e-8, 20,011 5.2e-8 /
+// 4.5e-8; with the tiles' and the rows' sums added plainly 3.2e-8 to 3.3e-8 and 6.3e-8,
+// in 1.6% (equal masses) and 2.2% less time.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -78,13 +83,11 @@ __global__ __launch_bounds__(256) void sym_reduce_kernel(DirectLaunch L, SymPlan
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int i = blockIdx.x * 64 + lane;
     float s[3];
-    core::sum_rows(reinterpret_cast<const float*>(L.part), P, L.n_pad, i, sums, wave, lane, s);
+    core::sum_rows(L.part, P, L.n_pad, i, sums, wave, lane, L.sums_out, s);
     if (wave != 0 || i >= L.n) return;
     float4 x = L.src[i];
     core::sums_of_a_lost_particle<LAW>(x, L.sc, s);
-    // equal masses: the rows are sums without the mass, in scaled units
-    const float out = L.gm_equal > 0.f ? L.gm_equal * L.sc.out : L.sc.out;
-    const float ax = s[0] * out, ay = s[1] * out, az = s[2] * out;
+    const float ax = s[0], ay = s[1], az = s[2];
     L.acc[i] = make_float4(ax, ay, az, 0.f);
     if (!kick) return;
     float4 v = L.vel[i];
@@ -105,8 +108,8 @@ SymPlan sym_plan(int n_pad) {
     // 0.058 ms against 0.059 one-sided; 16,384: 0.081 against 0.093).
     SymPlan p{};
     if (n_pad < 16384) return p;
-    // About 192 blocks: more give more rows of partial sums (12 bytes per
-    // particle and block, 2.1 GB at 2^20 with 171 blocks, 3.2 GB and 1% less
+    // About 192 blocks: more give more rows of partial sums (16 bytes per
+    // particle and block, 2.9 GB at 2^20 with 171 blocks, 4.3 GB and 1% less
     // time with 256), fewer leave a longer tail (128: 1% more time).
     constexpr int kStep = core::kRes * core::kWaves;
     p.block = ((n_pad + 191) / 192 + kStep - 1) / kStep * kStep;
@@ -120,17 +123,17 @@ SymPlan sym_plan(int n_pad) {
 
 size_t sym_part_records(const SymPlan& p, int n_pad) {
     const size_t H = p.nsb / 2;
-    return (((H + 1) * p.split + H) * 3 * static_cast<size_t>(n_pad) + 3) / 4;
+    return ((H + 1) * p.split + H) * static_cast<size_t>(n_pad);
 }
 
 hipError_t sym_step(const DirectLaunch& L, const SymPlan& P, bool kick, hipStream_t stream, hipEvent_t ev_b,
                     hipEvent_t ev_e) {
-    const core::SymArgs A{L.src, reinterpret_cast<float*>(L.part), L.n_pad, P, L.sc};
+    const core::SymArgs A{L.src, L.part, L.n_pad, P, L.sc};
     const dim3 grid(P.nsb, (P.nsb / 2 + 1) * P.split);
     hipError_t e = hipSuccess;
     if (ev_b && (e = hipEventRecord(ev_b, stream)) != hipSuccess) return e;
     using Fn = void (*)(core::SymArgs);
-    const bool r = L.law == NBODY_LAW_R, eq = L.gm_equal > 0.f;
+    const bool r = L.law == NBODY_LAW_R, eq = L.equal;
     const Fn fn = r ? (eq ? sym_force_kernel<NBODY_LAW_R, true> : sym_force_kernel<NBODY_LAW_R, false>)
                     : (eq ? sym_force_kernel<NBODY_LAW_P, true> : sym_force_kernel<NBODY_LAW_P, false>);
     hipLaunchKernelGGL(fn, grid, dim3(kTile), 0, stream, A);

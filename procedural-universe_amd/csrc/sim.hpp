@@ -40,7 +40,7 @@ struct nbody_sim {
     nbody::ReadStage read_stage;
     std::vector<double> mass_host;        // FP64 masses (FORCES read-back = m * a)
     double max_gm = 0.0;                  // largest |G*m| (the direct sum's mass scale)
-    float gm_equal = 0.f;                 // FP32 G*m if every particle has the same positive one, else 0
+    double gm_equal = 0.0;                // G*m if every particle has the same positive one in FP32, else 0
     bool massless = false;                // some particle has no FP32 G*m
     nbody::DirectScale dscale{1.f, 1.f, 0.f, 1.f};  // direct sum's scaled units
     bool acc_valid = false;
