@@ -116,7 +116,9 @@ typedef struct nbody_config {
     int32_t tune_i_per_lane; /* direct kernel: targets per lane (0 = auto)      */
     int32_t tune_block;      /* direct kernel: threads per workgroup (0 = auto) */
     int32_t tune_split;      /* direct kernel: j-chunks per target (0 = auto)   */
-    int32_t reserved[8];
+    int32_t inject_rows_failures; /* test hook: bit i set: a batch's i-th allocation of partial
+                                     sums fails as on a full device (0 in production) */
+    int32_t reserved[7];
 } nbody_config;
 
 /* G = 1, law P, eps^2 = 1e-4, scale = 1, theta = 0.5, dynamic root,
@@ -332,8 +334,8 @@ nbody_status nbody_bh_cells(nbody_sim* sim, nbody_bh_cell* out, size_t capacity,
 
 /* The reference advances one particle set per INBodySim; a batch advances many
  * independent systems (galaxies) with one persistent kernel per step that
- * drains a queue of (system, target block) work items, largest first, over a
- * shared device arena, and runs a captured hipGraph of the steps.  A system's
+ * drains a queue of (system, block) work items, largest systems first (those summed
+ * one-sided behind the others), over a shared device arena, and runs a captured hipGraph of the steps.  A system's
  * forces are bit-identical whether it runs alone or in any mix.  Systems may
  * be added and removed between steps (the server does so); a batch is not
  * thread-safe. */
@@ -361,7 +363,9 @@ typedef struct nbody_batch_info {
 /* cfg->method must be NBODY_METHOD_DIRECT; capacity = arena size in particles
  * (each system takes its size rounded up to 256).  Steps of systems of more than
  * 1,024 particles also use up to 1.43 GB of device memory for partial sums,
- * allocated as they need it (without it, slower and rounded differently). */
+ * allocated as they need it.  Where the device has no room for it, systems that do
+ * not fit what the batch already holds take a slower sum that rounds differently
+ * until systems next join or leave, when it is asked for again. */
 nbody_status nbody_batch_create(const nbody_config* cfg, size_t capacity, nbody_batch** out);
 nbody_status nbody_batch_destroy(nbody_batch* batch);
 

@@ -121,7 +121,8 @@ class Config(ctypes.Structure):
         ("tune_i_per_lane", ctypes.c_int32),
         ("tune_block", ctypes.c_int32),
         ("tune_split", ctypes.c_int32),
-        ("reserved", ctypes.c_int32 * 8),
+        ("inject_rows_failures", ctypes.c_int32),
+        ("reserved", ctypes.c_int32 * 7),
     ]
 
 

@@ -16,7 +16,7 @@
 // group's two kernels after the other's.  The smaller systems' items are drained
 // behind the last group's tasks; only a batch without any pairs has a kernel of
 // its own for them.  Which way a system takes, and its tasks, depend on its size
-// alone.
+// alone, as long as the device has room for its rows.
 //
 // The queue lives in device memory (items, their count, per-step counters), so
 // a captured hipGraph of k steps stays valid while systems join and leave: only
@@ -307,6 +307,7 @@ struct nbody_batch {
         size_t off = 0, n = 0, n_pad = 0;
         DirectScale sc{};
         double max_gm = 0.0;
+        SymPlan sym{};         // as the items in use have it
         double gm_equal = 0.0;  // G*m if every particle has the same positive one in FP32, else 0
     };
     std::vector<Sys> systems;  // index = id = descriptor slot
@@ -326,7 +327,7 @@ struct nbody_batch {
     float4* d_rows = nullptr;
     size_t rows_cap = 0;
     int n_tasks = 0, n_groups = 0;
-    bool no_rows = false;  // the rows buffer could not be allocated
+    int32_t rows_attempts = 0;  // allocations of the rows buffer, for inject_rows_failures
     unsigned* d_counters = nullptr;
     int counters_cap = 0;
     bool items_dirty = true;
@@ -438,106 +439,146 @@ void arena_free(nbody_batch* b, size_t off, size_t len) {
     }
 }
 
-// Rebuild the work-item list (largest systems first) and upload it.
-nbody_status rebuild_items(nbody_batch* b) {
-    if (!b->items_dirty) return NBODY_OK;
-    const int per = b->tuning.block * b->tuning.i_per_lane;
+// The work of a step: what each system's descriptor holds, the one-sided items of a
+// batch without pairs, or the groups with their tasks and sums.
+struct Layout {
+    std::vector<SysDesc> descs;
+    std::vector<WorkItem> items;
+    std::vector<SymTask> tasks;
+    std::vector<SumItem> sums;
+    std::vector<SymGroup> groups;
+    size_t rows = 0;  // records of the rows buffer
+    uint64_t interactions = 0;
+};
+
+// The batch's systems, largest first, over unordered pairs where the plan and
+// `limit` records of rows allow, in groups whose rows fit `limit` together.
+Layout lay_out(const nbody_batch* b, size_t limit) {
+    Layout L;
     std::vector<int> order;
     for (size_t s = 0; s < b->systems.size(); ++s)
         if (b->systems[s].live && b->systems[s].n > 0) order.push_back(static_cast<int>(s));
     std::stable_sort(order.begin(), order.end(),
                      [&](int a, int c) { return b->systems[a].n_pad > b->systems[c].n_pad; });
-    std::vector<WorkItem> items;
-    std::vector<SymTask> tasks;
-    std::vector<SumItem> sums;
-    std::vector<SymGroup> groups;
-    std::vector<SysDesc> descs(b->systems.size());
-    uint64_t inter = 0;
+    L.descs.resize(b->systems.size());
     for (size_t s = 0; s < b->systems.size(); ++s) {
         const auto& y = b->systems[s];
-        descs[s] = SysDesc{static_cast<int>(y.off), static_cast<int>(y.n), static_cast<int>(y.n_pad), y.gm_equal > 0,
-                           y.sc, sym_out(b->cfg.law, y.sc, y.gm_equal), {}, 0};
+        L.descs[s] = SysDesc{static_cast<int>(y.off), static_cast<int>(y.n), static_cast<int>(y.n_pad), y.gm_equal > 0,
+                             y.sc, sym_out(b->cfg.law, y.sc, y.gm_equal), {}, 0};
     }
-    // Groups of systems, largest first, whose rows fit the buffer together.
-    size_t rows = 0, rows_max = 0;
-    std::vector<int> in_group, one_sided;
-    auto close_group = [&] {
-        if (in_group.empty()) return;
-        SymGroup g{static_cast<int>(tasks.size()), 0, static_cast<int>(sums.size()), 0};
-        for (const bool diagonal : {false, true})  // the shorter tasks last
-            for (int s : in_group) {
-                const SymPlan& P = descs[s].sym;
-                for (int d = diagonal ? 0 : 1; d <= (diagonal ? 0 : P.nsb / 2); ++d)
-                    for (int a = 0; a < (d > 0 && 2 * d == P.nsb ? d : P.nsb); ++a)
-                        for (int h = 0; h < P.split; ++h) tasks.push_back(SymTask{s, a, d, h});
-            }
-        for (int s : in_group)
-            for (int i = 0; i < descs[s].n; i += 64) sums.push_back(SumItem{s, i});
-        g.task1 = static_cast<int>(tasks.size());
-        g.sum1 = static_cast<int>(sums.size());
-        groups.push_back(g);
-        in_group.clear();
-        rows_max = std::max(rows_max, rows);
-        rows = 0;
-    };
+    std::vector<int> one_sided, pairs;
     for (int s : order) {
         const auto& y = b->systems[s];
-        inter += static_cast<uint64_t>(y.n) * y.n;
-        const SymPlan P = b->no_rows ? SymPlan{} : batch_sym_plan(y.n_pad);
-        if (P.nsb > 0) {
-            const size_t need = sym_part_records(P, static_cast<int>(y.n_pad));
-            if (rows + need > kRowsRecords) close_group();
-            descs[s].sym = P;
-            descs[s].rows = rows;
-            rows += need;
-            in_group.push_back(s);
-        } else {
-            one_sided.push_back(s);
-        }
+        L.interactions += static_cast<uint64_t>(y.n) * y.n;
+        L.descs[s].sym = batch_sym_plan(y.n_pad);
+        if (L.descs[s].sym.nsb > 0 && sym_part_records(L.descs[s].sym, static_cast<int>(y.n_pad)) > limit)
+            L.descs[s].sym = SymPlan{};
+        (L.descs[s].sym.nsb > 0 ? pairs : one_sided).push_back(s);
+    }
+    if (pairs.empty()) {  // a kernel of their own
+        const int per = b->tuning.block * b->tuning.i_per_lane;
+        for (int s : one_sided)
+            for (int i = 0; i < L.descs[s].n_pad; i += per) L.items.push_back(WorkItem{s, i});
+        return L;
+    }
+    size_t rows = 0;
+    std::vector<int> in_group;
+    auto close_group = [&] {
+        if (in_group.empty()) return;
+        SymGroup g{static_cast<int>(L.tasks.size()), 0, static_cast<int>(L.sums.size()), 0};
+        for (const bool diagonal : {false, true})  // the shorter tasks last
+            for (int s : in_group) {
+                const SymPlan& P = L.descs[s].sym;
+                for (int d = diagonal ? 0 : 1; d <= (diagonal ? 0 : P.nsb / 2); ++d)
+                    for (int a = 0; a < (d > 0 && 2 * d == P.nsb ? d : P.nsb); ++a)
+                        for (int h = 0; h < P.split; ++h) L.tasks.push_back(SymTask{s, a, d, h});
+            }
+        for (int s : in_group)
+            for (int i = 0; i < L.descs[s].n; i += 64) L.sums.push_back(SumItem{s, i});
+        g.task1 = static_cast<int>(L.tasks.size());
+        g.sum1 = static_cast<int>(L.sums.size());
+        L.groups.push_back(g);
+        in_group.clear();
+        L.rows = std::max(L.rows, rows);
+        rows = 0;
+    };
+    for (int s : pairs) {
+        const size_t need = sym_part_records(L.descs[s].sym, L.descs[s].n_pad);
+        if (rows + need > limit) close_group();
+        L.descs[s].rows = rows;
+        rows += need;
+        in_group.push_back(s);
     }
     close_group();
-    // With the last group's tasks, behind them; without any, a kernel of their own.
-    for (int s : one_sided) {
-        const int n_pad = static_cast<int>(b->systems[s].n_pad);
-        if (groups.empty())
-            for (int i = 0; i < n_pad; i += per) items.push_back(WorkItem{s, i});
-        else
-            for (int i = 0; i < n_pad; i += kTile) tasks.push_back(SymTask{s, i / kTile, -1, 0});
+    // The one-sided items behind the last group's tasks, those of systems too large
+    // for rows too.  In front of the tasks, as the longest items, they gain less than
+    // they lose: two systems of 260,000 among 64 of 8,000 37.2 ms a step in place of
+    // 37.6, one of 300,000 among eight of 30,000 33.6 in place of 30.0.
+    for (int s : one_sided)
+        for (int i = 0; i < L.descs[s].n_pad; i += kTile) L.tasks.push_back(SymTask{s, i / kTile, -1, 0});
+    L.groups.back().task1 = static_cast<int>(L.tasks.size());
+    return L;
+}
+
+// Room for `need` records of rows, more if the device has it; the buffer held stays
+// where neither fits.
+nbody_status ensure_rows(nbody_batch* b, size_t need) {
+    if (need <= b->rows_cap) return NBODY_OK;
+    const int32_t attempt = b->rows_attempts++;
+    if (attempt < 31 && (b->cfg.inject_rows_failures >> attempt) & 1) {
+        set_error("injected allocation failure");
+        return NBODY_ERR_OUT_OF_MEMORY;
     }
-    if (!groups.empty()) groups.back().task1 = static_cast<int>(tasks.size());
-    if (rows_max > b->rows_cap) {
-        const nbody_status st = ensure_dev(reinterpret_cast<void**>(&b->d_rows), b->rows_cap, rows_max, sizeof(float4),
-                                           b->stream, kRowsRecords);
+    nbody_status st = ensure_dev(reinterpret_cast<void**>(&b->d_rows), b->rows_cap, need, sizeof(float4), b->stream,
+                                 kRowsRecords);
+    if (st != NBODY_ERR_OUT_OF_MEMORY) return st;
+    (void)hipGetLastError();
+    st = ensure_dev(reinterpret_cast<void**>(&b->d_rows), b->rows_cap, need, sizeof(float4), b->stream, need);
+    if (st == NBODY_ERR_OUT_OF_MEMORY) (void)hipGetLastError();
+    if (st == NBODY_OK) clear_error();
+    return st;
+}
+
+// Lay the work out anew and upload it.  On a device too full for the rows it wants,
+// what the buffer already held allows: more groups, and one-sided sums for the
+// systems that do not fit it alone; the next change of the systems asks again.
+nbody_status rebuild_items(nbody_batch* b) {
+    if (!b->items_dirty) return NBODY_OK;
+    try {
+        Layout L = lay_out(b, kRowsRecords);
+        nbody_status st = ensure_rows(b, L.rows);
         if (st == NBODY_ERR_OUT_OF_MEMORY) {
-            // A device too full for the rows: the one-sided sum for every
-            // system, from now on.
-            (void)hipGetLastError();
             clear_error();
-            b->no_rows = true;
-            return rebuild_items(b);
+            L = lay_out(b, b->rows_cap);
+            st = NBODY_OK;
         }
         NB_TRY(st);
-    }
-    auto upload = [&](auto** dev, size_t& cap, const auto& host) -> nbody_status {
-        const size_t elem = sizeof(host[0]);
-        NB_TRY(ensure_dev(reinterpret_cast<void**>(dev), cap, std::max<size_t>(host.size(), 1), elem, b->stream));
-        if (!host.empty())
-            NB_HIP(hipMemcpyAsync(*dev, host.data(), host.size() * elem, hipMemcpyHostToDevice, b->stream));
+        auto upload = [&](auto** dev, size_t& cap, const auto& host) -> nbody_status {
+            const size_t elem = sizeof(host[0]);
+            NB_TRY(ensure_dev(reinterpret_cast<void**>(dev), cap, std::max<size_t>(host.size(), 1), elem, b->stream));
+            if (!host.empty())
+                NB_HIP(hipMemcpyAsync(*dev, host.data(), host.size() * elem, hipMemcpyHostToDevice, b->stream));
+            return NBODY_OK;
+        };
+        NB_TRY(upload(&b->d_items, b->items_cap, L.items));
+        NB_TRY(upload(&b->d_sys, b->sys_cap, L.descs));
+        NB_TRY(upload(&b->d_tasks, b->tasks_cap, L.tasks));
+        NB_TRY(upload(&b->d_sums, b->sums_cap, L.sums));
+        NB_TRY(upload(&b->d_groups, b->groups_cap, L.groups));
+        b->n_items = static_cast<int>(L.items.size());
+        b->n_tasks = static_cast<int>(L.tasks.size());
+        b->n_groups = static_cast<int>(L.groups.size());
+        NB_HIP(hipMemcpyAsync(b->d_n_items, &b->n_items, sizeof(int), hipMemcpyHostToDevice, b->stream));
+        NB_HIP(hipStreamSynchronize(b->stream));  // host vectors go out of scope
+        for (size_t s = 0; s < L.descs.size(); ++s) b->systems[s].sym = L.descs[s].sym;
+        b->interactions_per_step = L.interactions;
+        b->items_dirty = false;
         return NBODY_OK;
-    };
-    NB_TRY(upload(&b->d_items, b->items_cap, items));
-    NB_TRY(upload(&b->d_sys, b->sys_cap, descs));
-    NB_TRY(upload(&b->d_tasks, b->tasks_cap, tasks));
-    NB_TRY(upload(&b->d_sums, b->sums_cap, sums));
-    NB_TRY(upload(&b->d_groups, b->groups_cap, groups));
-    b->n_items = static_cast<int>(items.size());
-    b->n_tasks = static_cast<int>(tasks.size());
-    b->n_groups = static_cast<int>(groups.size());
-    NB_HIP(hipMemcpyAsync(b->d_n_items, &b->n_items, sizeof(int), hipMemcpyHostToDevice, b->stream));
-    NB_HIP(hipStreamSynchronize(b->stream));  // host vectors go out of scope
-    b->interactions_per_step = inter;
-    b->items_dirty = false;
-    return NBODY_OK;
+    } catch (const std::bad_alloc&) {
+        (void)hipStreamSynchronize(b->stream);
+        set_error("no host memory for the work of %zu systems", b->systems.size());
+        return NBODY_ERR_OUT_OF_MEMORY;
+    }
 }
 
 // A graph exec is only destroyed once its launches have completed (they all
@@ -869,7 +910,7 @@ nbody_status nbody_batch_step_sequential(nbody_batch* b, float dt, int32_t nstep
         if (!y.live) continue;
         DirectShape shape = split_small ? direct_default_shape(static_cast<int>(y.n_pad)) : DirectShape{1, 256, 1};
         // the rows' buffer holds any one system's (rebuild_items)
-        const SymPlan P = split_small || b->no_rows ? SymPlan{} : batch_sym_plan(y.n_pad);
+        const SymPlan P = split_small ? SymPlan{} : y.sym;
         const size_t split =
             P.nsb > 0 ? 0 : static_cast<size_t>(direct_effective_split(shape, static_cast<int>(y.n_pad)));
         if (split * y.n_pad > b->part_elems) {
