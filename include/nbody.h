@@ -342,9 +342,10 @@ nbody_status nbody_bh_cells(nbody_sim* sim, nbody_bh_cell* out, size_t capacity,
 typedef struct nbody_batch nbody_batch;
 
 typedef struct nbody_batch_tuning {
-    int32_t i_per_lane;   /* targets per lane: 1 or 2                              */
-    int32_t block;        /* threads per workgroup: 128 or 256                     */
-    int32_t wg_per_cu;    /* persistent workgroups launched per CU (1..64)         */
+    int32_t i_per_lane;   /* targets per lane: 1 or 2 (one-sided kernel)           */
+    int32_t block;        /* threads per workgroup: 128 or 256 (one-sided kernel)  */
+    int32_t wg_per_cu;    /* persistent workgroups launched per CU (1..64; of the  */
+                          /* kernel that takes pairs at most 6, its resident ones) */
     int32_t reserved[5];
     double  ms_per_step;  /* the tuner's time for one step of this shape (0: none) */
 } nbody_batch_tuning;
@@ -397,7 +398,10 @@ nbody_status nbody_batch_get_info(nbody_batch* batch, nbody_batch_info* out);
 nbody_status nbody_batch_set_tuning(nbody_batch* batch, const nbody_batch_tuning* tuning);
 
 /* Time one step of each candidate (targets per lane, block, workgroups per
- * CU) on the live systems, keep the fastest, and leave the state as it was. */
+ * CU) on the live systems, keep the fastest, and leave the state as it was.  The
+ * one-sided kernel runs only where no system has more than 1,024 particles; with
+ * larger ones only the workgroups per CU are tried, and the targets per lane and
+ * block stay as they were set. */
 nbody_status nbody_batch_tune(nbody_batch* batch, float dt, nbody_batch_tuning* out);
 
 /* Run steps through a captured hipGraph (default) or as plain launches. */

@@ -622,6 +622,8 @@ nbody_status enqueue_steps(nbody_batch* b, float dt, int nsteps) {
     const int per = counters_per_step(b), counters = per * nsteps;
     hipLaunchKernelGGL(fill_u32_kernel, dim3((counters + 255) / 256), dim3(256), 0, b->stream, b->d_counters, counters, 0u);
     const dim3 grid(static_cast<unsigned>(b->tuning.wg_per_cu * b->cus));
+    // six workgroups of the pair kernel are resident per CU: more would only wait
+    const dim3 sym_grid(static_cast<unsigned>(std::min(b->tuning.wg_per_cu, 6) * b->cus));
     const auto sym = b->cfg.law == NBODY_LAW_R ? batch_sym_kernel<NBODY_LAW_R> : batch_sym_kernel<NBODY_LAW_P>;
     const auto sum = b->cfg.law == NBODY_LAW_R ? batch_sum_kernel<NBODY_LAW_R> : batch_sum_kernel<NBODY_LAW_P>;
     int parity = b->cur;
@@ -629,7 +631,7 @@ nbody_status enqueue_steps(nbody_batch* b, float dt, int nsteps) {
         const BatchLaunch L = launch_for(b, parity, dt);
         unsigned* counter = b->d_counters + static_cast<size_t>(s) * per;
         for (int g = 0; g < b->n_groups; ++g) {
-            hipLaunchKernelGGL(sym, dim3(6 * b->cus), dim3(kTile), 0, b->stream, L, g, counter + 1 + g);
+            hipLaunchKernelGGL(sym, sym_grid, dim3(kTile), 0, b->stream, L, g, counter + 1 + g);
             hipLaunchKernelGGL(sum, dim3(8 * b->cus), dim3(256), 0, b->stream, L, g);
         }
         if (b->n_items > 0) hipLaunchKernelGGL(fn, grid, dim3(b->tuning.block), 0, b->stream, L, counter);
@@ -1054,7 +1056,9 @@ nbody_status nbody_batch_get_timing(nbody_batch* b, nbody_timing* out) {
 
 // Time one step of each candidate shape on the live batch and keep the
 // fastest.  The state is saved before and restored after, so tuning leaves the
-// batch as it found it.
+// batch as it found it.  With pairs in the batch only the workgroups per CU are tried:
+// the one-sided kernel, whose targets per lane and block the others are, does not
+// run, and more workgroups than are resident are the same launch.
 nbody_status nbody_batch_tune(nbody_batch* b, float dt, nbody_batch_tuning* out) {
     clear_error();
     NB_CHECK(b, NBODY_ERR_INVALID_ARG, "batch is null");
@@ -1092,9 +1096,10 @@ nbody_status nbody_batch_tune(nbody_batch* b, float dt, nbody_batch_tuning* out)
     b->use_graph = false;
     nbody_batch_tuning best = keep;
     double best_ms = 1e300;
-    const int ks[] = {1, 2};
-    const int blocks[] = {256, 128};
-    const int wgs[] = {2, 4, 8, 16};
+    const bool pairs = b->n_groups > 0;
+    const std::vector<int> ks = pairs ? std::vector<int>{keep.i_per_lane} : std::vector<int>{1, 2};
+    const std::vector<int> blocks = pairs ? std::vector<int>{keep.block} : std::vector<int>{256, 128};
+    const std::vector<int> wgs = pairs ? std::vector<int>{2, 4, 8} : std::vector<int>{2, 4, 8, 16};
     for (int k : ks) {
         for (int blk : blocks) {
             for (int wg : wgs) {
