@@ -2067,16 +2067,36 @@ inline int mass_rows(int n) {
 //              0.7:   8,388,608                                                  5620  5837
 //   Plummer,   0.5:  16,777,216                                                 27142 28379
 //              1.0:  16,777,216                                                  8144  7989
+// Wide opening angles (a group's walk is short, and what several wavefronts add to
+// it counts for more), discs / spheres:
+//              n          theta      64x4           64x2           64x1
+//          100,000         1.0     73 /  84       83 /  83      150 / 146
+//                          1.2     68 /  71       67 /  65      115 / 105
+//                          2.0     50 /  50       41 /  42       44 /  45
+//          500,000         1.2    240 / 254      185 / 193      228 / 220
+//                          2.0    157 / 155      127 / 126      131 / 133
+//        1,000,000         1.5       395            272            286
+//        2,000,000         1.0   1116 /1185      841 / 928      842 / 952
+//                          1.2    934 / 991      675 / 709      642 / 673
+//        4,194,304         1.0                     1690           1749
+//                          1.2                     1354           1284
+//                          2.0                      875            853
+//        8,000,000         1.0                  3379 /3658     3387 /3742
+//                          1.5                  1948 /2039     1686 /1673
 // (One wavefront to a group of 8, 16 or 32: 53 at 4,000, 138 at 32,768, 234 at
 // 131,072, 309 at 200,003.)
 struct TravShape {
     int group, waves;
 };
 
-inline TravShape trav_shape(int n) {
+inline TravShape trav_shape(int n, double theta) {
     if (n <= 12288) return {16, 8};
     if (n <= 24576) return {32, 8};
     if (n <= 65536) return {32, 4};
+    if (theta > 1.1) {
+        if (n <= 1572864) return {64, 2};
+        return {64, 1};
+    }
     if (n <= 524288) return {64, 4};
     if (n <= 8388608) return {64, 2};
     return {64, 1};
@@ -2348,7 +2368,7 @@ nbody_status bh_step(nbody_sim* s, float dt, bool kick, hipEvent_t ev_b, hipEven
     A.dt = dt;
     A.dts = static_cast<float>(static_cast<double>(dt) / s->cfg.scale);
     if (ev_b) NB_HIP(hipEventRecord(ev_b, st));
-    const TravShape shape = trav_shape(n);
+    const TravShape shape = trav_shape(n, s->cfg.theta);
     const auto fn = s->cfg.law == NBODY_LAW_R ? traverse_fn<NBODY_LAW_R>(shape) : traverse_fn<NBODY_LAW_P>(shape);
     hipLaunchKernelGGL(fn, dim3(blocks_for(n, shape.group)), dim3(64 * shape.waves), 0, st, b->pos_sorted, b->blocks,
                        b->first, b->last, A);
