@@ -340,7 +340,9 @@ def bench_bh(pu, args):
             "walk": {
                 "list_entries_per_wave": 64.0 * stats["list_entries"] / (n * args.steps),
                 "cells_opened_per_wave": 64.0 * stats["cells_opened"] / (n * args.steps),
-                "lane_efficiency": interactions / (64.0 * max(1, stats["list_entries"])),
+                # the share of its group that an entry applies to; the lanes that evaluate it are the whole
+                # group or, at most sizes from 65,537 on, the half groups it reaches (55% of them at 2^22)
+                "group_share_per_entry": interactions / (64.0 * max(1, stats["list_entries"])),
             },
             "ic_seconds": t_ic,
         },
@@ -400,7 +402,7 @@ def bh_summary(pu):
         "tree_ms_per_step": c["tree_ms_per_step"],
         "traversal_ms_per_step": c["traversal_ms_per_step"],
         "interactions_per_particle": c["interactions_per_particle"],
-        "lane_efficiency": c["walk"]["lane_efficiency"],
+        "group_share_per_entry": c["walk"]["group_share_per_entry"],
         "traversal_frac_fp32_peak": r["roofline"]["frac"],
         "accuracy_vs_direct": r["accuracy_vs_direct"],
         "stack_overflow": c["stack_overflow"],
@@ -716,7 +718,7 @@ def main():
     sim.synchronize()
     elapsed = time.perf_counter() - t0
     timing = sim.timing()
-    # the shape that the sum over unordered pairs reports
+    # the shape that the sum over unordered pairs reports (this benchmark sets none by hand)
     pairs = n >= 16384 and (timing.i_per_lane, timing.block) == (4, 256)
 
     e1 = None if args.no_energy else sim.diagnostics()
@@ -765,7 +767,9 @@ def main():
             "traffic_source": "rocprofv3 FETCH_SIZE x2.0 + WRITE_SIZE x1.0 (256 MiB copy calibration), "
             "profiles/direct_force_n1m_law_r_traffic.md",
             "algorithmic_bytes": 80.0 * n,
-            "kernel": "sym_force_kernel + sym_reduce_kernel (unordered pairs, kick-drift)"
+            # kernel_ms brackets the force kernel alone: the pairs' row sums and kick-drift
+            # (sym_reduce_kernel, 0.3% of a step at 2^20) follow it
+            "kernel": "sym_force_kernel (unordered pairs)"
             if pairs
             else "direct_force_kernel or small_step_kernel (one-sided, fused kick-drift)",
             "kernel_ms": force_ms,

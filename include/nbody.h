@@ -214,9 +214,9 @@ nbody_status nbody_field(nbody_sim* sim, const float* points, size_t m, float* a
 /* nbody_field without any device allocation.  No counterpart in the
  * reference: for callers that cannot allocate device memory (code between
  * graph captures, tight serving loops, harnesses that forbid hipMalloc).  The
- * points and their accelerations are staged in a fixed device array of
- * NBODY_FIELD_NOALLOC_MAX_POINTS records each, which every device the library
- * runs on holds until the process ends (2 MiB); more points give
+ * points, then their accelerations, and partial sums are staged in a fixed device
+ * array of twice NBODY_FIELD_NOALLOC_MAX_POINTS records, which every device the
+ * library runs on holds until the process ends (2 MiB); more points give
  * NBODY_ERR_CAPACITY.  All calls on one device share that array: calls that
  * overlap on one device (from different threads or handles) race.  Results
  * equal nbody_field's bit for bit. */
@@ -258,7 +258,8 @@ typedef struct nbody_timing {
     double  tree_ms;            /* summed tree-build time (Barnes-Hut only)        */
     double  step_ms;            /* wall time of the call on the device (events)   */
     uint64_t interactions;      /* pair or node interactions evaluated             */
-    int32_t i_per_lane;         /* direct kernel launch shape in use               */
+    int32_t i_per_lane;         /* direct kernel launch shape in use: of whichever  */
+                                /* kernel the size chose, not always one for tune_* */
     int32_t block;
     int32_t split;
     int32_t reserved[5];
@@ -293,8 +294,9 @@ typedef struct nbody_bh_stats {
     uint64_t interactions;    /* cell + particle interactions since the last nbody_step began   */
     uint32_t outside_root;    /* particles clamped into a fixed root (the reference drops them) */
     uint32_t stack_overflow;  /* nonzero if a traversal stack overflowed (forces invalid)        */
-    uint64_t list_entries;    /* sources evaluated, each by a whole group of particles, some of  */
-                              /* them masked (64 of Morton order; 16 or 32 in small systems)     */
+    uint64_t list_entries;    /* sources taken for a group of particles (64 of Morton order; 16  */
+                              /* or 32 in small systems), once each, whether its lanes evaluate  */
+                              /* it together or, at most sizes from 65,537, by half groups       */
     uint64_t cells_opened;    /* cells whose children were examined for a group                  */
 } nbody_bh_stats;
 
@@ -427,7 +429,8 @@ typedef struct nbody_server nbody_server;
 
 typedef struct nbody_server_config {
     nbody_config sim;          /* law, G, softening, scale, theta, device (method ignored) */
-    uint64_t memory_budget;    /* device bytes the request states may hold                  */
+    uint64_t memory_budget;    /* device bytes the request states may hold (the batch's     */
+                               /* partial sums, at most 1.43 GB, come on top)               */
     uint64_t direct_capacity;  /* particles in the direct-sum arena                         */
     uint32_t bh_threshold;     /* requests with n >= bh_threshold use Barnes-Hut            */
     int32_t  max_active_bh;    /* concurrent Barnes-Hut requests                            */

@@ -5,9 +5,10 @@
 // Here every system lives in one device arena (the same padded SoA records as a
 // single simulation) and one persistent kernel per step drains a queue of
 // (system, target block) work items, largest systems first, so small and large
-// systems fill the machine together.  Each work item runs the single-system
-// core (direct_core.hpp) over its own system's sources, so a system's forces are
-// the same bits whether it runs alone or in any mix.
+// systems fill the machine together.  Each work item runs the one-sided core
+// (direct_core.hpp) over its own system's sources.  A system's forces are the same
+// bits whether it runs alone or in any mix (a simulation handle chooses its kernel
+// and its blocks by other sizes, so its bits differ).
 //
 // Systems of more than 1,024 particles take the sum over unordered pairs
 // (direct_sym.hip) instead: a persistent kernel drains their tasks, then one adds
@@ -19,8 +20,9 @@
 // alone, as long as the device has room for its rows.
 //
 // The queue lives in device memory (items, their count, per-step counters), so
-// a captured hipGraph of k steps stays valid while systems join and leave: only
-// the item list is rewritten between launches.  The per-step counters are
+// a captured hipGraph of k steps stays valid while systems join and leave and its
+// buffers, groups and kinds of kernels stay: only the item lists are rewritten
+// between launches.  The per-step counters are
 // cleared by a kernel inside the graph.
 #include <hip/hip_runtime.h>
 

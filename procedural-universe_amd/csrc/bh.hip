@@ -1338,7 +1338,7 @@ __device__ __forceinline__ void flush_list(const float4* lsrc, const float* lk, 
 // Workgroups are dealt to the accelerator's XCDs in turn (workgroup b to XCD
 // b mod 8), and each XCD has its own L2.  Neighbouring particle groups in
 // Morton order walk nearly the same cells, so the groups are renumbered to
-// give every XCD runs of 8 consecutive groups of the order (its L2 then holds
+// give every XCD runs of 2,048 particles of the order (its L2 then holds
 // the child blocks those waves share), the runs dealt round the XCDs so that
 // dense and sparse regions spread over all of them.  A bijection on [0, nb).
 constexpr int kXcds = 8;

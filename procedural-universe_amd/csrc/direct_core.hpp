@@ -1,5 +1,7 @@
-// Device core of the direct sum, shared by the single-system kernel and the
-// batch executor so that a system's forces are the same bits either way.
+// Device core of the one-sided direct sum, shared by the single-system kernel, the
+// field and the batch's small systems and baseline; the arithmetic that the sum over
+// unordered pairs (direct_sym_core.hpp) and whole steps of small systems (direct.hip)
+// take from it is described here too.
 //
 // Scaled units.  Each system carries two powers of two (DirectScale): a length
 // lambda and a mass scale c.  Sources and targets are multiplied by 1/lambda

@@ -51,6 +51,9 @@ namespace {
 // 412 B in all) and a large read's staging (12 B): 424 B, counted as 432 (an
 // upper bound).
 constexpr size_t kBhBytesPerParticle = 80 + 352;
+// A direct request's records in the batch's arena.  The batch's rows of partial sums
+// (at most 1.43 GB for all its systems) are outside the budget: where they find no
+// room the batch steps without them.
 constexpr size_t kDirectBytesPerParticle = 64;
 
 struct Request {
