@@ -208,6 +208,7 @@ double extent_of(const float4* p, size_t n) {
 // orders of magnitude keeps them, which the pair arithmetic's range allows).
 void set_scale(nbody_sim* s, double extent) {
     s->dscale = direct_scale_for(s->cfg.law, s->cfg.softening, extent, s->max_gm);
+    s->sym_units = sym_units(s->cfg.law, s->cfg.softening, s->dscale, s->gm_equal);
 }
 
 // What the direct sum chooses by the masses (n in FP64): whether every particle
@@ -316,8 +317,6 @@ DirectLaunch launch_for(nbody_sim* s, float dt) {
     L.n_pad = static_cast<int>(s->n_pad);
     L.law = s->cfg.law;
     L.sc = s->dscale;
-    L.equal = s->gm_equal > 0;
-    L.sums_out = sym_out(s->cfg.law, s->dscale, s->gm_equal);
     L.massless = s->massless;
     L.dt = dt;
     L.dts = static_cast<float>(static_cast<double>(dt) / s->cfg.scale);
@@ -339,7 +338,7 @@ nbody_status force_pass(nbody_sim* s, float dt, bool kick, hipEvent_t ev_b, hipE
     } else {
         DirectLaunch L = launch_for(s, dt);
         NB_HIP(s->small         ? small_step(L, kick, s->stream, ev_b, ev_e)
-               : s->sym.nsb > 0 ? sym_step(L, s->sym, kick, s->stream, ev_b, ev_e)
+               : s->sym.nsb > 0 ? sym_step(L, s->sym, s->sym_units, kick, s->stream, ev_b, ev_e)
                                 : direct_step(L, s->shape, kick, s->stream, ev_b, ev_e));
         s->step_interactions += static_cast<uint64_t>(s->n) * static_cast<uint64_t>(s->n);
     }

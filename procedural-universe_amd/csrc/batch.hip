@@ -50,9 +50,8 @@ struct SysDesc {
     int off;         // first record in the arena
     int n;           // real particles
     int n_pad;       // padded to kTile
-    int equal;       // every particle has the same positive G m
     DirectScale sc;  // the system's scaled units
-    SymOut out;      // its rows' sums back to accelerations
+    SymUnits units;  // and those of its pairs
     SymPlan sym;     // nsb > 0: over unordered pairs
     size_t rows;     // its partial sums in the rows buffer (records)
 };
@@ -221,16 +220,16 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(6))) void
             one_sided_item<LAW, 1, kTile>(B, D, w.a * kTile, S.tiles);
             continue;
         }
-        const core::SymArgs A{B.pos_in + D.off, B.rows + D.rows, D.n_pad, D.sym, D.sc};
+        const core::SymArgs A{B.pos_in + D.off, B.rows + D.rows, D.n_pad, D.sym, D.sc, D.units.alpha, D.units.soft};
         const int H = D.sym.nsb / 2;
         if (w.d == 0) {
-            if (D.equal) core::sym_task<LAW, false, true>(A, S.pairs, w.a, w.a, w.h, w.h, 0);
+            if (D.units.equal) core::sym_task<LAW, false, true>(A, S.pairs, w.a, w.a, w.h, w.h, 0);
             else core::sym_task<LAW, false, false>(A, S.pairs, w.a, w.a, w.h, w.h, 0);
         } else {
             int b = w.a + w.d;
             if (b >= D.sym.nsb) b -= D.sym.nsb;
             const int rowi = w.d * D.sym.split + w.h, rowj = (H + 1) * D.sym.split + w.d - 1;
-            if (D.equal) core::sym_task<LAW, true, true>(A, S.pairs, w.a, b, w.h, rowi, rowj);
+            if (D.units.equal) core::sym_task<LAW, true, true>(A, S.pairs, w.a, b, w.h, rowi, rowj);
             else core::sym_task<LAW, true, false>(A, S.pairs, w.a, b, w.h, rowi, rowj);
         }
     }
@@ -247,7 +246,7 @@ __global__ __launch_bounds__(256) void batch_sum_kernel(BatchLaunch B, int group
         const SysDesc D = B.sys[w.sys];
         const int i = w.i + lane;
         float s[3];
-        core::sum_rows(B.rows + D.rows, D.sym, D.n_pad, i, sums, wave, lane, D.out, s);
+        core::sum_rows(B.rows + D.rows, D.sym, D.n_pad, i, sums, wave, lane, D.units.out_hi, D.units.out_lo, s);
         if (wave == 0 && i < D.n) {
             const float4 x = B.pos_in[D.off + i];
             core::sums_of_a_lost_particle<LAW>(x, D.sc, s);
@@ -465,8 +464,8 @@ Layout lay_out(const nbody_batch* b, size_t limit) {
     L.descs.resize(b->systems.size());
     for (size_t s = 0; s < b->systems.size(); ++s) {
         const auto& y = b->systems[s];
-        L.descs[s] = SysDesc{static_cast<int>(y.off), static_cast<int>(y.n), static_cast<int>(y.n_pad), y.gm_equal > 0,
-                             y.sc, sym_out(b->cfg.law, y.sc, y.gm_equal), {}, 0};
+        L.descs[s] = SysDesc{static_cast<int>(y.off), static_cast<int>(y.n), static_cast<int>(y.n_pad), y.sc,
+                             sym_units(b->cfg.law, b->cfg.softening, y.sc, y.gm_equal), {}, 0};
     }
     std::vector<int> one_sided, pairs;
     for (int s : order) {
@@ -932,15 +931,14 @@ nbody_status nbody_batch_step_sequential(nbody_batch* b, float dt, int32_t nstep
             L.vel = b->vel + y.off;
             L.acc = b->acc + y.off;
             L.part = P.nsb > 0 ? b->d_rows : b->part;
-            L.equal = y.gm_equal > 0;
-            L.sums_out = sym_out(b->cfg.law, y.sc, y.gm_equal);
             L.n = static_cast<int>(y.n);
             L.n_pad = static_cast<int>(y.n_pad);
             L.law = b->cfg.law;
             L.sc = y.sc;
             L.dt = dt;
             L.dts = static_cast<float>(static_cast<double>(dt) / b->cfg.scale);
-            NB_HIP(P.nsb > 0 ? sym_step(L, P, true, b->stream, nullptr, nullptr)
+            NB_HIP(P.nsb > 0 ? sym_step(L, P, sym_units(b->cfg.law, b->cfg.softening, y.sc, y.gm_equal), true, b->stream,
+                                        nullptr, nullptr)
                              : direct_step(L, shape, true, b->stream, nullptr, nullptr));
             parity ^= 1;
         }

@@ -424,20 +424,6 @@ DirectScale direct_scale_for(int law, double softening, double extent, double ma
     sc.mass_k = law == NBODY_LAW_R ? std::ldexp(1.0f, e_mass) : std::ldexp(1.0f, -e_mass);
     sc.soft = static_cast<float>(std::ldexp(softening, -2 * e_len));
     sc.out = std::ldexp(1.0f, e_mass - 2 * e_len);
-    // With alpha = 1 the sum of r2, rounded already, and S' rounds the same way for
-    // every r2 of a binade, an error that no number of pairs averages out: 3% of
-    // the RMS error at N = 2^20, 7% at 2^21 (law R, unequal masses).  The product's
-    // bits below r2's last make it a random one, as the one-sided sum's folded
-    // mass does.  Of the 64 factors with seven such bits the one whose alpha S' is
-    // nearest a float.
-    sc.alpha = 1.0f;
-    const double s = std::ldexp(softening, -2 * e_len);
-    double best = 2.0;
-    for (int k = 1; law == NBODY_LAW_R && k < 128; k += 2) {
-        const double as = s * (128 + k) / 128.0, off = std::fabs(static_cast<double>(static_cast<float>(as)) - as);
-        if (off < best * as || s == 0.0) best = s == 0.0 ? 0.0 : off / as, sc.alpha = (128 + k) / 128.0f;
-    }
-    sc.alpha_soft = static_cast<float>(s * static_cast<double>(sc.alpha));
     return sc;
 }
 
@@ -452,12 +438,30 @@ double equal_gm(double G, const double* mass, size_t n) {
     return same ? G * mass[0] : static_cast<double>(first);
 }
 
-SymOut sym_out(int law, const DirectScale& sc, double gm_equal) {
-    double o = sc.out;
-    if (gm_equal > 0) o *= gm_equal * (law == NBODY_LAW_R ? 1.0 / sc.mass_k : sc.mass_k);
-    else o *= sc.alpha;
-    const float hi = static_cast<float>(o);
-    return SymOut{hi, std::isfinite(hi) ? static_cast<float>(o - static_cast<double>(hi)) : 0.f};
+SymUnits sym_units(int law, double softening, const DirectScale& sc, double gm_equal) {
+    SymUnits u{gm_equal > 0, 1.0f, sc.soft, 0.f, 0.f};
+    double out = sc.out;
+    if (u.equal) {
+        out *= gm_equal * (law == NBODY_LAW_R ? 1.0 / sc.mass_k : sc.mass_k);
+    } else if (law == NBODY_LAW_R) {
+        // With alpha = 1 the sum of r2, rounded already, and S' rounds the same way
+        // for every r2 of a binade, an error that no number of pairs averages out: 3%
+        // of the RMS error at N = 2^20, 7% at 2^21.  The product's bits below r2's
+        // last make it a random one, as the one-sided sum's folded mass does.  Of
+        // the 64 factors with seven such bits the one whose alpha S' is nearest a
+        // float.
+        const double s = softening * static_cast<double>(sc.inv_len) * static_cast<double>(sc.inv_len);
+        double best = 1.0;
+        for (int k = 1; k < 128; k += 2) {
+            const double as = s * (128 + k) / 128.0, off = std::fabs(static_cast<double>(static_cast<float>(as)) - as);
+            if (s == 0.0 || off < best * as) best = s == 0.0 ? 0.0 : off / as, u.alpha = (128 + k) / 128.0f;
+        }
+        u.soft = static_cast<float>(s * static_cast<double>(u.alpha));
+        out *= u.alpha;
+    }
+    u.out_hi = static_cast<float>(out);
+    if (std::isfinite(u.out_hi)) u.out_lo = static_cast<float>(out - static_cast<double>(u.out_hi));
+    return u;
 }
 
 int direct_effective_split(const DirectShape& s, int n_pad) {

@@ -37,21 +37,23 @@ struct DirectScale {
     float mass_k;   // law R: c; law P: 1 / c
     float soft;     // S / lambda^2 (law R) or eps^2 / lambda^2 (law P)
     float out;      // c / lambda^2
-    // Law R's sum over unordered pairs of unequal masses: the pair adds the
-    // softening as alpha r2 + alpha S', and the sums come back times alpha.
-    float alpha, alpha_soft;
 };
 
-// What the sums over unordered pairs come back multiplied by, in two floats.
-// gm_equal: every particle's G m if all are equal (the sums are then without the
-// mass), else 0.
-struct SymOut {
-    float hi, lo;
-};
 // G m of n masses if, in FP32 as the records hold it, all have the same positive
 // one (unrounded where the masses are equal in FP64 too), else 0.
 double equal_gm(double G, const double* mass, size_t n);
-SymOut sym_out(int law, const DirectScale& sc, double gm_equal);
+
+// What the sum over unordered pairs has of its own beside the scaled units.  Equal
+// masses: the sums are without the mass.  Unequal ones, law R: the pair adds the
+// softening as alpha r2 + alpha S', and the sums come back times alpha.
+struct SymUnits {
+    int equal;              // every real particle has the same positive G m
+    float alpha;            // 1 otherwise
+    float soft;             // alpha S' (law R) or eps'^2
+    float out_hi, out_lo;   // the sums back to accelerations, in two floats
+};
+// gm_equal: equal_gm's.
+SymUnits sym_units(int law, double softening, const DirectScale& sc, double gm_equal);
 
 // extent: the largest coordinate range of the system's positions (0 for a
 // single point); max_gm: its largest |G m| (0 when massless).
@@ -67,8 +69,6 @@ struct DirectLaunch {
     int n_pad;          // padded count, multiple of kTile
     int law;            // nbody_law
     DirectScale sc;     // the system's scaled units
-    bool equal;         // sym_step: every real particle has the same positive G m
-    SymOut sums_out;    // sym_step: the rows' sums back to accelerations
     bool massless;      // small_step: some real particle has no mass
     float dt;           // kick step
     float dts;          // drift factor dt / scale
@@ -109,7 +109,7 @@ SymPlan sym_plan(int n_pad);
 // Records of `part` that the plan writes.
 size_t sym_part_records(const SymPlan& p, int n_pad);
 // One force evaluation (kick: a full step), as direct_step.
-hipError_t sym_step(const DirectLaunch& L, const SymPlan& p, bool kick, hipStream_t stream, hipEvent_t ev_force_begin,
+hipError_t sym_step(const DirectLaunch& L, const SymPlan& p, const SymUnits& u, bool kick, hipStream_t stream, hipEvent_t ev_force_begin,
                     hipEvent_t ev_force_end);
 
 // Accelerations at m points (pts, 3m packed floats) from the n_src_pad sources

@@ -78,12 +78,13 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(6))) void
 // Adds each particle's rows, 64 particles a workgroup, scales the sums back and
 // kicks and drifts (kick != 0) or stores the acceleration only.
 template <int LAW>
-__global__ __launch_bounds__(256) void sym_reduce_kernel(DirectLaunch L, SymPlan P, int kick) {
+__global__ __launch_bounds__(256) void sym_reduce_kernel(DirectLaunch L, SymPlan P, float out_hi, float out_lo,
+                                                         int kick) {
     __shared__ core::SliceSums sums;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int i = blockIdx.x * 64 + lane;
     float s[3];
-    core::sum_rows(L.part, P, L.n_pad, i, sums, wave, lane, L.sums_out, s);
+    core::sum_rows(L.part, P, L.n_pad, i, sums, wave, lane, out_hi, out_lo, s);
     if (wave != 0 || i >= L.n) return;
     float4 x = L.src[i];
     core::sums_of_a_lost_particle<LAW>(x, L.sc, s);
@@ -126,20 +127,20 @@ size_t sym_part_records(const SymPlan& p, int n_pad) {
     return ((H + 1) * p.split + H) * static_cast<size_t>(n_pad);
 }
 
-hipError_t sym_step(const DirectLaunch& L, const SymPlan& P, bool kick, hipStream_t stream, hipEvent_t ev_b,
-                    hipEvent_t ev_e) {
-    const core::SymArgs A{L.src, L.part, L.n_pad, P, L.sc};
+hipError_t sym_step(const DirectLaunch& L, const SymPlan& P, const SymUnits& U, bool kick, hipStream_t stream,
+                    hipEvent_t ev_b, hipEvent_t ev_e) {
+    const core::SymArgs A{L.src, L.part, L.n_pad, P, L.sc, U.alpha, U.soft};
     const dim3 grid(P.nsb, (P.nsb / 2 + 1) * P.split);
     hipError_t e = hipSuccess;
     if (ev_b && (e = hipEventRecord(ev_b, stream)) != hipSuccess) return e;
     using Fn = void (*)(core::SymArgs);
-    const bool r = L.law == NBODY_LAW_R, eq = L.equal;
+    const bool r = L.law == NBODY_LAW_R, eq = U.equal != 0;
     const Fn fn = r ? (eq ? sym_force_kernel<NBODY_LAW_R, true> : sym_force_kernel<NBODY_LAW_R, false>)
                     : (eq ? sym_force_kernel<NBODY_LAW_P, true> : sym_force_kernel<NBODY_LAW_P, false>);
     hipLaunchKernelGGL(fn, grid, dim3(kTile), 0, stream, A);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (ev_e && (e = hipEventRecord(ev_e, stream)) != hipSuccess) return e;
-    hipLaunchKernelGGL((r ? sym_reduce_kernel<NBODY_LAW_R> : sym_reduce_kernel<NBODY_LAW_P>), dim3(L.n_pad / 64), dim3(256), 0, stream, L, P, kick ? 1 : 0);
+    hipLaunchKernelGGL((r ? sym_reduce_kernel<NBODY_LAW_R> : sym_reduce_kernel<NBODY_LAW_P>), dim3(L.n_pad / 64), dim3(256), 0, stream, L, P, U.out_hi, U.out_lo, kick ? 1 : 0);
     return hipGetLastError();
 }
 

@@ -31,6 +31,7 @@ struct SymArgs {
     int n_pad;
     SymPlan plan;
     DirectScale sc;
+    float alpha, soft;  // SymUnits
 };
 
 // A particle in scaled units: (x', y', z', G m / c).  With EQ the masses do not
@@ -155,8 +156,8 @@ __device__ __forceinline__ void sym_task(const SymArgs& A, SymShared& S, int blo
     const float tiny = in_vgpr(__FLT_MIN__);
     constexpr bool kAlpha = LAW == NBODY_LAW_R && !EQ;
     float alpha = 1.0f;
-    if constexpr (kAlpha) alpha = in_vgpr(A.sc.alpha);
-    const float soft = in_vgpr(kAlpha ? A.sc.alpha_soft : A.sc.soft);
+    if constexpr (kAlpha) alpha = in_vgpr(A.alpha);
+    const float soft = in_vgpr(A.soft);
     const int B = A.plan.block, S0 = B / A.plan.split;
     const int i0 = blockA * B, i1 = min(i0 + B, A.n_pad);
     const int j0 = blockB * B + h * S0, j1 = min(j0 + S0, A.n_pad);
@@ -257,10 +258,10 @@ __device__ __forceinline__ void sym_task(const SymArgs& A, SymShared& S, int blo
 // The sum of particle i's rows (i in block i / plan.block) in row order,
 // compensated: the workgroup's wave w takes a quarter of the rows, then the
 // waves' sums in order.  i is the same in every wave; every thread of the
-// workgroup must call it, and only wave 0 returns the sums, times `out` and
+// workgroup must call it, and only wave 0 returns the sums, times out and
 // rounded once, in s.
 __device__ __forceinline__ void sum_rows(const float4* __restrict__ part, const SymPlan& P, int n_pad, int i, SliceSums& sums,
-                                         int wave, int lane, const SymOut out, float (&s)[3]) {
+                                         int wave, int lane, float out_hi, float out_lo, float (&s)[3]) {
     const int b = i / P.block;
     const int H = P.nsb / 2, rows = (H + 1) * P.split + H, per = (rows + 3) / 4;
     float c[3] = {0.f, 0.f, 0.f};
@@ -284,7 +285,7 @@ __device__ __forceinline__ void sum_rows(const float4* __restrict__ part, const 
     }
     add_slices(sums, wave, lane, s, c);
 #pragma unroll
-    for (int a = 0; a < 3; ++a) s[a] = __builtin_fmaf(s[a], out.hi, __builtin_fmaf(s[a], out.lo, -(c[a] * out.hi)));
+    for (int a = 0; a < 3; ++a) s[a] = __builtin_fmaf(s[a], out_hi, __builtin_fmaf(s[a], out_lo, -(c[a] * out_hi)));
 }
 
 }  // namespace core

@@ -47,6 +47,7 @@ struct nbody_sim {
 
     nbody::DirectShape shape{4, 256, 1};
     bool small = false;    // the direct sum by whole steps of small systems instead
+    nbody::SymUnits sym_units{};
     nbody::SymPlan sym{};  // nsb > 0: the direct sum over unordered pairs instead
     nbody::BHState* bh = nullptr;
 
