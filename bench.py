@@ -33,20 +33,20 @@ FP32_PEAK_TFLOPS = 157.3   # MI355X FP32 vector peak (AMD public spec)
 # HBM-side bytes per step of the sum over unordered pairs at N = 2^20 (both
 # kernels), from rocprofv3 FETCH_SIZE and WRITE_SIZE scaled by a 256 MiB copy
 # (profiles/direct_force_n1m_law_r_traffic.md).
-DIRECT_1M_TRAFFIC_BYTES = 2.4161e10
+DIRECT_1M_TRAFFIC_BYTES = 2.9536e10
 # The force launch's SQ counters (profiles/direct_force_n1m_law_r_counters.md):
 # VALU instructions per interaction (two to a pair), VALU instructions issued per
 # SIMD per cycle and the clock that the launch ran at.
-DIRECT_1M_VALU = {"valu_instructions_per_interaction": 9.49, "rsq_per_interaction": 0.503,
-                  "valu_issue_per_simd_per_clock": 0.389, "valu_lane_ops_per_clock_per_cu": 99.5,
-                  "valu_busy_pct": 164, "lds_wait_pct_of_wave_time": 0.02, "clock_ghz": 2.134,
+DIRECT_1M_VALU = {"valu_instructions_per_interaction": 9.54, "rsq_per_interaction": 0.503,
+                  "valu_issue_per_simd_per_clock": 0.380, "valu_lane_ops_per_clock_per_cu": 97.3,
+                  "valu_busy_pct": 160, "lds_wait_pct_of_wave_time": 0.02, "clock_ghz": 2.179,
                   "source": "rocprofv3 --pmc, profiles/direct_force_n1m_law_r_counters.md"}
 # The same for the Barnes-Hut traversal step launch at N = 2^22, theta 0.5
 # (profiles/bh_traverse_n4m_theta05_traffic.md) and the 512-galaxy batch step
 # (profiles/batch_step_512_galaxies_traffic.md); they hold for the default
 # workloads only.
 BH_4M_TRAFFIC_BYTES = 2.7184e9
-BATCH_512_TRAFFIC_BYTES = 1.5905e10
+BATCH_512_TRAFFIC_BYTES = 1.7811e10
 FLOP_PER_INTERACTION = 20  # Nyland, Harris & Prins (GPU Gems 3, ch. 31) convention
 METRIC = "interactions/s & % FP32 VALU peak at N=1M; batched p50/p99 step latency"
 
