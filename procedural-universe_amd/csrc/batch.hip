@@ -995,6 +995,7 @@ nbody_status nbody_batch_get_info(nbody_batch* b, nbody_batch_info* out) {
     clear_error();
     NB_CHECK(b && out, NBODY_ERR_INVALID_ARG, "null argument");
     std::memset(out, 0, sizeof *out);
+    NB_HIP(hipSetDevice(b->cfg.device));  // laying the items out may allocate
     NB_TRY(rebuild_items(b));
     for (const auto& y : b->systems)
         if (y.live) {
