@@ -288,7 +288,11 @@ __global__ __launch_bounds__(kFieldThreads) __attribute__((amdgpu_waves_per_eu(8
                                                          cy, cz, turns);
     float s[3] = {sx[0], sy[0], sz[0]}, c[3] = {cx[0], cy[0], cz[0]};
     core::add_slices(sums, wave, lane, s, c);
-    if (wave == 0 && i < m) part[static_cast<size_t>(blockIdx.y) * m + i] = make_float4(s[0] - c[0], s[1] - c[1], s[2] - c[2], 0.f);
+    if (wave != 0 || i >= m) return;
+    float r[3] = {-c[0], -c[1], -c[2]};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) core::add_keeping_rest(s[a], r[a]);
+    part[static_cast<size_t>(blockIdx.y) * m + i] = core::pack_sums(s, r);
 }
 
 // Adds the chunks' sums of each point (compensated, in a fixed order) and scales
@@ -304,10 +308,13 @@ __global__ __launch_bounds__(256) void field_sum_kernel(const float4* __restrict
     if (i < m) {
 #pragma unroll 4
         for (int k = row; k < split; k += 16) {
-            const float4 p = part[static_cast<size_t>(k) * m + i];
-            kahan_add(s[0], c[0], p.x);
-            kahan_add(s[1], c[1], p.y);
-            kahan_add(s[2], c[2], p.z);
+            float x[3], r[3];
+            core::unpack_sums(part[static_cast<size_t>(k) * m + i], x, r);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                core::add_keeping_rest(s[a], x[a]);
+                c[a] -= x[a] + r[a];
+            }
         }
     }
 #pragma unroll
@@ -318,10 +325,11 @@ __global__ __launch_bounds__(256) void field_sum_kernel(const float4* __restrict
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         for (int r = 1; r < min(16, split); ++r) {
-            kahan_add(s[a], c[a], sums[a][r][pt]);
-            kahan_add(s[a], c[a], -sums[3 + a][r][pt]);
+            float x = sums[a][r][pt];
+            core::add_keeping_rest(s[a], x);
+            c[a] += sums[3 + a][r][pt] - x;
         }
-        o[a] = s[a] * sc.out;
+        o[a] = (s[a] - c[a]) * sc.out;
     }
 }
 

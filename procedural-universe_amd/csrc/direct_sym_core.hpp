@@ -56,34 +56,6 @@ __device__ __forceinline__ float4* part_row(float4* part, int r, int n_pad) {
     return part + static_cast<size_t>(r) * n_pad;
 }
 
-// A record: three sums s in FP32 and, in w, what their roundings left out, r (at
-// most half an ulp each), to 1 / 1,000 of an ulp in ten bits a sum; an ulp is 2^-23
-// times the sum's power of two, whose bits are its exponent's.  With rows rounded
-// to FP32 the RMS error is 1.5% larger at N = 2^20 and 2.5% at 2^21, where a streamed
-// particle's record is added to 12 times.
-__device__ __forceinline__ float4 pack_sums(const float (&s)[3], const float (&r)[3]) {
-    unsigned w = 0;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        const unsigned e = static_cast<unsigned>(__float_as_int(s[a])) & 0x7f800000u;
-        const float inv = __int_as_float(static_cast<int>(0x7f000000u - e));  // 2^-exponent
-        // the nearest whole number is in the last bits of its sum with 1.5 x 2^23
-        const float x = __builtin_fmaf(r[a] * inv, 511 * 0x1p24f, 0x1.8p23f);
-        w |= (static_cast<unsigned>(__float_as_int(x)) & 0x3ffu) << (10 * a);
-    }
-    return make_float4(s[0], s[1], s[2], __int_as_float(static_cast<int>(w)));
-}
-
-__device__ __forceinline__ void unpack_sums(const float4 q, float (&s)[3], float (&r)[3]) {
-    const int w = __float_as_int(q.w);
-    s[0] = q.x, s[1] = q.y, s[2] = q.z;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        const float p = __int_as_float(__float_as_int(s[a]) & 0x7f800000);
-        r[a] = static_cast<float>(static_cast<int>(__builtin_amdgcn_sbfe(w, 10 * a, 10))) * (p * (0x1p-24f / 511));
-    }
-}
-
 struct SymShared {
     float4 set[2][kWaves][2 * kSet];  // two tiles, every set twice in a row
     float sum[3][kWaves][kSet];       // the tile's sums
